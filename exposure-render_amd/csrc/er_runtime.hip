@@ -73,8 +73,10 @@ extern "C" hipError_t erd_launch_adj_wavefront(const DevParams* p, unsigned int*
                                                unsigned int* lcount, const uint32_t* s1start, const uint32_t* s2start,
                                                float* partials, int blocks, int n, size_t lds_bytes, hipStream_t st);
 extern "C" hipError_t erd_launch_adj_reset(unsigned int* counts, unsigned int* lcount, hipStream_t st);
-extern "C" hipError_t erd_launch_autofocus(const DevParams* p, int u, int v, uint32_t s0, uint32_t s1, float* out,
-                                           hipStream_t st);
+extern "C" size_t erd_autofocus_work_size(void);
+extern "C" size_t erd_autofocus_out_offset(void);
+extern "C" hipError_t erd_launch_autofocus(const DevParams* p, int u, int v, uint32_t s0, uint32_t s1, void* work, int full,
+                                           int serial, int lut_lds, size_t lds_bytes, hipStream_t st);
 extern "C" hipError_t erd_launch_adjoint(const DevParams* p, int mode, const float* lut_eval, const float* sigma_eval,
                                          const float4* adj, float4* value, float* partials, uint32_t* s1, uint32_t* s2,
                                          int W, int H, size_t lds_bytes, hipStream_t st);
@@ -370,6 +372,7 @@ struct Tracer {
     DevBuf<unsigned long long> counters;
     DevBuf<unsigned int> gm_tmp;
     DevBuf<char> bilateral;
+    DevBuf<char> focus;              /* the autofocus kernel's workspace, made by its first call */
     DevParams host_params{};
     uint64_t built_version = 0;
     int built_volume = -1;
@@ -398,7 +401,7 @@ struct Tracer {
         set[0].release(); set[1].release();
         running.release(); display.release(); disp_tmp.release(); disp_filt.release();
         seeds1.release(); seeds2.release(); lut.release(); mc_sigma.release(); wc_sigma.release(); params.release();
-        mc_bits.release(); clip_bits.release(); counters.release(); gm_tmp.release(); bilateral.release();
+        mc_bits.release(); clip_bits.release(); counters.release(); gm_tmp.release(); bilateral.release(); focus.release();
         tile_cost.release(); tile_order.release();
         if (stream) (void)hipStreamDestroy(stream);
         if (stream2) (void)hipStreamDestroy(stream2);
@@ -2501,10 +2504,20 @@ ER_API int er_get_autofocus_distance(int tracer_id, int film_u, int film_v, floa
     if ((st = build_params(*t))) return st;
     uint32_t s0, s1;
     er_autofocus_seeds(tracer_id, film_u, film_v, &s0, &s1);
-    DevBuf<float> d;
-    if ((st = d.alloc(1))) return st;
-    HIP_TRY(erd_launch_autofocus(t->params.ptr, film_u, film_v, s0, s1, d.ptr, t->stream));
-    HIP_TRY(hipMemcpyAsync(distance, d.ptr, sizeof(float), hipMemcpyDeviceToHost, t->stream));
+    const size_t work = erd_autofocus_work_size();
+    if (!t->focus.ptr) {
+        if ((st = t->focus.alloc(work))) return st;
+        const hipError_t e = hipMemset(t->focus.ptr, 0, work);
+        if (e != hipSuccess) {
+            t->focus.release();
+            return set_error(ER_ERROR, "%s (autofocus workspace)", hipGetErrorString(e));
+        }
+    }
+    const int full = t->desc.settings.estimator == ER_ESTIMATOR_FULL;
+    const int serial = full && t->desc.settings.sampler == ER_SAMPLER_WOODCOCK;
+    HIP_TRY(erd_launch_autofocus(t->params.ptr, film_u, film_v, s0, s1, t->focus.ptr, full, serial, t->lut_lds, t->lds_bytes,
+                                 t->stream));
+    HIP_TRY(hipMemcpyAsync(distance, t->focus.ptr + erd_autofocus_out_offset(), sizeof(float), hipMemcpyDeviceToHost, t->stream));
     HIP_TRY(hipStreamSynchronize(t->stream));
     return ER_OK;
 }

@@ -21,6 +21,10 @@
  */
 #include "er_path.h"
 
+#include <stddef.h>
+
+#define ER_FOCUS_RAYS 100   /* autofocus.cuh:34 */
+
 namespace erd {
 
 /* Stage the macrocell bits (always) and the opacity LUT (when LUT_LDS) in LDS. */
@@ -813,10 +817,31 @@ __global__ __launch_bounds__(256) void k_finish(const unsigned int* __restrict__
         finish_item(events[q], q, vis, frame);
 }
 
-/* ComputeAutoFocusDistance (autofocus.cuh:26-63), one lane: 100 rays through film point
- * (u, v), each jittered by 0.01 x a concentric-disk sample of the screen (Get2 in clang's
- * order), marched with SampleVolume on one RNG stream; the mean distance of the rays' volume
- * events, or the distance to the last event point (origin) when none. */
+/* ---- autofocus ------------------------------------------------------------------------- */
+
+/* One autofocus ray (autofocus.cuh:37-47): the camera ray through film point (u, v) moved by
+ * 0.01 x a concentric-disk sample of the screen. */
+__device__ __forceinline__ Ray focus_ray(const DevParams& p, int u, int v, float d0, float d1)
+{
+    float sx = p.screen00 + (p.invscreen0 * (float)u);
+    float sy = p.screen10 + (p.invscreen1 * (float)v);
+    float dx, dy;
+    concentric_disk(d0, d1, dx, dy);
+    sx += 0.01f * dx;
+    sy += 0.01f * dy;
+    Ray r;
+    r.O = ld3(p.cam_pos);
+    r.D = nrm(sub(add(ld3(p.cam_N), scl(sx, ld3(p.cam_U))), scl(sy, ld3(p.cam_V))));
+    r.MinT = p.clip_near;
+    r.MaxT = p.clip_far;
+    return r;
+}
+
+/* ComputeAutoFocusDistance (autofocus.cuh:26-63), one lane: ER_FOCUS_RAYS rays on one RNG
+ * stream (Get2 in clang's order), marched with SampleVolume; the mean distance of the rays'
+ * volume events, or the distance to the last event point (origin) when none. Woodcock
+ * tracking only: its draws per ray are not known before the ray is walked, so neither are the
+ * later rays' draws. */
 template<int FULL>
 __device__ void autofocus(const DevParams& p, int u, int v, uint32_t s0, uint32_t s1, float* out)
 {
@@ -826,22 +851,12 @@ __device__ void autofocus(const DevParams& p, int u, int v, uint32_t s0, uint32_
     rng.s0 = s0;
     rng.s1 = s1;
     Cnt cnt = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    const f3 O = ld3(p.cam_pos), N = ld3(p.cam_N), U = ld3(p.cam_U), V = ld3(p.cam_V);
+    const f3 O = ld3(p.cam_pos);
     float sum = 0.0f, w = 0.0f;
     f3 lastP = mk(0.0f, 0.0f, 0.0f);
-    for (int i = 0; i < 100; ++i) {
-        float sx = p.screen00 + (p.invscreen0 * (float)u);
-        float sy = p.screen10 + (p.invscreen1 * (float)v);
+    for (int i = 0; i < ER_FOCUS_RAYS; ++i) {
         const float d0 = rng.u(), d1 = rng.u();
-        float dx, dy;
-        concentric_disk(d0, d1, dx, dy);
-        sx += 0.01f * dx;
-        sy += 0.01f * dy;
-        Ray r;
-        r.O = O;
-        r.D = nrm(sub(add(N, scl(sx, U)), scl(sy, V)));
-        r.MinT = p.clip_near;
-        r.MaxT = p.clip_far;
+        const Ray r = focus_ray(p, u, v, d0, d1);
         float Tv; f3 Pv;
         if (march<FULL, 0, 1>(p, T, r, true, rng, Tv, Pv, cnt)) {
             sum += len(sub(Pv, O));
@@ -852,13 +867,117 @@ __device__ void autofocus(const DevParams& p, int u, int v, uint32_t s0, uint32_
     *out = sum <= 0.0f ? len(sub(lastP, O)) : sum / w;
 }
 
-__global__ __launch_bounds__(64) void k_autofocus(const DevParams* __restrict__ pp, int u, int v, uint32_t s0, uint32_t s1,
-                                                 float* __restrict__ out)
+__global__ __launch_bounds__(64) void k_autofocus_serial(const DevParams* __restrict__ pp, int u, int v, uint32_t s0, uint32_t s1,
+                                                        float* __restrict__ out)
 {
     if (threadIdx.x != 0) return;
+    autofocus<1>(*pp, u, v, s0, s1, out);
+}
+
+/* The same distance with the ray-march sampler, one wave per ray (coop_march), 4 rays to a
+ * workgroup. A ray takes two draws for its disk sample and two more when it meets the volume's
+ * box, so the draws of every ray follow from the box tests of the rays before it, without
+ * marching any: each workgroup writes the stream's states to LDS (one lane per generator), one
+ * thread per ray tests its box at its supposed place in the stream (every earlier ray a hit
+ * first), and the places are recomputed from the hits until they stand still; ray t's place is
+ * right after t rounds at the latest, after one where every ray hits. Each wave then marches
+ * its ray and the workgroup that finishes last adds the distances up in ray order. The march of
+ * a single ray is a chain of dependent loads: with one lane taking its 100 rays one after the
+ * other, sample by sample, the kernel took 3.6 ms and the call 3.7 to 6.6 ms on a 256^3 CT volume;
+ * now the call takes 0.088 ms. */
+struct FocusWork {
+    float dist[ER_FOCUS_RAYS], Px[ER_FOCUS_RAYS], Py[ER_FOCUS_RAYS], Pz[ER_FOCUS_RAYS];
+    int hit[ER_FOCUS_RAYS];
+    unsigned int done;            /* workgroups finished; the last one clears it again */
+    float out;
+};
+
+template<int FULL, int LUT_LDS>
+__global__ __launch_bounds__(256) void k_autofocus(const DevParams* __restrict__ pp, int u, int v, uint32_t s0, uint32_t s1,
+                                                  FocusWork* __restrict__ work)
+{
+    extern __shared__ uint32_t lds[];
+    __shared__ uint32_t st0[4 * ER_FOCUS_RAYS], st1[4 * ER_FOCUS_RAYS];   /* after draw 1, 2, ... */
+    __shared__ unsigned long long hits[2];
+    __shared__ int place[ER_FOCUS_RAYS];
+    __shared__ unsigned int arrived;
+    static_assert(ER_FOCUS_RAYS <= 128, "two waves of box tests");
     const DevParams& p = *pp;
-    if (p.estimator == ER_ESTIMATOR_FULL) autofocus<1>(p, u, v, s0, s1, out);
-    else autofocus<0>(p, u, v, s0, s1, out);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (threadIdx.x == 0) {
+        uint32_t s = s0;
+        for (int k = 0; k < 4 * ER_FOCUS_RAYS; ++k) { s = 36969u * (s & 65535u) + (s >> 16); st0[k] = s; }
+    } else if (threadIdx.x == 64) {
+        uint32_t s = s1;
+        for (int k = 0; k < 4 * ER_FOCUS_RAYS; ++k) { s = 18000u * (s & 65535u) + (s >> 16); st1[k] = s; }
+    }
+    const Tables T = stage_tables<LUT_LDS>(p, lds);   /* ends with a barrier */
+    auto draw = [&](int k) { return (float)(((st0[k] << 16) + st1[k]) & 0x007fffffu) * 1.1920928955078125e-07f; };
+    const int t = threadIdx.x;
+    int at = 4 * t;
+    for (int round = 0; round <= ER_FOCUS_RAYS; ++round) {
+        bool hit = false;
+        if (t < ER_FOCUS_RAYS) {
+            float nearT, farT;
+            hit = intersect_box(focus_ray(p, u, v, draw(at), draw(at + 1)), ld3(p.minp), ld3(p.maxp), nearT, farT);
+        }
+        const unsigned long long m = __ballot(hit);
+        if (lane == 0 && wave < 2) hits[wave] = m;
+        __syncthreads();
+        const int before = t < 64 ? __popcll(hits[0] & ((1ull << lane) - 1ull))
+                                  : __popcll(hits[0]) + __popcll(hits[1] & ((1ull << lane) - 1ull));
+        const bool moved = t < ER_FOCUS_RAYS && 2 * t + 2 * before != at;
+        if (t < ER_FOCUS_RAYS) at = 2 * t + 2 * before;
+        if (!__syncthreads_or(moved)) break;   /* workgroup-uniform; a barrier before hits is written again */
+    }
+    if (t < ER_FOCUS_RAYS) place[t] = at;
+    __syncthreads();
+    const int ray = blockIdx.x * 4 + wave;
+    if (ray < ER_FOCUS_RAYS) {
+        const int k = place[ray];
+        const Ray r = focus_ray(p, u, v, draw(k), draw(k + 1));
+        bool vol = false;
+        f3 P = mk(0.0f, 0.0f, 0.0f);
+        float nearT, farT;
+        if (intersect_box(r, ld3(p.minp), ld3(p.maxp), nearT, farT)) {
+            const float StepSize = p.step_primary * p.minstep;
+            Rng rng;
+            rng.s0 = st0[k + 1];
+            rng.s1 = st1[k + 1];
+            MarchState m;
+            if (march_begin(p, r, nearT, farT, StepSize, rng, -1.0f, m)) {
+                if (!(m.Sum < m.S)) {
+                    vol = true;
+                } else {
+                    Cnt cnt = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+                    int steps = 0;
+                    f3 Pv = P;
+                    vol = coop_march<FULL, 0>(p, T, m, StepSize, lane, cnt, Pv, steps) > 0;
+                    if (vol) P = Pv;
+                }
+            }
+        }
+        if (lane == 0) {
+            work->dist[ray] = len(sub(P, ld3(p.cam_pos)));
+            work->Px[ray] = P.x; work->Py[ray] = P.y; work->Pz[ray] = P.z;
+            work->hit[ray] = vol ? 1 : 0;
+        }
+    }
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0) arrived = atomicAdd(&work->done, 1u);
+    __syncthreads();
+    if (arrived != gridDim.x - 1u || threadIdx.x != 0) return;
+    __threadfence();
+    /* the last workgroup: every ray's result is in memory (volatile: not from a stale line) */
+    volatile FocusWork* w = work;
+    float sum = 0.0f, n = 0.0f;
+    int last = -1;
+    for (int i = 0; i < ER_FOCUS_RAYS; ++i)
+        if (w->hit[i]) { sum += w->dist[i]; n += 1.0f; last = i; }
+    const f3 lastP = last >= 0 ? mk(w->Px[last], w->Py[last], w->Pz[last]) : mk(0.0f, 0.0f, 0.0f);
+    w->out = sum <= 0.0f ? len(sub(lastP, ld3(p.cam_pos))) : sum / n;
+    w->done = 0u;
 }
 
 /* ---- batches: the same pass over many tracers per launch (er_render_batch) ------------ */
@@ -1268,9 +1387,25 @@ extern "C" hipError_t erd_launch_primary_shade(const erd::DevParams* p, float4* 
     return hipGetLastError();
 }
 
-extern "C" hipError_t erd_launch_autofocus(const erd::DevParams* p, int u, int v, uint32_t s0, uint32_t s1, float* out,
-                                           hipStream_t st)
+extern "C" size_t erd_autofocus_work_size(void) { return sizeof(erd::FocusWork); }
+extern "C" size_t erd_autofocus_out_offset(void) { return offsetof(erd::FocusWork, out); }
+
+/* work: erd_autofocus_work_size() bytes, zero before the first call; the distance is left at
+ * erd_autofocus_out_offset(). serial: the one-lane form (Woodcock tracking). */
+extern "C" hipError_t erd_launch_autofocus(const erd::DevParams* p, int u, int v, uint32_t s0, uint32_t s1, void* work,
+                                           int full, int serial, int lut_lds, size_t lds_bytes, hipStream_t st)
 {
-    hipLaunchKernelGGL(erd::k_autofocus, dim3(1), dim3(64), 0, st, p, u, v, s0, s1, out);
+    erd::FocusWork* w = (erd::FocusWork*)work;
+    const dim3 grid((ER_FOCUS_RAYS + 3) / 4), block(256);
+    if (serial)
+        hipLaunchKernelGGL(erd::k_autofocus_serial, dim3(1), dim3(64), 0, st, p, u, v, s0, s1, &w->out);
+    else if (full && lut_lds)
+        hipLaunchKernelGGL((erd::k_autofocus<1, 1>), grid, block, lds_bytes, st, p, u, v, s0, s1, w);
+    else if (full)
+        hipLaunchKernelGGL((erd::k_autofocus<1, 0>), grid, block, lds_bytes, st, p, u, v, s0, s1, w);
+    else if (lut_lds)
+        hipLaunchKernelGGL((erd::k_autofocus<0, 1>), grid, block, lds_bytes, st, p, u, v, s0, s1, w);
+    else
+        hipLaunchKernelGGL((erd::k_autofocus<0, 0>), grid, block, lds_bytes, st, p, u, v, s0, s1, w);
     return hipGetLastError();
 }

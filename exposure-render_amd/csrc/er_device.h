@@ -109,8 +109,7 @@ struct DevParams {
     int   cstride_y, cstride_z;      /* (Rx+1), (Rx+1)(Ry+1) */
     const float* sigma_lut;          /* DensityScale * Opacity(i), i in [0, lut_max] */
     int   lut_max;
-    const float* mc_sigma;           /* per macrocell max sigma */
-    const uint32_t* mc_bits;         /* bit m set <=> mc_sigma[m] > 0 */
+    const uint32_t* mc_bits;         /* bit m set <=> a sample in macrocell m can have sigma > 0 */
     int   mc_dim[3];
     int   mc_shift;                  /* macrocell edge = 2^mc_shift cells */
     int   mc_words;                  /* 32-bit words of mc_bits: macrocell bits, group bits, group clip-free bits */

@@ -158,135 +158,333 @@ __global__ __launch_bounds__(256) void k_bilateral(const BilateralParams* __rest
     out[(size_t)y * W + x] = d;
 }
 
-/* cell (cx, cy, cz) in [0, R]^3 holds the corners of lattice cell (cx-1, cy-1, cz-1) */
+/* cell (cx, cy, cz) in [0, R]^3 holds the corners of lattice cell (cx-1, cy-1, cz-1). Bound by the 16-byte records it writes: a thread owns one (cx, cy) column
+ * of ER_CELL_RUN cells along z and carries the column's upper corners over to the next cell, so
+ * a cell costs four 2-byte loads and no 64-bit division: 256^3 in 70 us, 3.9 TB/s written (the
+ * flat form with three divisions 85 us), 512 x 512 x 460 in 540 us (640). */
+#define ER_CELL_RUN 8
 __global__ __launch_bounds__(256) void k_build_cells(const uint16_t* __restrict__ vox, uint4* __restrict__ cells,
                                                     int rx, int ry, int rz)
 {
-    const int sx = rx + 1, sy = ry + 1, sz = rz + 1;
-    const size_t n = (size_t)sx * sy * sz;
-    for (size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (size_t)gridDim.x * blockDim.x) {
-        const int cx = (int)(k % sx);
-        const int cy = (int)((k / sx) % sy);
-        const int cz = (int)(k / ((size_t)sx * sy));
+    const unsigned int sx = (unsigned int)rx + 1u, sy = (unsigned int)ry + 1u;
+    const unsigned int n = sx * sy;                                     /* below 2^24 */
+    const unsigned int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < n) {
+        const int cy = (int)udiv24(k, sx);
+        const int cx = (int)(k - (unsigned int)cy * sx);
         const int x0 = max(cx - 1, 0), x1 = min(cx, rx - 1);
         const int y0 = max(cy - 1, 0), y1 = min(cy, ry - 1);
-        const int z0 = max(cz - 1, 0), z1 = min(cz, rz - 1);
-        auto at = [&](int x, int y, int z) -> uint32_t { return vox[((size_t)z * ry + y) * rx + x]; };
-        uint4 c;
-        c.x = at(x0, y0, z0) | (at(x1, y0, z0) << 16);
-        c.y = at(x0, y1, z0) | (at(x1, y1, z0) << 16);
-        c.z = at(x0, y0, z1) | (at(x1, y0, z1) << 16);
-        c.w = at(x0, y1, z1) | (at(x1, y1, z1) << 16);
-        cells[k] = c;
+        const size_t a = (size_t)y0 * rx + x0, b = (size_t)y0 * rx + x1, c = (size_t)y1 * rx + x0, d = (size_t)y1 * rx + x1;
+        const size_t plane = (size_t)rx * ry;
+        for (int z_first = (int)blockIdx.y * ER_CELL_RUN; z_first <= rz; z_first += (int)gridDim.y * ER_CELL_RUN) {
+            const uint16_t* v = vox + plane * (size_t)max(z_first - 1, 0);
+            uint32_t lo0 = (uint32_t)v[a] | ((uint32_t)v[b] << 16), lo1 = (uint32_t)v[c] | ((uint32_t)v[d] << 16);
+            for (int cz = z_first; cz < min(z_first + ER_CELL_RUN, rz + 1); ++cz) {
+                v = vox + plane * (size_t)min(cz, rz - 1);
+                const uint32_t hi0 = (uint32_t)v[a] | ((uint32_t)v[b] << 16), hi1 = (uint32_t)v[c] | ((uint32_t)v[d] << 16);
+                cells[(size_t)cz * n + k] = make_uint4(lo0, lo1, hi0, hi1);
+                lo0 = hi0;
+                lo1 = hi1;
+            }
+        }
     }
 }
 
 /* min/max voxel over [m*E, m*E + E] (E = 2^shift, clamped) on each axis: every voxel a sample
- * whose floor(L) >> shift == m (after clamping) can read */
+ * whose floor(L) >> shift == m (after clamping) can read.
+ * k_macro_rows, E <= 8: a workgroup takes a row of macrocells along x; each thread reduces one
+ * column of (E + 1)^2 voxels, all loads coalesced along x and independent, and the macrocells
+ * then reduce their E + 1 columns from LDS. Bound by the voxel loads: 1.3 passes over the volume.
+ * k_macro_minmax, E >= 16: a wave per macrocell, 16 lanes along x and 4 rows at once (few, large
+ * macrocells, whose rows alone would not fill the device).
+ * 8-cell macrocells of 192^3 / 512 x 512 x 460: 10.5 / 119 us; one lane per macrocell took 94 /
+ * 215 us, a wave per macrocell 24 / 400 us. */
+#define ER_ROW_COLUMNS 256
+__global__ __launch_bounds__(ER_ROW_COLUMNS) void k_macro_rows(const uint16_t* __restrict__ vox, uint32_t* __restrict__ mm,
+                                                               int rx, int ry, int rz, int mx, int my, int shift, int mrows)
+{
+    __shared__ uint32_t clo[ER_ROW_COLUMNS], chi[ER_ROW_COLUMNS];
+    const int E = 1 << shift;
+    const int per = (ER_ROW_COLUMNS - 1) >> shift;   /* macrocells a workgroup takes, and one more column */
+    const int m0 = (int)blockIdx.x * per;
+    const int x = min(m0 * E + (int)threadIdx.x, rx - 1);
+    for (int row = (int)blockIdx.y; row < mrows; row += (int)gridDim.y) {
+        const int by = row % my, bz = row / my;
+        const int y1 = min(by * E + E, ry - 1), z1 = min(bz * E + E, rz - 1);
+        uint32_t lo = 0xffff, hi = 0;
+        if ((int)threadIdx.x <= per * E)
+            for (int z = bz * E; z <= z1; ++z) {
+                const uint16_t* v = vox + ((size_t)z * ry + by * E) * rx + x;
+#pragma unroll 3
+                for (int y = by * E; y <= y1; ++y, v += rx) {
+                    const uint32_t u = *v;
+                    lo = min(lo, u);
+                    hi = max(hi, u);
+                }
+            }
+        clo[threadIdx.x] = lo;
+        chi[threadIdx.x] = hi;
+        __syncthreads();
+        const int m = m0 + (int)threadIdx.x;
+        if ((int)threadIdx.x < per && m < mx) {
+            for (int k = 0; k <= E; ++k) {
+                lo = k ? min(lo, clo[threadIdx.x * E + k]) : clo[threadIdx.x * E];
+                hi = k ? max(hi, chi[threadIdx.x * E + k]) : chi[threadIdx.x * E];
+            }
+            mm[(size_t)row * mx + m] = lo | (hi << 16);
+        }
+        __syncthreads();
+    }
+}
+
 __global__ __launch_bounds__(256) void k_macro_minmax(const uint16_t* __restrict__ vox, uint32_t* __restrict__ mm,
                                                      int rx, int ry, int rz, int mx, int my, int mz, int shift)
 {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
+    const int m = (int)(blockIdx.x * 4 + (threadIdx.x >> 6));
+    const int lx = threadIdx.x & 15, lr = (threadIdx.x >> 4) & 3;
+    uint32_t lo = 0xffff, hi = 0;
     if (m >= mx * my * mz) return;
     const int E = 1 << shift;
     const int bx = m % mx, by = (m / mx) % my, bz = m / (mx * my);
     const int x0 = bx * E, x1 = min(bx * E + E, rx - 1);
     const int y0 = by * E, y1 = min(by * E + E, ry - 1);
     const int z0 = bz * E, z1 = min(bz * E + E, rz - 1);
-    uint32_t lo = 0xffff, hi = 0;
     for (int z = z0; z <= z1; ++z)
-        for (int y = y0; y <= y1; ++y)
-            for (int x = x0; x <= x1; ++x) {
+        for (int y = y0 + lr; y <= y1; y += 4)
+            for (int x = x0 + lx; x <= x1; x += 16) {
                 const uint32_t v = vox[((size_t)z * ry + y) * rx + x];
                 lo = min(lo, v);
                 hi = max(hi, v);
             }
-    mm[m] = lo | (hi << 16);
+    for (int o = 32; o > 0; o >>= 1) {
+        lo = min(lo, (uint32_t)__shfl_xor((int)lo, o));
+        hi = max(hi, (uint32_t)__shfl_xor((int)hi, o));
+    }
+    if ((threadIdx.x & 63) == 0) mm[m] = lo | (hi << 16);
 }
 
-/* max sigma over the intensities a truncating trilinear sample can take in the macrocell:
- * each of the three lerp levels can lose at most one unit below the smallest corner */
+/* the largest voxel from a macrocell grid's ranges (one workgroup) */
+__global__ __launch_bounds__(1024) void k_range_top(const uint32_t* __restrict__ mm, int n, unsigned int* __restrict__ top)
+{
+    __shared__ uint32_t part[16];
+    uint32_t hi = 0;
+    for (int k = threadIdx.x; k < n; k += 1024) hi = max(hi, mm[k] >> 16);
+    for (int o = 32; o > 0; o >>= 1) hi = max(hi, (uint32_t)__shfl_xor((int)hi, o));
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = hi;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 16; ++w) hi = max(hi, part[w]);
+        *top = hi;
+    }
+}
+
+/* the intensities a truncating trilinear sample can take in a macrocell of min/max mm: each of
+ * the three lerp levels can lose at most one unit below the smallest corner */
+__device__ __forceinline__ void sample_range(uint32_t mm, int lut_max, int& lo, int& hi)
+{
+    lo = max((int)(mm & 0xffff) - 3, 0);
+    hi = min((int)(mm >> 16), lut_max);
+}
+
+/* max sigma over those intensities (the Woodcock majorants), 16 lanes to a macrocell: a range
+ * may span the whole table, which one lane per macrocell read entry by entry in 230 us */
 __global__ __launch_bounds__(256) void k_macro_sigma(const uint32_t* __restrict__ mm, const float* __restrict__ lut,
                                                     int lut_max, float* __restrict__ out, int n)
 {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= n) return;
-    const int lo = max((int)(mm[m] & 0xffff) - 3, 0);
-    const int hi = min((int)(mm[m] >> 16), lut_max);
+    const int m = (int)(blockIdx.x * (blockDim.x >> 4) + (threadIdx.x >> 4));
     float s = 0.0f;
-    for (int i = lo; i <= hi; ++i) s = fmaxf(s, lut[i]);
-    out[m] = s;
+    if (m < n) {
+        int lo, hi;
+        sample_range(mm[m], lut_max, lo, hi);
+        for (int i = lo + (int)(threadIdx.x & 15); i <= hi; i += 16) s = fmaxf(s, lut[i]);
+    }
+    for (int o = 8; o > 0; o >>= 1) s = fmaxf(s, __shfl_xor(s, o));
+    if (m < n && (threadIdx.x & 15) == 0) out[m] = s;
+}
+
+/* occupancy bit of macrocell m: it can hold a sample with sigma > 0 that is not clipped away.
+ * next[i] is the smallest intensity >= i whose sigma is positive (0xffffffff: none), so the test
+ * over the macrocell's range of intensities is one table read; gone (may be NULL) has bit m set
+ * when every sample of macrocell m is clipped away (the host's conservative test; clipping
+ * objects apply in the full estimator only). One lane per macrocell, a ballot for 64 bits. */
+__global__ __launch_bounds__(256) void k_macro_bits(const uint32_t* __restrict__ mm, const uint32_t* __restrict__ next,
+                                                   int lut_max, const uint32_t* __restrict__ gone,
+                                                   uint32_t* __restrict__ bits, int n, int words)
+{
+    const int m = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    bool occ = false;
+    if (m < n) {
+        int lo, hi;
+        sample_range(mm[m], lut_max, lo, hi);
+        occ = next[lo] <= (uint32_t)hi && !(gone && ((gone[m >> 5] >> (m & 31)) & 1u));
+    }
+    const unsigned long long v = __ballot(occ);
+    if ((threadIdx.x & 31) == 0 && (m >> 5) < words) bits[m >> 5] = (uint32_t)(v >> (threadIdx.x & 32));
 }
 
 /* group bits: bit g set iff any macrocell of group g (2^ER_GROUP_SHIFT macrocells a side, clipped to the
  * grid) has its bit set, from word `occ_base` of the same array; the groups' clip-free bits
  * from word `free_base`: bit g set iff every occupied macrocell of group g is wholly unclipped
  * (bit m of `unclipped`, the host's conservative test; NULL: no clipping objects, every bit
- * clear), so the march need not test its samples against them. */
+ * clear), so the march need not test its samples against them. One lane per group, which reads
+ * its macrocells' bits a row of 4 at a time (one lane per 32 groups, bit by bit, took 340 us for
+ * 16^3 groups; this takes 5). */
+__device__ __forceinline__ uint32_t bit_run(const uint32_t* __restrict__ w, int first, int count)
+{
+    const int s = first & 31;
+    uint32_t v = w[first >> 5] >> s;
+    if (s + count > 32) v |= w[(first >> 5) + 1] << (32 - s);
+    return v & ((1u << count) - 1u);
+}
 __global__ __launch_bounds__(256) void k_group_bits(uint32_t* __restrict__ bits, const uint32_t* __restrict__ unclipped,
                                                    int mx, int my, int mz, int gx, int gy, int gz, int occ_base,
                                                    int free_base, int words)
 {
-    const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= words) return;
-    uint32_t v = 0, f = 0;
-    for (int b = 0; b < 32; ++b) {
-        const int g = w * 32 + b;
-        if (g >= gx * gy * gz) break;
-        const int x = g % gx, y = (g / gx) % gy, z = g / (gx * gy);
-        bool any = false, free = unclipped != nullptr;
+    const int g = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    bool any = false, free = unclipped != nullptr;
+    if (g < gx * gy * gz) {
         const int E = 1 << ER_GROUP_SHIFT;
+        const int x = g % gx, y = (g / gx) % gy, z = g / (gx * gy);
+        const int nx = min(E, mx - E * x);
         for (int k = E * z; k < min(E * z + E, mz); ++k)
-            for (int j = E * y; j < min(E * y + E, my); ++j)
-                for (int i = E * x; i < min(E * x + E, mx); ++i) {
-                    const int m = (k * my + j) * mx + i;
-                    if ((bits[m >> 5] >> (m & 31)) & 1u) {
-                        any = true;
-                        free = free && ((unclipped[m >> 5] >> (m & 31)) & 1u);
-                    }
-                }
-        if (any) v |= 1u << b;
-        if (free) f |= 1u << b;
+            for (int j = E * y; j < min(E * y + E, my); ++j) {
+                const int m = (k * my + j) * mx + E * x;
+                const uint32_t o = bit_run(bits, m, nx);
+                any = any || o != 0u;
+                if (unclipped) free = free && (o & ~bit_run(unclipped, m, nx)) == 0u;
+            }
+    } else {
+        free = false;
     }
-    bits[occ_base + w] = v;
-    bits[free_base + w] = f;
+    const unsigned long long va = __ballot(any), vf = __ballot(free);
+    if ((threadIdx.x & 31) == 0 && (g >> 5) < words) {
+        bits[occ_base + (g >> 5)] = (uint32_t)(va >> (threadIdx.x & 32));
+        bits[free_base + (g >> 5)] = (uint32_t)(vf >> (threadIdx.x & 32));
+    }
 }
 
-/* occupancy bit of macrocell m: it can hold a sample with sigma > 0 that is not clipped away;
- * clipped (may be NULL) has bit m set when every sample of macrocell m is clipped away (the
- * host's conservative test; clipping objects apply in the full estimator only) */
-__global__ __launch_bounds__(256) void k_macro_bits(const float* __restrict__ mc_sigma, const uint32_t* __restrict__ clipped,
-                                                   uint32_t* __restrict__ bits, int n, int words)
+/* The empty-space radius of every group: its Chebyshev distance to the nearest occupied group,
+ * at most 15 (0 for an occupied group). The distance is taken axis by axis - along a row, the
+ * steps to the nearest occupied group; then along each further axis the minimum over its
+ * neighbours of the larger of the step and the neighbour's distance so far. AXIS 0 reads the
+ * groups' occupancy bits, AXIS 2 packs the result, eight groups to a word. (The host did this,
+ * between two copies that waited for the device.) */
+template<int AXIS>
+__global__ __launch_bounds__(256) void k_group_radii(const uint32_t* __restrict__ occ, const uint8_t* __restrict__ in,
+                                                    uint8_t* __restrict__ out, uint32_t* __restrict__ packed, int gx, int gy,
+                                                    int gz)
 {
-    const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= words) return;
-    const uint32_t gone = clipped ? clipped[w] : 0u;
-    uint32_t v = 0;
-    for (int b = 0; b < 32; ++b) {
-        const int m = w * 32 + b;
-        if (m < n && mc_sigma[m] > 0.0f && !((gone >> b) & 1u)) v |= 1u << b;
+    const int g = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    const int n = gx * gy * gz;
+    int d = 15;
+    if (g < n) {
+        const int dim = AXIS == 0 ? gx : (AXIS == 1 ? gy : gz);
+        const int step = AXIS == 0 ? 1 : (AXIS == 1 ? gx : gx * gy);
+        const int at = AXIS == 0 ? g % gx : (AXIS == 1 ? (g / gx) % gy : g / (gx * gy));
+        /* a neighbour r steps away cannot lower a distance of at most r */
+        for (int r = 0; r < d; ++r)
+            for (int s = -1; s <= 1; s += 2) {
+                if (at + s * r < 0 || at + s * r >= dim) continue;
+                const int h = g + s * r * step;
+                const int v = AXIS == 0 ? (((occ[h >> 5] >> (h & 31)) & 1u) ? 0 : 15) : (int)in[h];
+                d = min(d, max(r, v));
+            }
     }
-    bits[w] = v;
+    if (AXIS < 2) {
+        if (g < n) out[g] = (uint8_t)d;
+    } else {
+        uint32_t w = g < n ? (uint32_t)d << ((g & 7) * 4) : 0u;
+        for (int o = 1; o < 8; o <<= 1) w |= (uint32_t)__shfl_xor((int)w, o);
+        if ((g & 7) == 0 && g < n) packed[g >> 3] = w;
+    }
 }
 
-/* maximum GradientMagnitude over voxel centres (design: gradientmagnitude.cuh:28-70) */
-__global__ __launch_bounds__(256) void k_gm_max(const DevParams* __restrict__ pp, unsigned int* __restrict__ out)
+/* ---- maximum GradientMagnitude over voxel centres (design: gradientmagnitude.cuh:28-70) ----
+ * The six samples of a voxel take some 500 instructions (every voxel of 256^3: 240 us, of
+ * 512 x 512 x 460: 1680 us, all of it instruction issue; now 179 and 426 us), and few bricks of 8^3 voxels can hold the maximum: a sample in the brick
+ * lies between (the smallest voxel it can read) - 3 (truncating lerps) and the largest, so with R
+ * their difference no gradient there exceeds the expression's value for a difference of R on
+ * every axis (each operation is monotone). k_gm_bound finds that bound for every brick, one wave
+ * per brick; in k_gm_max each wave takes ER_GM_RUN bricks, the one of the largest bound first,
+ * offers its result as a lower limit for all waves, and then only the bricks whose bound exceeds
+ * the largest offer so far. Which bricks are left out depends on timing, the maximum does not.
+ * Few atomics: operations on one address go one after the other, some 6 ns each (an exchange
+ * per brick took 790 us). prune = 0, where lattice coordinates are too coarse for the two-voxel
+ * margin, takes every brick. */
+#define ER_GM_RUN 64
+__global__ __launch_bounds__(256) void k_gm_bound(const DevParams* __restrict__ pp, const uint16_t* __restrict__ vox,
+                                                 float* __restrict__ bounds, int bx, int by, int nb, int prune)
 {
     const DevParams& p = *pp;
-    const size_t n = (size_t)p.res[0] * p.res[1] * p.res[2];
-    float best = 0.0f;
-    for (size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (size_t)gridDim.x * blockDim.x) {
-        const int x = (int)(k % p.res[0]);
-        const int y = (int)((k / p.res[0]) % p.res[1]);
-        const int z = (int)(k / ((size_t)p.res[0] * p.res[1]));
-        const f3 P = mk(p.minp[0] + p.size[0] * (((float)x + 0.5f) / (float)p.res[0]),
-                        p.minp[1] + p.size[1] * (((float)y + 0.5f) / (float)p.res[1]),
-                        p.minp[2] + p.size[2] * (((float)z + 0.5f) / (float)p.res[2]));
-        best = fmaxf(best, gradient_magnitude(p, P));
+    const int rx = p.res[0], ry = p.res[1], rz = p.res[2];
+    const int lane = threadIdx.x & 63;
+    const int b = (int)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
+    if (b >= nb) return;
+    const int X = (b % bx) * 8, Y = ((b / bx) % by) * 8, Z = (b / (bx * by)) * 8;
+    /* voxels [X - 2, X + 9], clamped to the volume, 12 on each axis */
+    const int x = min(max(X - 2 + min(lane & 15, 11), 0), rx - 1);
+    uint32_t lo = 0xffff, hi = 0;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const int y = min(max(Y - 2 + 4 * j + (lane >> 4), 0), ry - 1);
+#pragma unroll
+        for (int i = 0; i < 12; ++i) {
+            const int z = min(max(Z - 2 + i, 0), rz - 1);
+            const uint32_t v = vox[((size_t)z * ry + y) * rx + x];
+            lo = min(lo, v);
+            hi = max(hi, v);
+        }
     }
-    /* non-negative floats order like their bit patterns */
-    for (int off = 32; off > 0; off >>= 1) best = fmaxf(best, __shfl_xor(best, off));
-    if ((threadIdx.x & 63) == 0) atomicMax(out, __float_as_uint(best));
+    for (int o = 32; o > 0; o >>= 1) {
+        lo = min(lo, (uint32_t)__shfl_xor((int)lo, o));
+        hi = max(hi, (uint32_t)__shfl_xor((int)hi, o));
+    }
+    const float R = (float)(hi - lo + 3u);
+    const float g[6] = {0.0f, R, 0.0f, R, 0.0f, R};
+    if (lane == 0) bounds[b] = prune ? gradient_magnitude_cd(p, g) : 3.402823466e+38f;
+}
+
+__global__ __launch_bounds__(256) void k_gm_max(const DevParams* __restrict__ pp, const float* __restrict__ bounds,
+                                               unsigned int* __restrict__ out, int bx, int by, int nb)
+{
+    const DevParams& p = *pp;
+    const int rx = p.res[0], ry = p.res[1], rz = p.res[2];
+    const int lane = threadIdx.x & 63;
+    const int waves = (int)(gridDim.x * (blockDim.x >> 6));
+    const int w = (int)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
+    /* the wave's bricks: w, w + waves, ...; lane k holds the bound of the k-th (at most ER_GM_RUN) */
+    const int mine = w + lane * waves;
+    float bound = lane < ER_GM_RUN && mine < nb ? bounds[mine] : -1.0f;
+    if (!(bound == bound)) bound = 3.402823466e+38f;   /* a NaN excludes nothing */
+    float best = 0.0f, seen = 0.0f;
+    for (bool first = true;; first = false) {
+        float top = bound;
+        for (int o = 32; o > 0; o >>= 1) top = fmaxf(top, __shfl_xor(top, o));
+        if (!(top > fmaxf(best, seen))) break;
+        const int k = __ffsll((long long)__ballot(bound == top)) - 1;
+        const int b = w + k * waves;
+        if (lane == k) bound = -1.0f;
+        const int X = (b % bx) * 8, Y = ((b / bx) % by) * 8, Z = (b / (bx * by)) * 8;
+        const int x = X + (lane & 7), y = Y + (lane >> 3);
+        float m = 0.0f;
+        if (x < rx && y < ry) {
+            for (int z = Z; z < min(Z + 8, rz); ++z) {
+                const f3 P = mk(p.minp[0] + p.size[0] * (((float)x + 0.5f) / (float)rx),
+                                p.minp[1] + p.size[1] * (((float)y + 0.5f) / (float)ry),
+                                p.minp[2] + p.size[2] * (((float)z + 0.5f) / (float)rz));
+                m = fmaxf(m, gradient_magnitude(p, P));
+            }
+        }
+        for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+        best = fmaxf(best, m);
+        if (first) {
+            /* non-negative floats order like their bit patterns */
+            unsigned int s = 0u;
+            if (lane == 0) s = atomicMax(out, __float_as_uint(best));
+            seen = __uint_as_float(__builtin_amdgcn_readfirstlane(s));
+        }
+    }
+    if (lane == 0 && best > seen) atomicMax(out, __float_as_uint(best));
 }
 
 } /* namespace erd */
@@ -312,42 +510,71 @@ extern "C" size_t erd_bilateral_params_size(void) { return sizeof(erd::Bilateral
 
 extern "C" hipError_t erd_launch_build_cells(const uint16_t* vox, uint4* cells, int rx, int ry, int rz, hipStream_t st)
 {
-    hipLaunchKernelGGL(erd::k_build_cells, dim3(2048), dim3(256), 0, st, vox, cells, rx, ry, rz);
+    const unsigned int n = (unsigned int)(rx + 1) * (unsigned int)(ry + 1);
+    const int runs = std::min((rz + 1 + ER_CELL_RUN - 1) / ER_CELL_RUN, 32768);   /* the kernel strides over more */
+    hipLaunchKernelGGL(erd::k_build_cells, dim3((n + 255) / 256, runs), dim3(256), 0, st, vox, cells, rx, ry, rz);
+    return hipGetLastError();
+}
+
+extern "C" hipError_t erd_launch_range_top(const uint32_t* mm, int n, unsigned int* top, hipStream_t st)
+{
+    hipLaunchKernelGGL(erd::k_range_top, dim3(1), dim3(1024), 0, st, mm, n, top);
     return hipGetLastError();
 }
 
 extern "C" hipError_t erd_launch_macro_minmax(const uint16_t* vox, uint32_t* mm, int rx, int ry, int rz, int mx, int my,
                                               int mz, int shift, hipStream_t st)
 {
-    const int n = mx * my * mz;
-    hipLaunchKernelGGL(erd::k_macro_minmax, dim3((n + 255) / 256), dim3(256), 0, st, vox, mm, rx, ry, rz, mx, my, mz, shift);
+    if (shift <= 3) {
+        const int per = (ER_ROW_COLUMNS - 1) >> shift;
+        hipLaunchKernelGGL(erd::k_macro_rows, dim3((mx + per - 1) / per, std::min(my * mz, 32768)), dim3(ER_ROW_COLUMNS), 0, st,
+                           vox, mm, rx, ry, rz, mx, my, shift, my * mz);
+    } else {
+        hipLaunchKernelGGL(erd::k_macro_minmax, dim3((mx * my * mz + 3) / 4), dim3(256), 0, st, vox, mm, rx, ry, rz, mx, my, mz,
+                           shift);
+    }
     return hipGetLastError();
 }
 
-extern "C" hipError_t erd_launch_macro_bits(const float* mc_sigma, const uint32_t* clipped, uint32_t* bits, int n, int words,
-                                            hipStream_t st)
+extern "C" hipError_t erd_launch_macro_bits(const uint32_t* mm, const uint32_t* next, int lut_max, const uint32_t* gone,
+                                            uint32_t* bits, int n, int words, hipStream_t st)
 {
-    hipLaunchKernelGGL(erd::k_macro_bits, dim3((words + 255) / 256), dim3(256), 0, st, mc_sigma, clipped, bits, n, words);
+    hipLaunchKernelGGL(erd::k_macro_bits, dim3((n + 255) / 256), dim3(256), 0, st, mm, next, lut_max, gone, bits, n, words);
     return hipGetLastError();
 }
 
-extern "C" hipError_t erd_launch_group_bits(uint32_t* bits, const uint32_t* unclipped, int mx, int my, int mz, int gx, int gy,
-                                            int gz, int occ_base, int free_base, int words, hipStream_t st)
+/* the groups' occupancy bits (from word occ_base), clip-free bits (free_base) and radii
+ * (radii_base); tmp: two bytes a group */
+extern "C" hipError_t erd_launch_group_tables(uint32_t* bits, const uint32_t* unclipped, uint8_t* tmp, int mx, int my, int mz,
+                                              int gx, int gy, int gz, int occ_base, int free_base, int radii_base, int words,
+                                              hipStream_t st)
 {
-    hipLaunchKernelGGL(erd::k_group_bits, dim3((words + 255) / 256), dim3(256), 0, st, bits, unclipped, mx, my, mz, gx, gy,
-                       gz, occ_base, free_base, words);
+    const int n = gx * gy * gz;
+    const dim3 grid((n + 255) / 256), block(256);
+    uint8_t* tmp2 = tmp + n;
+    const uint32_t* occ = bits + occ_base;
+    hipLaunchKernelGGL(erd::k_group_bits, grid, block, 0, st, bits, unclipped, mx, my, mz, gx, gy, gz, occ_base, free_base, words);
+    hipLaunchKernelGGL(erd::k_group_radii<0>, grid, block, 0, st, occ, (const uint8_t*)nullptr, tmp, (uint32_t*)nullptr, gx, gy, gz);
+    hipLaunchKernelGGL(erd::k_group_radii<1>, grid, block, 0, st, occ, (const uint8_t*)tmp, tmp2, (uint32_t*)nullptr, gx, gy, gz);
+    hipLaunchKernelGGL(erd::k_group_radii<2>, grid, block, 0, st, occ, (const uint8_t*)tmp2, tmp, bits + radii_base, gx, gy, gz);
     return hipGetLastError();
 }
 
 extern "C" hipError_t erd_launch_macro_sigma(const uint32_t* mm, const float* lut, int lut_max, float* out, int n, hipStream_t st)
 {
-    hipLaunchKernelGGL(erd::k_macro_sigma, dim3((n + 255) / 256), dim3(256), 0, st, mm, lut, lut_max, out, n);
+    hipLaunchKernelGGL(erd::k_macro_sigma, dim3((n + 15) / 16), dim3(256), 0, st, mm, lut, lut_max, out, n);
     return hipGetLastError();
 }
 
-extern "C" hipError_t erd_launch_gm_max(const erd::DevParams* p, unsigned int* out, hipStream_t st)
+/* out: one word, zero before the call; bounds: one float per brick of 8^3 voxels */
+extern "C" hipError_t erd_launch_gm_max(const erd::DevParams* p, const uint16_t* vox, float* bounds, unsigned int* out, int rx,
+                                        int ry, int rz, int prune, hipStream_t st)
 {
-    hipLaunchKernelGGL(erd::k_gm_max, dim3(2048), dim3(256), 0, st, p, out);
+    const int bx = (rx + 7) / 8, by = (ry + 7) / 8, nb = bx * by * ((rz + 7) / 8);
+    hipLaunchKernelGGL(erd::k_gm_bound, dim3((nb + 3) / 4), dim3(256), 0, st, p, vox, bounds, bx, by, nb, prune);
+    /* ER_GM_RUN bricks to a wave, fewer where that would leave the device's 4 waves per CU idle */
+    const int waves = std::max((nb + ER_GM_RUN - 1) / ER_GM_RUN, std::min(nb, 1024));
+    hipLaunchKernelGGL(erd::k_gm_max, dim3((waves + 3) / 4), dim3(256), 0, st, p, (const float*)bounds, out, bx, by, nb);
     return hipGetLastError();
 }
 

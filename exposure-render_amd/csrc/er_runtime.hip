@@ -43,19 +43,22 @@ extern "C" hipError_t erd_launch_trace(const DevParams* p, float4* frame, uint32
 extern "C" void erd_pass_record_sizes(size_t* scatter, size_t* event, size_t* job);
 extern "C" hipError_t erd_launch_post(const DevParams* p, const float4* frame, float4* running, uchar4* display,
                                       int no_iterations, unsigned int* qcount, int W, int H, hipStream_t st);
-extern "C" hipError_t erd_launch_macro_bits(const float* mc_sigma, const uint32_t* clipped, uint32_t* bits, int n, int words,
-                                            hipStream_t st);
-extern "C" hipError_t erd_launch_group_bits(uint32_t* bits, const uint32_t* unclipped, int mx, int my, int mz, int gx, int gy,
-                                            int gz, int occ_base, int free_base, int words, hipStream_t st);
+extern "C" hipError_t erd_launch_macro_bits(const uint32_t* mm, const uint32_t* next, int lut_max, const uint32_t* gone,
+                                            uint32_t* bits, int n, int words, hipStream_t st);
+extern "C" hipError_t erd_launch_group_tables(uint32_t* bits, const uint32_t* unclipped, uint8_t* tmp, int mx, int my, int mz,
+                                              int gx, int gy, int gz, int occ_base, int free_base, int radii_base, int words,
+                                              hipStream_t st);
 extern "C" hipError_t erd_launch_bilateral(const void* bp, const uchar4* in, uchar4* tmp, uchar4* out, int W, int H,
                                            hipStream_t st);
 extern "C" size_t erd_bilateral_params_size(void);
 extern "C" hipError_t erd_launch_build_cells(const uint16_t* vox, uint4* cells, int rx, int ry, int rz, hipStream_t st);
+extern "C" hipError_t erd_launch_range_top(const uint32_t* mm, int n, unsigned int* top, hipStream_t st);
 extern "C" hipError_t erd_launch_macro_minmax(const uint16_t* vox, uint32_t* mm, int rx, int ry, int rz, int mx, int my,
                                               int mz, int shift, hipStream_t st);
 extern "C" hipError_t erd_launch_macro_sigma(const uint32_t* mm, const float* lut, int lut_max, float* out, int n,
                                              hipStream_t st);
-extern "C" hipError_t erd_launch_gm_max(const DevParams* p, unsigned int* out, hipStream_t st);
+extern "C" hipError_t erd_launch_gm_max(const DevParams* p, const uint16_t* vox, float* bounds, unsigned int* out, int rx,
+                                        int ry, int rz, int prune, hipStream_t st);
 extern "C" hipError_t erd_launch_batch_trace(const erd::BatchJob* J, int na, int full, int primary_blocks,
                                              int lds_words, int shade_blocks, hipStream_t stream,
                                              hipStream_t stream2, hipEvent_t shaded, int lpr, int shadow_lpr);
@@ -299,13 +302,14 @@ struct Volume {
     er_volume_desc desc{};
     DevBuf<uint16_t> vox;
     DevBuf<uint4> cells;
+    DevBuf<unsigned int> top;       /* the largest voxel, as the device finds it */
     std::map<int, MacroGrid> grids;
     int mc_shift = 3;               /* default brick: 8 cells, coarser for very large volumes */
     uint16_t vmax = 0;
     uint64_t upload = 0;            /* upload serial number (autotuner cache key) */
     ~Volume()
     {
-        vox.release(); cells.release();
+        vox.release(); cells.release(); top.release();
         for (auto& g : grids) g.second.mm.release();
     }
 };
@@ -364,13 +368,15 @@ struct Tracer {
     DevBuf<float4> running;
     DevBuf<uchar4> display, disp_tmp, disp_filt;
     DevBuf<uint32_t> seeds1, seeds2;
-    DevBuf<float> lut, mc_sigma, wc_sigma;
-    DevBuf<uint32_t> mc_bits, clip_bits;
+    DevBuf<float> lut, wc_sigma;
+    DevBuf<uint32_t> lut_next, mc_bits, clip_bits;
+    DevBuf<uint8_t> group_tmp;
     size_t lds_bytes = 0;
     int lut_lds = 0;
     DevBuf<DevParams> params;
     DevBuf<unsigned long long> counters;
     DevBuf<unsigned int> gm_tmp;
+    DevBuf<float> gm_bounds;
     DevBuf<char> bilateral;
     DevBuf<char> focus;              /* the autofocus kernel's workspace, made by its first call */
     DevParams host_params{};
@@ -400,8 +406,8 @@ struct Tracer {
         for (hipEvent_t e : timing_events) (void)hipEventDestroy(e);
         set[0].release(); set[1].release();
         running.release(); display.release(); disp_tmp.release(); disp_filt.release();
-        seeds1.release(); seeds2.release(); lut.release(); mc_sigma.release(); wc_sigma.release(); params.release();
-        mc_bits.release(); clip_bits.release(); counters.release(); gm_tmp.release(); bilateral.release(); focus.release();
+        seeds1.release(); seeds2.release(); lut.release(); lut_next.release(); wc_sigma.release(); group_tmp.release(); params.release();
+        mc_bits.release(); clip_bits.release(); counters.release(); gm_tmp.release(); gm_bounds.release(); bilateral.release(); focus.release();
         tile_cost.release(); tile_order.release();
         if (stream) (void)hipStreamDestroy(stream);
         if (stream2) (void)hipStreamDestroy(stream2);
@@ -613,6 +619,29 @@ void camera_update(DevParams& P, const er_camera& c)
     P.film_h = c.film_size[1];
 }
 
+/* the volume's macrocell grid of 2^shift cells a side, built on first use */
+MacroGrid* volume_grid(Volume& v, int shift, int& st)
+{
+    st = ER_OK;
+    auto it = v.grids.find(shift);
+    if (it != v.grids.end()) return &it->second;
+    const er_volume_desc& d = v.desc;
+    const int E = 1 << shift;
+    MacroGrid& g = v.grids[shift];
+    for (int i = 0; i < 3; ++i) g.mc[i] = (d.resolution[i] + E - 1) / E;
+    if ((st = g.mm.alloc((size_t)g.mc[0] * g.mc[1] * g.mc[2]))) { v.grids.erase(shift); return nullptr; }
+    hipError_t e = erd_launch_macro_minmax(v.vox.ptr, g.mm.ptr, d.resolution[0], d.resolution[1], d.resolution[2], g.mc[0],
+                                           g.mc[1], g.mc[2], shift, 0);
+    if (e == hipSuccess) e = hipStreamSynchronize(0);
+    if (e != hipSuccess) {
+        g.mm.release();
+        v.grids.erase(shift);
+        st = set_error(ER_ERROR, "%s (macrocell grid)", hipGetErrorString(e));
+        return nullptr;
+    }
+    return &g;
+}
+
 int upload_volume(Volume& v)
 {
     const er_volume_desc& d = v.desc;
@@ -628,45 +657,25 @@ int upload_volume(Volume& v)
     int st;
     if ((st = v.vox.alloc(n))) return st;
     HIP_TRY(hipMemcpy(v.vox.ptr, d.voxels, n * sizeof(uint16_t), hipMemcpyHostToDevice));
-    uint16_t vmax = 0;
-    for (size_t i = 0; i < n; ++i) vmax = std::max(vmax, d.voxels[i]);
-    v.vmax = vmax;
     const size_t nc = (size_t)(rx + 1) * (ry + 1) * (rz + 1);
-    if ((st = v.cells.alloc(nc))) return st;
+    if ((st = v.cells.alloc(nc)) || (st = v.top.alloc(1))) return st;
+    for (auto& g : v.grids) g.second.mm.release();
+    v.grids.clear();
     HIP_TRY(erd_launch_build_cells(v.vox.ptr, v.cells.ptr, rx, ry, rz, 0));
+    /* the largest voxel, from the ranges of the 8-cell macrocells (the usual default grid) */
+    MacroGrid* grid = volume_grid(v, 3, st);
+    if (!grid) return st;
+    HIP_TRY(erd_launch_range_top(grid->mm.ptr, grid->mc[0] * grid->mc[1] * grid->mc[2], v.top.ptr, 0));
+    unsigned int vmax = 0;
+    HIP_TRY(hipMemcpy(&vmax, v.top.ptr, sizeof(vmax), hipMemcpyDeviceToHost));
+    v.vmax = (uint16_t)vmax;
     /* default macrocell edge: 8 cells, coarser when the occupancy bits and the opacity table
      * would not fit their 52.5 KB of LDS */
     v.mc_shift = 3;
     while (!brick_fits(d, v.vmax, v.mc_shift) && v.mc_shift < 8) v.mc_shift++;
     static uint64_t uploads = 0;
     v.upload = ++uploads;
-    for (auto& g : v.grids) g.second.mm.release();
-    v.grids.clear();
-    HIP_TRY(hipDeviceSynchronize());
     return ER_OK;
-}
-
-/* the volume's macrocell grid of 2^shift cells a side, built on first use */
-MacroGrid* volume_grid(Volume& v, int shift, int& st)
-{
-    st = ER_OK;
-    auto it = v.grids.find(shift);
-    if (it != v.grids.end()) return &it->second;
-    const er_volume_desc& d = v.desc;
-    const int E = 1 << shift;
-    MacroGrid& g = v.grids[shift];
-    for (int i = 0; i < 3; ++i) g.mc[i] = (d.resolution[i] + E - 1) / E;
-    if ((st = g.mm.alloc((size_t)g.mc[0] * g.mc[1] * g.mc[2]))) { v.grids.erase(shift); return nullptr; }
-    hipError_t e = erd_launch_macro_minmax(v.vox.ptr, g.mm.ptr, d.resolution[0], d.resolution[1], d.resolution[2], g.mc[0],
-                                           g.mc[1], g.mc[2], shift, 0);
-    if (e == hipSuccess) e = hipDeviceSynchronize();
-    if (e != hipSuccess) {
-        g.mm.release();
-        v.grids.erase(shift);
-        st = set_error(ER_ERROR, "%s (macrocell grid)", hipGetErrorString(e));
-        return nullptr;
-    }
-    return &g;
 }
 
 bool needs_gm(const er_tracer_desc& d)
@@ -826,48 +835,6 @@ void clip_classes(const DevParams& P, int nmc, double edge_ext, std::vector<uint
             }
         });
     for (auto& x : th) x.join();
-}
-
-/* The empty-space radius of every group of macrocells from the groups' occupancy bits (dims:
- * the group grid), 4 bits each, eight to a word: 0 for an occupied group, else the smallest
- * r >= 1 such that the groups within Chebyshev distance r of it include an occupied one, at
- * most 15. Every group within distance r - 1 is then empty, so a march in that group may skip
- * the whole cube at once. The set of groups within distance r of an occupied group grows by
- * one group along each axis per round (a cube dilates as three axis segments). */
-void group_radii(const std::vector<uint32_t>& occ, const int dims[3], std::vector<uint32_t>& out)
-{
-    const int nx = dims[0], ny = dims[1], nz = dims[2];
-    const size_t ng = (size_t)nx * ny * nz, sy = (size_t)nx, sz = (size_t)nx * ny;
-    std::vector<uint8_t> cur(ng), tmp(ng), rad(ng);
-    for (size_t g = 0; g < ng; ++g) {
-        cur[g] = (uint8_t)((occ[g >> 5] >> (g & 31)) & 1u);
-        rad[g] = cur[g] ? 0 : 15;
-    }
-    for (int r = 1; r < 15; ++r) {
-        for (int z = 0; z < nz; ++z)
-            for (int y = 0; y < ny; ++y)
-                for (int x = 0; x < nx; ++x) {
-                    const size_t i = z * sz + y * sy + x;
-                    tmp[i] = cur[i] | (x > 0 ? cur[i - 1] : 0) | (x < nx - 1 ? cur[i + 1] : 0);
-                }
-        for (int z = 0; z < nz; ++z)
-            for (int y = 0; y < ny; ++y)
-                for (int x = 0; x < nx; ++x) {
-                    const size_t i = z * sz + y * sy + x;
-                    cur[i] = tmp[i] | (y > 0 ? tmp[i - sy] : 0) | (y < ny - 1 ? tmp[i + sy] : 0);
-                }
-        for (int z = 0; z < nz; ++z)
-            for (int y = 0; y < ny; ++y)
-                for (int x = 0; x < nx; ++x) {
-                    const size_t i = z * sz + y * sy + x;
-                    tmp[i] = cur[i] | (z > 0 ? cur[i - sz] : 0) | (z < nz - 1 ? cur[i + sz] : 0);
-                }
-        cur.swap(tmp);
-        for (size_t g = 0; g < ng; ++g)
-            if (rad[g] == 15 && cur[g]) rad[g] = (uint8_t)r;
-    }
-    out.assign((ng + 7) / 8, 0u);
-    for (size_t g = 0; g < ng; ++g) out[g >> 3] |= (uint32_t)rad[g] << ((g & 7) * 4);
 }
 
 /* Rebuild the tracer's DevParams (and the LUT / macrocell maxima / gm_max that depend on it). */
@@ -1077,10 +1044,13 @@ int build_params(Tracer& t)
     HIP_TRY(hipMemcpy(t.lut.ptr, lut.data(), lut_n * sizeof(float), hipMemcpyHostToDevice));
     P.sigma_lut = t.lut.ptr;
     P.lut_max = lut_n - 1;
+    /* the next intensity with a positive sigma, for the macrocells' occupancy bits */
+    std::vector<uint32_t> next(lut_n);
+    uint32_t following = 0xffffffffu;
+    for (int i = lut_n - 1; i >= 0; --i) next[i] = following = lut[i] > 0.0f ? (uint32_t)i : following;
+    if ((st = t.lut_next.alloc(lut_n))) return st;
+    HIP_TRY(hipMemcpy(t.lut_next.ptr, next.data(), lut_n * sizeof(uint32_t), hipMemcpyHostToDevice));
     const int nmc = grid->mc[0] * grid->mc[1] * grid->mc[2];
-    if ((st = t.mc_sigma.alloc(nmc))) return st;
-    HIP_TRY(erd_launch_macro_sigma(grid->mm.ptr, t.lut.ptr, P.lut_max, t.mc_sigma.ptr, nmc, t.stream));
-    P.mc_sigma = t.mc_sigma.ptr;
     P.mc_shift = mc_shift;
     /* Woodcock majorants on their own fixed grid of 2^ER_WC_SHIFT-cell macrocells */
     P.wc_sigma = nullptr;
@@ -1127,23 +1097,19 @@ int build_params(Tracer& t)
         clipped = t.clip_bits.ptr;
         unclipped = t.clip_bits.ptr + mc_words;
     }
-    HIP_TRY(erd_launch_macro_bits(t.mc_sigma.ptr, clipped, t.mc_bits.ptr, nmc, mc_words, t.stream));
-    HIP_TRY(erd_launch_group_bits(t.mc_bits.ptr, unclipped, grid->mc[0], grid->mc[1], grid->mc[2], P.mc2_dim[0],
-                                  P.mc2_dim[1], P.mc2_dim[2], occ_base, P.mc3_base, g_words, t.stream));
-    {
-        std::vector<uint32_t> occ((size_t)g_words), radii;
-        HIP_TRY(hipMemcpyAsync(occ.data(), t.mc_bits.ptr + occ_base, occ.size() * sizeof(uint32_t), hipMemcpyDeviceToHost,
-                               t.stream));
-        HIP_TRY(hipStreamSynchronize(t.stream));
-        group_radii(occ, P.mc2_dim, radii);
-        HIP_TRY(hipMemcpyAsync(t.mc_bits.ptr + P.mc2_base, radii.data(), radii.size() * sizeof(uint32_t),
-                               hipMemcpyHostToDevice, t.stream));
-        HIP_TRY(hipStreamSynchronize(t.stream));
-    }
+    if ((st = t.group_tmp.alloc((size_t)ng * 2))) return st;
+    HIP_TRY(erd_launch_macro_bits(grid->mm.ptr, t.lut_next.ptr, P.lut_max, clipped, t.mc_bits.ptr, nmc, mc_words, t.stream));
+    HIP_TRY(erd_launch_group_tables(t.mc_bits.ptr, unclipped, t.group_tmp.ptr, grid->mc[0], grid->mc[1], grid->mc[2],
+                                    P.mc2_dim[0], P.mc2_dim[1], P.mc2_dim[2], occ_base, P.mc3_base, P.mc2_base, g_words,
+                                    t.stream));
     if (needs_gm(d)) {
-        if ((st = t.gm_tmp.alloc(1))) return st;
+        const size_t bricks = (size_t)((P.res[0] + 7) / 8) * ((P.res[1] + 7) / 8) * ((P.res[2] + 7) / 8);
+        if ((st = t.gm_tmp.alloc(1)) || (st = t.gm_bounds.alloc(bricks))) return st;
         HIP_TRY(hipMemsetAsync(t.gm_tmp.ptr, 0, sizeof(unsigned int), t.stream));
-        HIP_TRY(erd_launch_gm_max(t.params.ptr, t.gm_tmp.ptr, t.stream));
+        bool prune = true;   /* where the kernel's bound on a brick holds (see there) */
+        for (int i = 0; i < 3; ++i) prune = prune && P.spacing[i] > 0.0f && P.spacing[i] < 3.0e38f && P.res[i] <= 65536;
+        HIP_TRY(erd_launch_gm_max(t.params.ptr, vol->vox.ptr, t.gm_bounds.ptr, t.gm_tmp.ptr, P.res[0], P.res[1], P.res[2], prune,
+                                  t.stream));
         unsigned int bits = 0;
         HIP_TRY(hipMemcpyAsync(&bits, t.gm_tmp.ptr, sizeof(bits), hipMemcpyDeviceToHost, t.stream));
         HIP_TRY(hipStreamSynchronize(t.stream));

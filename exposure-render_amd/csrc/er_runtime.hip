@@ -189,12 +189,19 @@ template<class T> struct DevBuf {
         n = count;
         return ER_OK;
     }
+    /* at least count elements: for buffers whose size varies from call to call */
+    int reserve(size_t count) { return ptr && n >= count ? ER_OK : alloc(count); }
     void release()
     {
         if (ptr) (void)hipFree(ptr);
         ptr = nullptr;
         n = 0;
     }
+};
+
+/* a buffer of one call */
+template<class T> struct ScopedBuf : DevBuf<T> {
+    ~ScopedBuf() { this->release(); }
 };
 
 /* ---- host-side restatements used to build device data (same op order as the kernels) -- */
@@ -306,7 +313,10 @@ struct Volume {
     std::map<int, MacroGrid> grids;
     int mc_shift = 3;               /* default brick: 8 cells, coarser for very large volumes */
     uint16_t vmax = 0;
-    uint64_t upload = 0;            /* upload serial number (autotuner cache key) */
+    uint64_t upload = 0;            /* upload serial number (key of what is derived from the voxels) */
+    /* the gradient-magnitude maximum of this upload, and the geometry it was taken with */
+    float gm_max = 0.0f, gm_geometry[6] = {0, 0, 0, 0, 0, 0};
+    uint64_t gm_upload = 0;
     ~Volume()
     {
         vox.release(); cells.release(); top.release();
@@ -360,6 +370,55 @@ struct PassSet {
     }
 };
 
+/* The work buffers of er_adjoint_lut, kept with the tracer: two sets of one pass's queues, so
+ * that pass k + 1's primary and shading kernels (first stream) overlap pass k's adjoint kernels
+ * (second stream), as the forward passes do. Made by the first call and resized with the film. */
+struct AdjWork {
+    struct Set {
+        DevBuf<uint32_t> s1s, s2s, counts, lcount;
+        DevBuf<float> tvis;
+        DevBuf<float4> frame;
+        DevBuf<char> queue, events, jobs;
+        DevBuf<uint2> list;
+        hipEvent_t shaded = nullptr, done = nullptr;
+        bool pending = false;
+    } set[2];
+    DevBuf<uint32_t> d1, d2;
+    DevBuf<float> dldr, partials;
+    DevBuf<float4> adj;
+    DevBuf<double> out;
+    int fit(size_t n, size_t blocks, size_t per_block)
+    {
+        int st;
+        size_t rs = 0, re = 0, rj = 0;
+        erd_pass_record_sizes(&rs, &re, &rj);
+        if ((st = d1.alloc(n)) || (st = d2.alloc(n)) || (st = dldr.alloc(n * 3)) || (st = adj.alloc(n)) ||
+            (st = partials.alloc(3 * blocks * per_block)) || (st = out.alloc(per_block)))
+            return st;
+        for (Set& A : set) {
+            if ((st = A.s1s.alloc(n)) || (st = A.s2s.alloc(n)) || (st = A.counts.alloc(4)) || (st = A.lcount.alloc(1)) ||
+                (st = A.tvis.alloc(2 * n)) || (st = A.frame.alloc(n)) || (st = A.queue.alloc(n * rs)) ||
+                (st = A.events.alloc(n * re)) || (st = A.jobs.alloc(2 * n * rj)) || (st = A.list.alloc(n)))
+                return st;
+            if (!A.shaded) HIP_TRY(hipEventCreateWithFlags(&A.shaded, hipEventDisableTiming));
+            if (!A.done) HIP_TRY(hipEventCreateWithFlags(&A.done, hipEventDisableTiming));
+            A.pending = false;
+        }
+        return ER_OK;
+    }
+    void release()
+    {
+        for (Set& A : set) {
+            A.s1s.release(); A.s2s.release(); A.counts.release(); A.lcount.release(); A.tvis.release(); A.frame.release();
+            A.queue.release(); A.events.release(); A.jobs.release(); A.list.release();
+            if (A.shaded) (void)hipEventDestroy(A.shaded);
+            if (A.done) (void)hipEventDestroy(A.done);
+            A.shaded = A.done = nullptr;
+        }
+        d1.release(); d2.release(); dldr.release(); partials.release(); adj.release(); out.release();
+    }
+};
+
 struct Tracer {
     er_tracer_desc desc{};
     int W = 0, H = 0;
@@ -374,10 +433,15 @@ struct Tracer {
     size_t lds_bytes = 0;
     int lut_lds = 0;
     DevBuf<DevParams> params;
+    DevParams* params_pinned = nullptr;   /* the copy the upload reads */
+    /* what the tables above (opacity, occupancy, radii, majorants) were built from, by value:
+     * they are rebuilt when it changes, not with every bind */
+    std::string tables_key;
     DevBuf<unsigned long long> counters;
     DevBuf<unsigned int> gm_tmp;
     DevBuf<float> gm_bounds;
     DevBuf<char> bilateral;
+    std::string bilateral_key;       /* the radius and sigmas of the tables in it */
     DevBuf<char> focus;              /* the autofocus kernel's workspace, made by its first call */
     DevParams host_params{};
     uint64_t built_version = 0;
@@ -387,6 +451,7 @@ struct Tracer {
     std::vector<float> tf_lut;       /* node table (er_set_tf_lut), empty when the PLFs are used */
     float tf_scale = 0.0f;
     DevBuf<float> tf_lut_dev;
+    AdjWork adjoint;
     /* launch configuration (er_autotune / er_set_tune): brick edge 2^mc_shift (0: the
      * volume's default), primary tiles 2^tile_shift pixels wide, persistent primary
      * workgroups per CU (0: the library default) */
@@ -409,6 +474,8 @@ struct Tracer {
         seeds1.release(); seeds2.release(); lut.release(); lut_next.release(); wc_sigma.release(); group_tmp.release(); params.release();
         mc_bits.release(); clip_bits.release(); counters.release(); gm_tmp.release(); gm_bounds.release(); bilateral.release(); focus.release();
         tile_cost.release(); tile_order.release();
+        tf_lut_dev.release(); adjoint.release();
+        if (params_pinned) (void)hipHostFree(params_pinned);
         if (stream) (void)hipStreamDestroy(stream);
         if (stream2) (void)hipStreamDestroy(stream2);
     }
@@ -1023,43 +1090,80 @@ int build_params(Tracer& t)
     P.opacity = d.opacity; P.glossiness = d.glossiness;
     P.diffuse = d.diffuse; P.specular = d.specular; P.emission = d.emission;
 
+    /* what the tracer's tables depend on: the volume's contents and brick size, the opacity (by
+     * node table or PLF), and - through the occupancy bits - the clipping objects with the
+     * geometry their classes are taken in */
+    const bool woodcock = s.estimator == ER_ESTIMATOR_FULL && s.sampler == ER_SAMPLER_WOODCOCK;
+    /* rounded up to a power of two, so that a moving camera seldom changes it */
+    double edge_ext = 0.0;
+    if (P.clip_count > 0) {
+        int e = 0;
+        (void)frexp(ray_origin_bound(P, objs) * 1.0e-5, &e);
+        edge_ext = ldexp(1.0, e);
+    }
+    std::string key;
+    auto add = [&key](const void* data, size_t bytes) { key.append((const char*)data, bytes); };
+    const int head[3] = {mc_shift, woodcock, (int)t.tf_lut.size()};
+    add(&vol->upload, sizeof(vol->upload));
+    add(head, sizeof(head));
+    add(&s.density_scale, sizeof(float));
+    if (t.tf_lut.empty()) {
+        add(&d.opacity, sizeof(d.opacity));
+    } else {
+        add(t.tf_lut.data(), t.tf_lut.size() * sizeof(float));
+        add(&t.tf_scale, sizeof(float));
+    }
+    if (P.clip_count > 0) {
+        add(P.clips, (size_t)P.clip_count * sizeof(P.clips[0]));
+        add(&edge_ext, sizeof(edge_ext));
+        add(P.minp, sizeof(P.minp)); add(P.size, sizeof(P.size)); add(P.invsize, sizeof(P.invsize));
+    }
+    const bool rebuild = key != t.tables_key;
+    if (rebuild) t.tables_key.clear();
+
     /* node-table transfer function */
     P.tf_lut = nullptr;
     P.tf_lut_scale = t.tf_scale;
     if (!t.tf_lut.empty()) {
         if ((st = t.tf_lut_dev.alloc(t.tf_lut.size()))) return st;
-        HIP_TRY(hipMemcpy(t.tf_lut_dev.ptr, t.tf_lut.data(), t.tf_lut.size() * sizeof(float), hipMemcpyHostToDevice));
+        if (rebuild)
+            HIP_TRY(hipMemcpyAsync(t.tf_lut_dev.ptr, t.tf_lut.data(), t.tf_lut.size() * sizeof(float), hipMemcpyHostToDevice,
+                                   t.stream));
         P.tf_lut = t.tf_lut_dev.ptr;
     }
 
-    /* exact opacity LUT over the intensities the volume can produce */
+    /* exact opacity LUT over the intensities the volume can produce, and for each of them the
+     * next intensity with a positive sigma, for the macrocells' occupancy bits (both until the
+     * stream is waited for below) */
     const int lut_n = (int)vol->vmax + 1;
-    std::vector<float> lut(lut_n);
-    for (int i = 0; i < lut_n; ++i) {
-        const float o = t.tf_lut.empty() ? plf_eval_host(d.opacity, (float)i)
-                                         : erd::tf_lut_eval(t.tf_lut.data(), t.tf_scale, (float)i, 0);
-        lut[i] = s.density_scale * o;
+    std::vector<float> lut;
+    std::vector<uint32_t> next, classes;
+    if ((st = t.lut.reserve(lut_n)) || (st = t.lut_next.reserve(lut_n))) return st;
+    if (rebuild) {
+        lut.resize(lut_n);
+        next.resize(lut_n);
+        for (int i = 0; i < lut_n; ++i) {
+            const float o = t.tf_lut.empty() ? plf_eval_host(d.opacity, (float)i)
+                                             : erd::tf_lut_eval(t.tf_lut.data(), t.tf_scale, (float)i, 0);
+            lut[i] = s.density_scale * o;
+        }
+        uint32_t following = 0xffffffffu;
+        for (int i = lut_n - 1; i >= 0; --i) next[i] = following = lut[i] > 0.0f ? (uint32_t)i : following;
+        HIP_TRY(hipMemcpyAsync(t.lut.ptr, lut.data(), lut_n * sizeof(float), hipMemcpyHostToDevice, t.stream));
+        HIP_TRY(hipMemcpyAsync(t.lut_next.ptr, next.data(), lut_n * sizeof(uint32_t), hipMemcpyHostToDevice, t.stream));
     }
-    if ((st = t.lut.alloc(lut_n))) return st;
-    HIP_TRY(hipMemcpy(t.lut.ptr, lut.data(), lut_n * sizeof(float), hipMemcpyHostToDevice));
     P.sigma_lut = t.lut.ptr;
     P.lut_max = lut_n - 1;
-    /* the next intensity with a positive sigma, for the macrocells' occupancy bits */
-    std::vector<uint32_t> next(lut_n);
-    uint32_t following = 0xffffffffu;
-    for (int i = lut_n - 1; i >= 0; --i) next[i] = following = lut[i] > 0.0f ? (uint32_t)i : following;
-    if ((st = t.lut_next.alloc(lut_n))) return st;
-    HIP_TRY(hipMemcpy(t.lut_next.ptr, next.data(), lut_n * sizeof(uint32_t), hipMemcpyHostToDevice));
     const int nmc = grid->mc[0] * grid->mc[1] * grid->mc[2];
     P.mc_shift = mc_shift;
     /* Woodcock majorants on their own fixed grid of 2^ER_WC_SHIFT-cell macrocells */
     P.wc_sigma = nullptr;
-    if (s.estimator == ER_ESTIMATOR_FULL && s.sampler == ER_SAMPLER_WOODCOCK) {
+    if (woodcock) {
         MacroGrid* wg = volume_grid(*vol, ER_WC_SHIFT, st);
         if (!wg) return st;
         const int nw = wg->mc[0] * wg->mc[1] * wg->mc[2];
         if ((st = t.wc_sigma.alloc(nw))) return st;
-        HIP_TRY(erd_launch_macro_sigma(wg->mm.ptr, t.lut.ptr, P.lut_max, t.wc_sigma.ptr, nw, t.stream));
+        if (rebuild) HIP_TRY(erd_launch_macro_sigma(wg->mm.ptr, t.lut.ptr, P.lut_max, t.wc_sigma.ptr, nw, t.stream));
         P.wc_sigma = t.wc_sigma.ptr;
         for (int i = 0; i < 3; ++i) P.wc_dim[i] = wg->mc[i];
     }
@@ -1074,65 +1178,90 @@ int build_params(Tracer& t)
     P.mc3_base = mc_words + r_words;
     P.mc_words = mc_words + r_words + g_words;
     const int occ_base = P.mc_words;
-    if ((st = t.mc_bits.alloc(P.mc_words + g_words))) return st;
+    if ((st = t.mc_bits.alloc(P.mc_words + g_words)) || (st = t.group_tmp.alloc((size_t)ng * 2))) return st;
     P.mc_bits = t.mc_bits.ptr;
     t.lut_lds = (size_t)lut_n * sizeof(float) <= 32768u;
     t.lds_bytes = (size_t)P.mc_words * 4 + (t.lut_lds ? (size_t)lut_n * sizeof(float) : 0);
+    if (rebuild) {
+        /* macrocells wholly clipped away count as empty */
+        const uint32_t* clipped = nullptr;
+        const uint32_t* unclipped = nullptr;
+        if (P.clip_count > 0) {
+            std::vector<uint32_t> free;
+            clip_classes(P, nmc, edge_ext, classes, free);
+            classes.insert(classes.end(), free.begin(), free.end());
+            if ((st = t.clip_bits.alloc(classes.size()))) return st;
+            HIP_TRY(hipMemcpyAsync(t.clip_bits.ptr, classes.data(), classes.size() * sizeof(uint32_t), hipMemcpyHostToDevice,
+                                   t.stream));
+            clipped = t.clip_bits.ptr;
+            unclipped = t.clip_bits.ptr + mc_words;
+        }
+        HIP_TRY(erd_launch_macro_bits(grid->mm.ptr, t.lut_next.ptr, P.lut_max, clipped, t.mc_bits.ptr, nmc, mc_words, t.stream));
+        HIP_TRY(erd_launch_group_tables(t.mc_bits.ptr, unclipped, t.group_tmp.ptr, grid->mc[0], grid->mc[1], grid->mc[2],
+                                        P.mc2_dim[0], P.mc2_dim[1], P.mc2_dim[2], occ_base, P.mc3_base, P.mc2_base, g_words,
+                                        t.stream));
+    }
 
     if ((st = t.params.alloc(1))) return st;
+    if (!t.params_pinned) HIP_TRY(hipHostMalloc((void**)&t.params_pinned, sizeof(DevParams), hipHostMallocDefault));
+    /* an upload the last call left in the stream has read the pinned copy before it changes */
+    auto upload = [&t, &P]() -> int {
+        HIP_TRY(hipStreamSynchronize(t.stream));
+        *t.params_pinned = P;
+        HIP_TRY(hipMemcpyAsync(t.params.ptr, t.params_pinned, sizeof(P), hipMemcpyHostToDevice, t.stream));
+        return ER_OK;
+    };
     P.gm_inv = 0.0f;
     t.gm_max = 0.0f;
-    HIP_TRY(hipMemcpyAsync(t.params.ptr, &P, sizeof(P), hipMemcpyHostToDevice, t.stream));
-    /* macrocells wholly clipped away count as empty (the bits kernel reads the clipping objects
-     * from the parameters just uploaded) */
-    const uint32_t* clipped = nullptr;
-    const uint32_t* unclipped = nullptr;
-    if (P.clip_count > 0) {
-        std::vector<uint32_t> gone, free;
-        clip_classes(P, nmc, ray_origin_bound(P, objs) * 1.0e-5, gone, free);
-        gone.insert(gone.end(), free.begin(), free.end());
-        if ((st = t.clip_bits.alloc(gone.size()))) return st;
-        HIP_TRY(hipMemcpyAsync(t.clip_bits.ptr, gone.data(), gone.size() * sizeof(uint32_t), hipMemcpyHostToDevice, t.stream));
-        HIP_TRY(hipStreamSynchronize(t.stream));
-        clipped = t.clip_bits.ptr;
-        unclipped = t.clip_bits.ptr + mc_words;
-    }
-    if ((st = t.group_tmp.alloc((size_t)ng * 2))) return st;
-    HIP_TRY(erd_launch_macro_bits(grid->mm.ptr, t.lut_next.ptr, P.lut_max, clipped, t.mc_bits.ptr, nmc, mc_words, t.stream));
-    HIP_TRY(erd_launch_group_tables(t.mc_bits.ptr, unclipped, t.group_tmp.ptr, grid->mc[0], grid->mc[1], grid->mc[2],
-                                    P.mc2_dim[0], P.mc2_dim[1], P.mc2_dim[2], occ_base, P.mc3_base, P.mc2_base, g_words,
-                                    t.stream));
     if (needs_gm(d)) {
-        const size_t bricks = (size_t)((P.res[0] + 7) / 8) * ((P.res[1] + 7) / 8) * ((P.res[2] + 7) / 8);
-        if ((st = t.gm_tmp.alloc(1)) || (st = t.gm_bounds.alloc(bricks))) return st;
-        HIP_TRY(hipMemsetAsync(t.gm_tmp.ptr, 0, sizeof(unsigned int), t.stream));
-        bool prune = true;   /* where the kernel's bound on a brick holds (see there) */
-        for (int i = 0; i < 3; ++i) prune = prune && P.spacing[i] > 0.0f && P.spacing[i] < 3.0e38f && P.res[i] <= 65536;
-        HIP_TRY(erd_launch_gm_max(t.params.ptr, vol->vox.ptr, t.gm_bounds.ptr, t.gm_tmp.ptr, P.res[0], P.res[1], P.res[2], prune,
-                                  t.stream));
-        unsigned int bits = 0;
-        HIP_TRY(hipMemcpyAsync(&bits, t.gm_tmp.ptr, sizeof(bits), hipMemcpyDeviceToHost, t.stream));
-        HIP_TRY(hipStreamSynchronize(t.stream));
-        memcpy(&t.gm_max, &bits, 4);
+        /* the volume's: taken once per upload and geometry */
+        float geometry[6];
+        for (int i = 0; i < 3; ++i) { geometry[i] = P.spacing[i]; geometry[3 + i] = P.size[i]; }
+        if (vol->gm_upload != vol->upload || memcmp(geometry, vol->gm_geometry, sizeof(geometry)) != 0) {
+            const size_t bricks = (size_t)((P.res[0] + 7) / 8) * ((P.res[1] + 7) / 8) * ((P.res[2] + 7) / 8);
+            DevBuf<float>& bounds = t.gm_bounds;
+            if ((st = t.gm_tmp.alloc(1)) || (st = bounds.reserve(bricks)) || (st = upload())) return st;
+            HIP_TRY(hipMemsetAsync(t.gm_tmp.ptr, 0, sizeof(unsigned int), t.stream));
+            bool prune = true;   /* where the kernel's bound on a brick holds (see there) */
+            for (int i = 0; i < 3; ++i) prune = prune && P.spacing[i] > 0.0f && P.spacing[i] < 3.0e38f && P.res[i] <= 65536;
+            HIP_TRY(erd_launch_gm_max(t.params.ptr, vol->vox.ptr, bounds.ptr, t.gm_tmp.ptr, P.res[0], P.res[1], P.res[2], prune,
+                                      t.stream));
+            unsigned int bits = 0;
+            HIP_TRY(hipMemcpyAsync(&bits, t.gm_tmp.ptr, sizeof(bits), hipMemcpyDeviceToHost, t.stream));
+            HIP_TRY(hipStreamSynchronize(t.stream));
+            memcpy(&vol->gm_max, &bits, 4);
+            memcpy(vol->gm_geometry, geometry, sizeof(geometry));
+            vol->gm_upload = vol->upload;
+        }
+        t.gm_max = vol->gm_max;
         P.gm_inv = t.gm_max > 0.0f ? 1.0f / t.gm_max : 0.0f;
-        HIP_TRY(hipMemcpyAsync(t.params.ptr, &P, sizeof(P), hipMemcpyHostToDevice, t.stream));
     }
+    if ((st = upload())) return st;
     /* bilateral tables (Source/filter.h:34-40) */
     if (s.estimator == ER_ESTIMATOR_FULL && s.bilateral) {
         const int R = s.bilateral_radius;
         if (R < 0 || R > 32) return set_error(ER_ERROR, "bilateral radius must be in [0, 32]");
-        std::vector<char> bp(erd_bilateral_params_size(), 0);
-        int* radius = (int*)bp.data();
-        float* kd = (float*)(bp.data() + sizeof(int));
-        float* gs = kd + 65;
-        *radius = R;
         const float ss = s.bilateral_sigma_spatial, sr = s.bilateral_sigma_range;
-        for (int k = -R; k <= R; ++k) kd[k + R] = erm::expf_(-((float)(k * k)) / (2.0f * ss * ss));
-        for (int q = 0; q < 256; ++q) gs[q] = erm::expf_(-((float)(q * q)) / (2.0f * sr * sr));
-        if ((st = t.bilateral.alloc(bp.size()))) return st;
-        HIP_TRY(hipMemcpyAsync(t.bilateral.ptr, bp.data(), bp.size(), hipMemcpyHostToDevice, t.stream));
+        std::string filter((const char*)&R, sizeof(R));
+        filter.append((const char*)&ss, sizeof(ss)).append((const char*)&sr, sizeof(sr));
+        if (filter != t.bilateral_key) {
+            t.bilateral_key.clear();
+            std::vector<char> bp(erd_bilateral_params_size(), 0);
+            int* radius = (int*)bp.data();
+            float* kd = (float*)(bp.data() + sizeof(int));
+            float* gs = kd + 65;
+            *radius = R;
+            for (int k = -R; k <= R; ++k) kd[k + R] = erm::expf_(-((float)(k * k)) / (2.0f * ss * ss));
+            for (int q = 0; q < 256; ++q) gs[q] = erm::expf_(-((float)(q * q)) / (2.0f * sr * sr));
+            if ((st = t.bilateral.alloc(bp.size()))) return st;
+            HIP_TRY(hipMemcpy(t.bilateral.ptr, bp.data(), bp.size(), hipMemcpyHostToDevice));
+            t.bilateral_key = filter;
+        }
     }
-    HIP_TRY(hipStreamSynchronize(t.stream));
+    if (rebuild) {
+        HIP_TRY(hipStreamSynchronize(t.stream));
+        t.tables_key = key;
+    }
     t.built_version = g_scene_version;
     return ER_OK;
 }
@@ -2206,80 +2335,48 @@ ER_API int er_adjoint_lut(int tracer_id, const uint32_t* seeds1, const uint32_t*
     const size_t n = (size_t)t->W * t->H;
     const int blocks = ER_ADJ_BLOCKS;
     const size_t per_block = erd_adj_partials_per_block();
-    size_t rs = 0, re = 0, rj = 0;
-    erd_pass_record_sizes(&rs, &re, &rj);
-    /* two buffer sets: pass k + 1's primary and shading kernels (first stream) overlap pass k's
-     * adjoint kernels (second stream), as the forward passes do */
-    struct AdjSet {
-        DevBuf<uint32_t> s1s, s2s, counts, lcount;
-        DevBuf<float> tvis;
-        DevBuf<float4> frame;
-        DevBuf<char> queue, events, jobs;
-        DevBuf<uint2> list;
-        hipEvent_t shaded = nullptr, done = nullptr;
-        bool pending = false;
-        ~AdjSet()
-        {
-            if (shaded) (void)hipEventDestroy(shaded);
-            if (done) (void)hipEventDestroy(done);
-        }
-    } S[2];
-    DevBuf<uint32_t> d1, d2;
-    DevBuf<float> dldr, partials;
-    DevBuf<float4> adj;
-    DevBuf<double> out;
-    if ((st = d1.alloc(n)) || (st = d2.alloc(n)) || (st = dldr.alloc(n * 3)) || (st = adj.alloc(n)) ||
-        (st = partials.alloc(3 * (size_t)blocks * per_block)) || (st = out.alloc(per_block)))
-        return st;
-    for (AdjSet& A : S) {
-        if ((st = A.s1s.alloc(n)) || (st = A.s2s.alloc(n)) || (st = A.counts.alloc(4)) || (st = A.lcount.alloc(1)) ||
-            (st = A.tvis.alloc(2 * n)) || (st = A.frame.alloc(n)) || (st = A.queue.alloc(n * rs)) ||
-            (st = A.events.alloc(n * re)) || (st = A.jobs.alloc(2 * n * rj)) || (st = A.list.alloc(n)))
-            return st;
-        HIP_TRY(hipEventCreateWithFlags(&A.shaded, hipEventDisableTiming));
-        HIP_TRY(hipEventCreateWithFlags(&A.done, hipEventDisableTiming));
-        HIP_TRY(hipMemset(A.counts.ptr, 0, 4 * sizeof(uint32_t)));
-        HIP_TRY(hipMemset(A.lcount.ptr, 0, sizeof(uint32_t)));
-    }
+    AdjWork& W = t->adjoint;
+    if ((st = W.fit(n, blocks, per_block))) return st;
     hipStream_t s = t->stream, s2 = t->stream2;
-    HIP_TRY(hipMemcpy(d1.ptr, seeds1, n * 4, hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(d2.ptr, seeds2, n * 4, hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(dldr.ptr, dL_drunning_xyz, n * 12, hipMemcpyHostToDevice));
-    HIP_TRY(hipMemset(out.ptr, 0, per_block * sizeof(double)));
+    HIP_TRY(hipMemcpyAsync(W.d1.ptr, seeds1, n * 4, hipMemcpyHostToDevice, s));
+    HIP_TRY(hipMemcpyAsync(W.d2.ptr, seeds2, n * 4, hipMemcpyHostToDevice, s));
+    HIP_TRY(hipMemcpyAsync(W.dldr.ptr, dL_drunning_xyz, n * 12, hipMemcpyHostToDevice, s));
+    HIP_TRY(erd_launch_zero_words((uint32_t*)W.out.ptr, per_block * sizeof(double) / 4, s));
+    for (AdjWork::Set& A : W.set) HIP_TRY(erd_launch_adj_reset(A.counts.ptr, A.lcount.ptr, s));
     const int shade_blocks = std::max(1, std::min((int)((n + 255) / 256), 2048));
     const size_t lds_bits = (size_t)t->host_params.mc_words * 4;
     float cur_w = -1.0f;
     /* the running estimate after N passes is the mean of the filtered frames of passes 2..N
      * (the first pass is discarded, Q1), or the first frame when N == 1 */
     for (int k = 1; k <= passes; ++k) {
-        AdjSet& A = S[k & 1];
+        AdjWork::Set& A = W.set[k & 1];
         const float w = passes == 1 ? 1.0f : (k >= 2 ? 1.0f / (float)(passes - 1) : 0.0f);
         if (A.pending) HIP_TRY(hipStreamWaitEvent(s, A.done, 0));
         if (w != 0.0f) {
-            HIP_TRY(hipMemcpyAsync(A.s1s.ptr, d1.ptr, n * 4, hipMemcpyDeviceToDevice, s));
-            HIP_TRY(hipMemcpyAsync(A.s2s.ptr, d2.ptr, n * 4, hipMemcpyDeviceToDevice, s));
+            HIP_TRY(hipMemcpyAsync(A.s1s.ptr, W.d1.ptr, n * 4, hipMemcpyDeviceToDevice, s));
+            HIP_TRY(hipMemcpyAsync(A.s2s.ptr, W.d2.ptr, n * 4, hipMemcpyDeviceToDevice, s));
         }
         /* the forward pass's primary and shading kernels: decisions, queues, final seeds */
-        HIP_TRY(erd_launch_primary_shade(t->params.ptr, A.frame.ptr, d1.ptr, d2.ptr, A.queue.ptr, A.counts.ptr, A.events.ptr,
+        HIP_TRY(erd_launch_primary_shade(t->params.ptr, A.frame.ptr, W.d1.ptr, W.d2.ptr, A.queue.ptr, A.counts.ptr, A.events.ptr,
                                          A.jobs.ptr, t->W, t->H, t->lut_lds, t->lds_bytes, lds_bits, shade_blocks,
                                          primary_blocks(*t), t->tile_shift, s));
         HIP_TRY(hipEventRecord(A.shaded, s));
         HIP_TRY(hipStreamWaitEvent(s2, A.shaded, 0));
         if (w != 0.0f) {
             if (w != cur_w) {
-                HIP_TRY(erd_launch_adj_filter_t(dldr.ptr, adj.ptr, t->W, t->H, w, s2));
+                HIP_TRY(erd_launch_adj_filter_t(W.dldr.ptr, W.adj.ptr, t->W, t->H, w, s2));
                 cur_w = w;
             }
-            HIP_TRY(erd_launch_adj_wavefront(t->params.ptr, A.counts.ptr, A.jobs.ptr, A.events.ptr, A.queue.ptr, adj.ptr,
+            HIP_TRY(erd_launch_adj_wavefront(t->params.ptr, A.counts.ptr, A.jobs.ptr, A.events.ptr, A.queue.ptr, W.adj.ptr,
                                              A.tvis.ptr, A.frame.ptr, A.list.ptr, A.lcount.ptr, A.s1s.ptr, A.s2s.ptr,
-                                             partials.ptr, blocks, (int)n, t->lds_bytes, s2));
-            HIP_TRY(erd_launch_adj_reduce(partials.ptr, 3 * blocks, out.ptr, s2));
+                                             W.partials.ptr, blocks, (int)n, t->lds_bytes, s2));
+            HIP_TRY(erd_launch_adj_reduce(W.partials.ptr, 3 * blocks, W.out.ptr, s2));
         }
         HIP_TRY(erd_launch_adj_reset(A.counts.ptr, A.lcount.ptr, s2));
         HIP_TRY(hipEventRecord(A.done, s2));
         A.pending = true;
     }
-    HIP_TRY(hipMemcpyAsync(dL_dlut, out.ptr, per_block * sizeof(double), hipMemcpyDeviceToHost, s2));
+    HIP_TRY(hipMemcpyAsync(dL_dlut, W.out.ptr, per_block * sizeof(double), hipMemcpyDeviceToHost, s2));
     HIP_TRY(hipStreamSynchronize(s2));
     if ((st = sync_tracer(*t))) return st;
     return ER_OK;
@@ -2374,10 +2471,10 @@ ER_API int er_adjoint_value(int tracer_id, const uint32_t* seeds1, const uint32_
     std::vector<float> sig((size_t)P.lut_max + 1);
     for (int i = 0; i <= P.lut_max; ++i)
         sig[i] = P.density_scale * erd::tf_lut_eval(eval_lut, t->tf_scale, (float)i, 0);
-    DevBuf<uint32_t> d1, d2, qc;
-    DevBuf<float> lut_e, sig_e;
-    DevBuf<float4> frame, running;
-    DevBuf<uchar4> display;
+    ScopedBuf<uint32_t> d1, d2, qc;
+    ScopedBuf<float> lut_e, sig_e;
+    ScopedBuf<float4> frame, running;
+    ScopedBuf<uchar4> display;
     if ((st = d1.alloc(n)) || (st = d2.alloc(n)) || (st = qc.alloc(4)) || (st = lut_e.alloc(ER_TF_LUT_NODES * 4)) ||
         (st = sig_e.alloc(sig.size())) || (st = frame.alloc(n)) || (st = running.alloc(n)) || (st = display.alloc(n)))
         return st;

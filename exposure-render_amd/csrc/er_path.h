@@ -1262,31 +1262,6 @@ __device__ int visible_defer(const DevParams& p, f3 P1, f3 P2, Rng& rng, Cnt& cn
     return 2;
 }
 
-/* Visible (transport.h:46-56) -> Intersect (transport.h:30-44) */
-template<int FULL, int COUNT>
-__device__ bool visible(const DevParams& p, const Tables& T, f3 P1, f3 P2, Rng& rng, Cnt& cnt)
-{
-    if (!p.shadows) return true;
-    const Ray r = shadow_ray(p, P1, P2);
-    if (COUNT) cnt.shadow_rays++;
-    if (intersects_any_light(p, r)) return false;
-    if (p.object_count > 0 && intersects_any_object(p, r)) return false;
-    float Tt; f3 P;
-    const Tables& Tb = T;
-    if (FULL && p.sampler == ER_SAMPLER_WOODCOCK) {
-        /* own stream for the march; the path's stream takes the two draws of a ray-march test
-         * when the ray meets the volume (Q18) */
-        float nearT, farT;
-        if (!intersect_box(r, ld3(p.minp), ld3(p.maxp), nearT, farT)) return true;
-        Rng rs = shadow_stream(rng);
-        (void)rng.next_bits();
-        (void)rng.next_bits();
-        return !march<FULL, COUNT>(p, Tb, r, false, rs, Tt, P, cnt);
-    }
-    if (march<FULL, COUNT>(p, Tb, r, false, rng, Tt, P, cnt)) return false;
-    return true;
-}
-
 /* SampleLightSurface (lights.h:28-41) */
 __device__ void sample_light_surface(const DevParams& p, const DevLight& L, float u0, float u1, float u2, f3& P, f3& N, float& U, float& V)
 {
@@ -1348,49 +1323,6 @@ __device__ void sample_light_surface(const DevParams& p, const DevLight& L, floa
 
 struct Sample { float comp, dir0, dir1, uvw0, uvw1, uvw2, lightnum, film0, film1, lens0, lens1; };
 
-/* EstimateDirectLight (transport.h:58-113) */
-template<int FULL, int COUNT>
-__device__ f3 estimate_direct(const DevParams& p, const Tables& T, const DevLight& L, int light_pos, const Sample& smp, f3 SEP, f3 SEN, f3 Wo,
-                              const Shader& sh, Rng& rng, Cnt& cnt)
-{
-    f3 Ld = mk(0.0f, 0.0f, 0.0f);
-    f3 SP, SN; float su, sv;
-    sample_light_surface(p, L, smp.uvw0, smp.uvw1, smp.uvw2, SP, SN, su, sv);
-    f3 Wi = nrm(sub(SP, SEP));
-    f3 Li = scl(L.multiplier, eval_texture(p, L.texture_id, su, sv));
-    if (L.one_sided && dot(sub(SEP, SP), SN) < 0.0f) Li = mk(0.0f, 0.0f, 0.0f);
-    if (L.unit == ER_UNIT_LUX) Li = mk(Li.x / L.area, Li.y / L.area, Li.z / L.area);
-    f3 F = shader_f<FULL>(sh, Wo, Wi);
-    float BsdfPdf = shader_pdf<FULL>(sh, Wo, Wi);
-    if (!black(Li) && !black(F) && BsdfPdf > 0.0f && visible<FULL, COUNT>(p, T, SEP, SP, rng, cnt)) {
-        const f3 d = sub(SEP, SP);
-        const float LightPdf = dot(d, d) / (absdot(SN, neg(Wi)) * L.area);
-        const float Weight = power_heuristic(LightPdf, BsdfPdf);
-        const f3 FL = mul(F, Li);
-        if (sh.brdf) Ld = add(Ld, scl(absdot(Wi, SEN) * Weight / LightPdf, FL));
-        else if (FULL) Ld = add(Ld, scl(Weight / LightPdf, FL));
-        else Ld = add(Ld, mk(FL.x / LightPdf, FL.y / LightPdf, FL.z / LightPdf));
-    }
-    if (!FULL) return Ld;
-
-    F = shader_sample_f(sh, Wo, Wi, BsdfPdf, smp.comp, smp.dir0, smp.dir1);
-    if (black(F) || BsdfPdf <= 0.0f) return Ld;
-    Ray r2;
-    r2.O = SEP; r2.D = Wi; r2.MinT = 0.0f; r2.MaxT = 1000000.0f;
-    float T2; f3 P2, N2, Le2;
-    const int idx2 = intersect_lights(p, r2, false, T2, P2, N2, Le2);
-    if (idx2 < 0 || idx2 != light_pos) return Ld;
-    if (!black(Le2) && visible<FULL, COUNT>(p, T, SEP, P2, rng, cnt)) {
-        const f3 d = sub(SEP, P2);
-        const float LightPdf = dot(d, d) / (absdot(N2, neg(Wi)) * L.area);
-        const float Weight = power_heuristic(BsdfPdf, LightPdf);
-        const f3 FL = mul(F, Le2);
-        if (sh.brdf) Ld = add(Ld, scl(absdot(Wi, SEN) * Weight / BsdfPdf, FL));
-        else Ld = add(Ld, scl(Weight / BsdfPdf, FL));
-    }
-    return Ld;
-}
-
 /* The shader of an event (transport.h:133-150). Volume event (obj < 0): BRDF in compat (Q9);
  * in full mode the shading type picks BRDF or phase function, the stochastic types with one
  * extra draw (design: scatterevent.h:155-212). Object event: BRDF with diffuse, specular and
@@ -1439,32 +1371,10 @@ __device__ __forceinline__ void event_shader(const DevParams& p, float I, int ob
     sh.Nv = nrm(crs(SEN, sh.Nu));
 }
 
-/* UniformSampleOneLight (transport.h:115-156) with the full-mode shader selection
- * (design at scatterevent.h:155-212) */
-template<int FULL, int COUNT>
-__device__ f3 uniform_sample_one_light(const DevParams& p, const Tables& T, const Sample& smp, f3 SEP, f3 SEN, f3 Wo, Rng& rng, Cnt& cnt,
-                                       int obj = -1, float U = 0.0f, float V = 0.0f)
-{
-    f3 Ld = mk(0.0f, 0.0f, 0.0f);
-    const float I = intensity(p, SEP);
-    if (COUNT) cnt.shading += 1 + gradient_samples(p);
-    Ld = add(Ld, ctf_eval(p.emission, I));
-    const int count = p.light_count;
-    if (count <= 0) return Ld;
-    const int pos = (int)floorf(smp.lightnum * (float)count);
-    const int LightID = p.light_ids[pos];
-    const DevLight* L = light_by_id(p, LightID);
-    if (LightID < 0 || !L) return Ld;
-    Shader sh;
-    event_shader<FULL, COUNT>(p, I, obj, U, V, SEP, SEN, Wo, rng, cnt, sh);
-    Ld = add(Ld, estimate_direct<FULL, COUNT>(p, T, *L, pos, smp, SEP, SEN, Wo, sh, rng, cnt));
-    return scl((float)count, Ld);
-}
-
-/* Shading of one volume event with the shadow-ray marches deferred (ray-march sampler only,
- * whose shadow march consumes exactly two draws whenever it starts). Same operations and
- * order as uniform_sample_one_light / estimate_direct; the contributions that wait for a
- * visibility result are kept with their state. */
+/* Shading of one event, UniformSampleOneLight and EstimateDirectLight (transport.h:58-156) with
+ * the full-mode shader selection (design at scatterevent.h:155-212) and with the shadow-ray
+ * marches deferred (a shadow march takes exactly two draws of the path's stream whenever it
+ * starts). The contributions that wait for a visibility result are kept with their state. */
 struct EventRec {
     uint32_t pixel, state;        /* state: 2 bits per contribution: 0 none, 1 add, 2 add if visible */
     float count;                  /* light count scaling, or 0 when the result is not scaled */

@@ -35,8 +35,7 @@ using erd::DevParams;
 extern "C" hipError_t erd_launch_trace(const DevParams* p, float4* frame, uint32_t* s1, uint32_t* s2, void* queue,
                                        unsigned int* counts, void* events, void* jobs, unsigned char* vis,
                                        unsigned long long* counters, int W, int H, int full, int count, int lut_lds,
-                                       int split, size_t lds_bytes, size_t lds_bits, int shade_blocks,
-                                       int primary_blocks, int shadow_blocks, int tile_shift, hipStream_t st,
+                                       size_t lds_bytes, int shade_blocks, int primary_blocks, int shadow_blocks, int tile_shift, hipStream_t st,
                                        hipStream_t st2, hipEvent_t shaded, hipEvent_t after_primary,
                                        const uint32_t* order_in, uint32_t* cost, uint32_t* order_out, int heavy_cap,
                                        int lanes_per_ray, int shadow_lanes_per_ray, int heavy_lanes_per_ray);
@@ -69,7 +68,7 @@ extern "C" hipError_t erd_batch_params_upload(const erd::DevParams* host, int n)
 extern "C" size_t erd_adj_partials_per_block(void);
 extern "C" hipError_t erd_launch_primary_shade(const DevParams* p, float4* frame, uint32_t* s1, uint32_t* s2, void* queue,
                                                unsigned int* counts, void* events, void* jobs, int W, int H, int lut_lds,
-                                               size_t lds_bytes, size_t lds_bits, int shade_blocks, int primary_blocks,
+                                               size_t lds_bytes, int shade_blocks, int primary_blocks,
                                                int tile_shift, hipStream_t st);
 extern "C" hipError_t erd_launch_adj_wavefront(const DevParams* p, unsigned int* counts, const void* jobs, const void* events,
                                                const void* queue, const float4* adj, float* tvis, float4* frame, uint2* list,
@@ -1288,10 +1287,8 @@ int enqueue_pass(Tracer& t, hipEvent_t* e)
     /* the set was last used two passes ago: its post must have consumed the frame and queues */
     if (S.pending) HIP_TRY(hipStreamWaitEvent(t.stream, S.posted, 0));
     if (e) HIP_TRY(hipEventRecord(e[0], t.stream));
-    const int split = 1;   /* every sampler defers its shadow marches (Woodcock's run on their own stream) */
     /* Woodcock tracking is per lane: its marches take one lane per ray, primary and shadow */
     const bool woodcock = full && t.desc.settings.sampler == ER_SAMPLER_WOODCOCK;
-    const size_t lds_bits = (size_t)t.host_params.mc_words * 4;
     const int ntiles = ((t.W + (1 << t.tile_shift) - 1) >> t.tile_shift) * ((t.H + (64 >> t.tile_shift) - 1) / (64 >> t.tile_shift));
     if (t.tile_cost.n < (size_t)ntiles) {
         /* every pass writes the cost of each of its tiles before the order kernel reads them */
@@ -1308,7 +1305,7 @@ int enqueue_pass(Tracer& t, hipEvent_t* e)
     const bool reorder = !order_valid || (t.desc.no_iterations & ER_REORDER_MASK) == 0;
     HIP_TRY(erd_launch_trace(t.params.ptr, S.frame.ptr, t.seeds1.ptr, t.seeds2.ptr, S.queue.ptr, S.qcount.ptr,
                              S.events.ptr, S.jobs.ptr, S.vis.ptr, t.counters.ptr, t.W, t.H, full, t.counting, t.lut_lds,
-                             split, t.lds_bytes, lds_bits, shade_blocks, primary_blocks(t), shadow_blocks(t), t.tile_shift, t.stream,
+                             t.lds_bytes, shade_blocks, primary_blocks(t), shadow_blocks(t), t.tile_shift, t.stream,
                              t.stream2, S.shaded, e ? e[1] : nullptr, order_valid ? t.tile_order.ptr : nullptr,
                              t.tile_cost.ptr, reorder ? t.tile_order.ptr : nullptr, t.heavy_tiles,
                              woodcock ? 1 : 64 / t.rays_per_wave, woodcock ? 1 : 64 / t.shadow_rays_per_wave,
@@ -2344,7 +2341,6 @@ ER_API int er_adjoint_lut(int tracer_id, const uint32_t* seeds1, const uint32_t*
     HIP_TRY(erd_launch_zero_words((uint32_t*)W.out.ptr, per_block * sizeof(double) / 4, s));
     for (AdjWork::Set& A : W.set) HIP_TRY(erd_launch_adj_reset(A.counts.ptr, A.lcount.ptr, s));
     const int shade_blocks = std::max(1, std::min((int)((n + 255) / 256), 2048));
-    const size_t lds_bits = (size_t)t->host_params.mc_words * 4;
     float cur_w = -1.0f;
     /* the running estimate after N passes is the mean of the filtered frames of passes 2..N
      * (the first pass is discarded, Q1), or the first frame when N == 1 */
@@ -2358,7 +2354,7 @@ ER_API int er_adjoint_lut(int tracer_id, const uint32_t* seeds1, const uint32_t*
         }
         /* the forward pass's primary and shading kernels: decisions, queues, final seeds */
         HIP_TRY(erd_launch_primary_shade(t->params.ptr, A.frame.ptr, W.d1.ptr, W.d2.ptr, A.queue.ptr, A.counts.ptr, A.events.ptr,
-                                         A.jobs.ptr, t->W, t->H, t->lut_lds, t->lds_bytes, lds_bits, shade_blocks,
+                                         A.jobs.ptr, t->W, t->H, t->lut_lds, t->lds_bytes, shade_blocks,
                                          primary_blocks(*t), t->tile_shift, s));
         HIP_TRY(hipEventRecord(A.shaded, s));
         HIP_TRY(hipStreamWaitEvent(s2, A.shaded, 0));
@@ -2431,7 +2427,6 @@ ER_API int er_adjoint_lut_noalloc(int tracer_id, const uint32_t* seeds1, const u
     HIP_TRY(erd_launch_adj_reset(counts, lcount, s));
     HIP_TRY(erd_launch_zero_words((uint32_t*)out, per_block * sizeof(double) / 4, s));
     const int shade_blocks = std::max(1, std::min((int)((n + 255) / 256), 2048));
-    const size_t lds_bits = (size_t)t->host_params.mc_words * 4;
     float cur_w = -1.0f;
     for (int k = 1; k <= passes; ++k) {
         const float w = passes == 1 ? 1.0f : (k >= 2 ? 1.0f / (float)(passes - 1) : 0.0f);
@@ -2440,7 +2435,7 @@ ER_API int er_adjoint_lut_noalloc(int tracer_id, const uint32_t* seeds1, const u
             HIP_TRY(hipMemcpyAsync(s2s, d2, n * 4, hipMemcpyDeviceToDevice, s));
         }
         HIP_TRY(erd_launch_primary_shade(t->params.ptr, frame, d1, d2, queue, counts, events, jobs, t->W, t->H, t->lut_lds,
-                                         t->lds_bytes, lds_bits, shade_blocks, primary_blocks(*t), t->tile_shift, s));
+                                         t->lds_bytes, shade_blocks, primary_blocks(*t), t->tile_shift, s));
         if (w != 0.0f) {
             if (w != cur_w) {
                 HIP_TRY(erd_launch_adj_filter_t(dldr, adj, t->W, t->H, w, s));

@@ -279,14 +279,13 @@ __device__ __forceinline__ void primary_tile(const DevParams& p, const Tables& T
 }
 
 /* One wave shades queue entries q0 .. q0 + 63 (those below n): NormalizedGradient at the
- * event (raymarching.h:70) and UniformSampleOneLight (transport.h:115-156). SPLIT: the shadow
- * marches are appended to the shadow-job queue (*jcount) and the event waits in an EventRec;
- * otherwise (Woodcock, whose draw count per march is not known in advance) the marches run
- * inline. Every lane of the wave must call this (the append is wave-wide). */
-template<int FULL, int COUNT, int SPLIT>
-__device__ __forceinline__ void shade_chunk(const DevParams& p, const Tables& T, unsigned int q0, unsigned int n, int lane,
-                                            float4* __restrict__ frame, uint32_t* __restrict__ seeds1,
-                                            uint32_t* __restrict__ seeds2, const ScatterRec* __restrict__ queue,
+ * event (raymarching.h:70) and UniformSampleOneLight (transport.h:115-156). The shadow marches
+ * are appended to the shadow-job queue (*jcount) and the event waits in an EventRec. Every lane
+ * of the wave must call this (the append is wave-wide). */
+template<int FULL, int COUNT>
+__device__ __forceinline__ void shade_chunk(const DevParams& p, unsigned int q0, unsigned int n, int lane,
+                                            uint32_t* __restrict__ seeds1, uint32_t* __restrict__ seeds2,
+                                            const ScatterRec* __restrict__ queue,
                                             EventRec* __restrict__ events, ShadowJob* __restrict__ jobq,
                                             unsigned int* __restrict__ jcount, Cnt& cnt)
 {
@@ -321,36 +320,27 @@ __device__ __forceinline__ void shade_chunk(const DevParams& p, const Tables& T,
         } else {
             Nv = normalized_gradient(p, Pv);
         }
-        if (SPLIT) {
-            EventRec ev;
-            ev.pixel = rec.pixel;
-            ev.c1x = ev.c1y = ev.c1z = ev.c2x = ev.c2y = ev.c2z = 0.0f;
-            ev.pad = ev.pad2 = 0.0f;
-            shade_split<FULL, COUNT>(p, smp, Pv, Nv, Wo, rng, cnt, ev, job0, job1, has0, has1, rec.obj, rec.U, rec.V,
-                                     Iv, cd);
-            events[q] = ev;
-        } else {
-            f3 Lv = mk(0.0f, 0.0f, 0.0f);
-            Lv = add(Lv, uniform_sample_one_light<FULL, COUNT>(p, T, smp, Pv, Nv, Wo, rng, cnt, rec.obj, rec.U, rec.V));
-            frame[rec.pixel] = make_float4(Lv.x, Lv.y, Lv.z, 1.0f);
-        }
+        EventRec ev;
+        ev.pixel = rec.pixel;
+        ev.c1x = ev.c1y = ev.c1z = ev.c2x = ev.c2y = ev.c2z = 0.0f;
+        ev.pad = ev.pad2 = 0.0f;
+        shade_split<FULL, COUNT>(p, smp, Pv, Nv, Wo, rng, cnt, ev, job0, job1, has0, has1, rec.obj, rec.U, rec.V, Iv, cd);
+        events[q] = ev;
         seeds1[rec.pixel] = rng.s0;
         seeds2[rec.pixel] = rng.s1;
     }
-    if (SPLIT) {
-        /* wave-aggregated append of 0..2 shadow jobs per lane */
-        const unsigned long long m1 = __ballot(has0), m2 = __ballot(has1);
-        const unsigned int total = (unsigned int)(__popcll(m1) + __popcll(m2));
-        if (total) {
-            const int leader = __ffsll((long long)(m1 | m2)) - 1;
-            unsigned int base = 0;
-            if (lane == leader) base = atomicAdd(jcount, total);
-            base = __shfl(base, leader);
-            const unsigned long long below = (1ull << lane) - 1ull;
-            const unsigned int slot = base + (unsigned int)(__popcll(m1 & below) + __popcll(m2 & below));
-            if (has0) { job0.event = q; job0.pad = 0; jobq[slot] = job0; }
-            if (has1) { job1.event = q; job1.pad = 0; jobq[slot + (has0 ? 1u : 0u)] = job1; }
-        }
+    /* wave-aggregated append of 0..2 shadow jobs per lane */
+    const unsigned long long m1 = __ballot(has0), m2 = __ballot(has1);
+    const unsigned int total = (unsigned int)(__popcll(m1) + __popcll(m2));
+    if (total) {
+        const int leader = __ffsll((long long)(m1 | m2)) - 1;
+        unsigned int base = 0;
+        if (lane == leader) base = atomicAdd(jcount, total);
+        base = __shfl(base, leader);
+        const unsigned long long below = (1ull << lane) - 1ull;
+        const unsigned int slot = base + (unsigned int)(__popcll(m1 & below) + __popcll(m2 & below));
+        if (has0) { job0.event = q; job0.pad = 0; jobq[slot] = job0; }
+        if (has1) { job1.event = q; job1.pad = 0; jobq[slot + (has0 ? 1u : 0u)] = job1; }
     }
 }
 
@@ -522,24 +512,23 @@ __global__ __launch_bounds__(1024) void k_tile_order(uint32_t* __restrict__ cost
 #define ER_SHADE_WAVES_PER_EU 1
 #endif
 
-/* Shading kernel over the scatter queue (counts[0] entries), wave-aligned grid stride. */
-template<int FULL, int COUNT, int LUT_LDS, int SPLIT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ER_SHADE_WAVES_PER_EU))) void k_shade(const DevParams* __restrict__ pp, float4* __restrict__ frame,
+/* Shading kernel over the scatter queue (counts[0] entries), wave-aligned grid stride. It reads
+ * the volume only at its events, without the march tables. */
+template<int FULL, int COUNT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ER_SHADE_WAVES_PER_EU))) void k_shade(const DevParams* __restrict__ pp,
                                               uint32_t* __restrict__ seeds1, uint32_t* __restrict__ seeds2,
                                               const ScatterRec* __restrict__ queue, unsigned int* __restrict__ counts,
                                               EventRec* __restrict__ events, ShadowJob* __restrict__ jobq,
                                               unsigned long long* __restrict__ counters)
 {
-    extern __shared__ uint32_t lds[];
     const DevParams& p = *pp;
-    const Tables T = stage_tables<SPLIT ? 0 : LUT_LDS>(p, lds);
     const unsigned int n = counts[0];
     const int lane = threadIdx.x & 63;
     Cnt cnt = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     const unsigned int stride = gridDim.x * blockDim.x;
     const unsigned int base_q = blockIdx.x * blockDim.x + (threadIdx.x & ~63u);
     for (unsigned int q0 = base_q; q0 < n; q0 += stride)
-        shade_chunk<FULL, COUNT, SPLIT>(p, T, q0, n, lane, frame, seeds1, seeds2, queue, events, jobq, &counts[1], cnt);
+        shade_chunk<FULL, COUNT>(p, q0, n, lane, seeds1, seeds2, queue, events, jobq, &counts[1], cnt);
     flush_counters<COUNT>(cnt, true, 0, counters);
 }
 
@@ -1141,8 +1130,7 @@ __global__ __launch_bounds__(256) void k_shade_b(const BatchJob* __restrict__ J,
         n = __builtin_amdgcn_readfirstlane(n);
         const BatchJob& B = J[job];
         const DevParams& p = c_batch_params[job];
-        const Tables T = global_tables(p);
-        shade_chunk<FULL, 0, 1>(p, T, q0, n, lane, B.frame, B.seeds1, B.seeds2, B.queue, B.events, B.jobs, &B.counts[1], cnt);
+        shade_chunk<FULL, 0>(p, q0, n, lane, B.seeds1, B.seeds2, B.queue, B.events, B.jobs, &B.counts[1], cnt);
     }
 }
 
@@ -1225,7 +1213,7 @@ template<int FULL, int COUNT, int LUT_LDS>
 static void launch_all(const erd::DevParams* p, float4* frame, uint32_t* s1, uint32_t* s2, erd::ScatterRec* queue,
                        unsigned int* counts, erd::EventRec* events, erd::ShadowJob* jobs, unsigned char* vis,
                        unsigned long long* counters, int tiles_x, int ntiles, int nblocks, int shade_blocks,
-                       int shadow_blocks, int split, size_t lds, size_t lds_bits, hipStream_t st, hipStream_t st2,
+                       int shadow_blocks, size_t lds, hipStream_t st, hipStream_t st2,
                        hipEvent_t shaded, hipEvent_t after_primary, const uint32_t* order_in, uint32_t* cost,
                        uint32_t* order_out, int heavy_cap, int lpr, int shadow_lpr, int heavy_lanes)
 {
@@ -1237,25 +1225,18 @@ static void launch_all(const erd::DevParams* p, float4* frame, uint32_t* s1, uin
     else ER_PRIMARY(1);
 #undef ER_PRIMARY
     if (after_primary) (void)hipEventRecord(after_primary, st);
-    if (split) {
-        hipLaunchKernelGGL((erd::k_shade<FULL, COUNT, LUT_LDS, 1>), dim3(shade_blocks), dim3(256), lds_bits, st, p, frame, s1,
-                           s2, (const erd::ScatterRec*)queue, counts, events, jobs, counters);
-        (void)hipEventRecord(shaded, st);
-        (void)hipStreamWaitEvent(st2, shaded, 0);
+    hipLaunchKernelGGL((erd::k_shade<FULL, COUNT>), dim3(shade_blocks), dim3(256), 0, st, p, s1, s2,
+                       (const erd::ScatterRec*)queue, counts, events, jobs, counters);
+    (void)hipEventRecord(shaded, st);
+    (void)hipStreamWaitEvent(st2, shaded, 0);
 #define ER_SHADOW(G) hipLaunchKernelGGL((erd::k_shadow<FULL, COUNT, LUT_LDS, G>), dim3(shadow_blocks), dim3(256), lds, st2, \
-                                        p, counts, (const erd::ShadowJob*)jobs, vis, counters)
-        if (shadow_lpr == 4) ER_SHADOW(4);
-        else if (shadow_lpr == 16) ER_SHADOW(16);
-        else ER_SHADOW(1);
+                                    p, counts, (const erd::ShadowJob*)jobs, vis, counters)
+    if (shadow_lpr == 4) ER_SHADOW(4);
+    else if (shadow_lpr == 16) ER_SHADOW(16);
+    else ER_SHADOW(1);
 #undef ER_SHADOW
-        hipLaunchKernelGGL(erd::k_finish, dim3(shade_blocks), dim3(256), 0, st2, (const unsigned int*)counts,
-                           (const erd::EventRec*)events, (const unsigned char*)vis, frame);
-    } else {
-        hipLaunchKernelGGL((erd::k_shade<FULL, COUNT, LUT_LDS, 0>), dim3(shade_blocks), dim3(256), lds, st, p, frame, s1, s2,
-                           (const erd::ScatterRec*)queue, counts, events, jobs, counters);
-        (void)hipEventRecord(shaded, st);
-        (void)hipStreamWaitEvent(st2, shaded, 0);
-    }
+    hipLaunchKernelGGL(erd::k_finish, dim3(shade_blocks), dim3(256), 0, st2, (const unsigned int*)counts,
+                       (const erd::EventRec*)events, (const unsigned char*)vis, frame);
     /* the next pass's tile order from this pass's tile costs (after the primary kernel has
      * read the current order; stream order keeps the next primary kernel behind it) */
     if (cost && order_out)
@@ -1267,8 +1248,7 @@ static void launch_all(const erd::DevParams* p, float4* frame, uint32_t* s1, uin
 extern "C" hipError_t erd_launch_trace(const erd::DevParams* p, float4* frame, uint32_t* s1, uint32_t* s2, void* queue,
                                        unsigned int* counts, void* events, void* jobs, unsigned char* vis,
                                        unsigned long long* counters, int W, int H, int full, int count, int lut_lds,
-                                       int split, size_t lds_bytes, size_t lds_bits, int shade_blocks,
-                                       int primary_blocks, int shadow_blocks, int tile_shift, hipStream_t st,
+                                       size_t lds_bytes, int shade_blocks, int primary_blocks, int shadow_blocks, int tile_shift, hipStream_t st,
                                        hipStream_t st2, hipEvent_t shaded, hipEvent_t after_primary,
                                        const uint32_t* order_in, uint32_t* cost, uint32_t* order_out, int heavy_cap,
                                        int lanes_per_ray, int shadow_lanes_per_ray, int heavy_lanes_per_ray)
@@ -1285,7 +1265,7 @@ extern "C" hipError_t erd_launch_trace(const erd::DevParams* p, float4* frame, u
     erd::EventRec* ev = (erd::EventRec*)events;
     erd::ShadowJob* jb = (erd::ShadowJob*)jobs;
 #define ER_ALL(F, C, L) launch_all<F, C, L>(p, frame, s1, s2, q, counts, ev, jb, vis, counters, tiles_x, ntiles, nblocks, \
-                                            shade_blocks, std::max(1, shadow_blocks), split, lds_bytes, lds_bits, st, st2, \
+                                            shade_blocks, std::max(1, shadow_blocks), lds_bytes, st, st2, \
                                             shaded, after_primary, order_in, cost, order_out, heavy_cap, lpr, \
                                             (shadow_lanes_per_ray == 4 || shadow_lanes_per_ray == 16) ? shadow_lanes_per_ray : 1, \
                                             heavy_lanes_per_ray)
@@ -1366,7 +1346,7 @@ extern "C" hipError_t erd_launch_round_end(const erd::BatchJob* J, int njobs, hi
  * follows them with its own kernels) */
 extern "C" hipError_t erd_launch_primary_shade(const erd::DevParams* p, float4* frame, uint32_t* s1, uint32_t* s2,
                                                void* queue, unsigned int* counts, void* events, void* jobs, int W, int H,
-                                               int lut_lds, size_t lds_bytes, size_t lds_bits, int shade_blocks,
+                                               int lut_lds, size_t lds_bytes, int shade_blocks,
                                                int primary_blocks, int tile_shift, hipStream_t st)
 {
     const int tw = 1 << tile_shift, th = 64 >> tile_shift;
@@ -1381,8 +1361,7 @@ extern "C" hipError_t erd_launch_primary_shade(const erd::DevParams* p, float4* 
     else
         hipLaunchKernelGGL((erd::k_primary<1, 0, 0, 1>), dim3(nblocks), dim3(ER_PRIMARY_WG), lds_bytes, st, p, frame, s1, s2, q, counts,
                            (unsigned long long*)nullptr, tiles_x, ntiles, (const uint32_t*)nullptr, (uint32_t*)nullptr, 64);
-    hipLaunchKernelGGL((erd::k_shade<1, 0, 1, 1>), dim3(shade_blocks), dim3(256), lds_bits, st, p, frame, s1, s2,
-                       (const erd::ScatterRec*)q, counts, (erd::EventRec*)events, (erd::ShadowJob*)jobs,
+    hipLaunchKernelGGL((erd::k_shade<1, 0>), dim3(shade_blocks), dim3(256), 0, st, p, s1, s2, (const erd::ScatterRec*)q, counts, (erd::EventRec*)events, (erd::ShadowJob*)jobs,
                        (unsigned long long*)nullptr);
     return hipGetLastError();
 }

@@ -307,7 +307,7 @@ __device__ __forceinline__ CellFetch cell_fetch(const DevParams& p, const Lattic
     const float fx = floorf(l.Lx), fy = floorf(l.Ly), fz = floorf(l.Lz);
     const int vx = (int)fx, vy = (int)fy, vz = (int)fz;
     CellFetch f;
-    f.dx = l.Lx - (float)vx; f.dy = l.Ly - (float)vy; f.dz = l.Lz - (float)vz;
+    f.dx = l.Lx - fx; f.dy = l.Ly - fy; f.dz = l.Lz - fz;
     const int cx = min(max(vx, -1), p.res[0] - 1) + 1;
     const int cy = min(max(vy, -1), p.res[1] - 1) + 1;
     const int cz = min(max(vz, -1), p.res[2] - 1) + 1;
@@ -322,8 +322,10 @@ __device__ __forceinline__ CellFetch cell_fetch(const DevParams& p, const Lattic
 }
 
 /* Buffer3D<ushort>::operator()(Vec3f) (buffer3d.h:222-242) from one cell record: 7 lerps,
- * each truncated to uint16 (geometry.h:87-90). */
-__device__ __forceinline__ float cell_value(const CellFetch& f)
+ * each truncated to uint16 (geometry.h:87-90); cell_lerp leaves the last truncation to the
+ * caller. With all corners at most M (an integer below 65536) and weights in [0, 1] that add up
+ * to 1 within a rounding, every lerp is below M + 1, so the truncated values are at most M. */
+__device__ __forceinline__ float cell_lerp(const CellFetch& f)
 {
     const uint4 c = f.c;
     const float dx = f.dx, dy = f.dy, dz = f.dz;
@@ -338,8 +340,11 @@ __device__ __forceinline__ float cell_value(const CellFetch& f)
     const float d11 = trunc16(ox * v011 + dx * v111);
     const float d0 = trunc16(oy * d00 + dy * d10);
     const float d1 = trunc16(oy * d01 + dy * d11);
-    return trunc16(oz * d0 + dz * d1);
+    return oz * d0 + dz * d1;
 }
+__device__ __forceinline__ float cell_value(const CellFetch& f) { return trunc16(cell_lerp(f)); }
+/* the truncated value as an integer, at most the largest corner */
+__device__ __forceinline__ uint32_t cell_index(const CellFetch& f) { return (uint32_t)cell_lerp(f); }
 
 __device__ __forceinline__ float trilinear_cell(const DevParams& p, const Lattice& l) { return cell_value(cell_fetch(p, l)); }
 

@@ -34,8 +34,9 @@ using erd::DevParams;
 
 extern "C" hipError_t erd_launch_trace(const DevParams* p, float4* frame, uint32_t* s1, uint32_t* s2, void* queue,
                                        unsigned int* counts, void* events, void* jobs, unsigned char* vis,
-                                       unsigned long long* counters, int W, int H, int full, int count, int lut_lds,
-                                       size_t lds_bytes, int shade_blocks, int primary_blocks, int shadow_blocks, int tile_shift, hipStream_t st,
+                                       unsigned long long* counters, int W, int H, int full, int plain, int count,
+                                       int lut_lds, size_t lds_bytes, int shade_blocks, int primary_blocks,
+                                       int shadow_blocks, int tile_shift, hipStream_t st,
                                        hipStream_t st2, hipEvent_t shaded, hipEvent_t after_primary,
                                        const uint32_t* order_in, uint32_t* cost, uint32_t* order_out, int heavy_cap,
                                        int lanes_per_ray, int shadow_lanes_per_ray, int heavy_lanes_per_ray);
@@ -58,7 +59,7 @@ extern "C" hipError_t erd_launch_macro_sigma(const uint32_t* mm, const float* lu
                                              hipStream_t st);
 extern "C" hipError_t erd_launch_gm_max(const DevParams* p, const uint16_t* vox, float* bounds, unsigned int* out, int rx,
                                         int ry, int rz, int prune, hipStream_t st);
-extern "C" hipError_t erd_launch_batch_trace(const erd::BatchJob* J, int na, int full, int primary_blocks,
+extern "C" hipError_t erd_launch_batch_trace(const erd::BatchJob* J, int na, int full, int plain, int primary_blocks,
                                              int lds_words, int shade_blocks, hipStream_t stream,
                                              hipStream_t stream2, hipEvent_t shaded, int lpr, int shadow_lpr);
 extern "C" hipError_t erd_launch_batch_post(const erd::BatchJob* J, int na, unsigned int round, int active_tiles,
@@ -67,7 +68,7 @@ extern "C" hipError_t erd_launch_round_end(const erd::BatchJob* J, int njobs, hi
 extern "C" hipError_t erd_batch_params_upload(const erd::DevParams* host, int n);
 extern "C" size_t erd_adj_partials_per_block(void);
 extern "C" hipError_t erd_launch_primary_shade(const DevParams* p, float4* frame, uint32_t* s1, uint32_t* s2, void* queue,
-                                               unsigned int* counts, void* events, void* jobs, int W, int H, int lut_lds,
+                                               unsigned int* counts, void* events, void* jobs, int W, int H, int plain, int lut_lds,
                                                size_t lds_bytes, int shade_blocks, int primary_blocks,
                                                int tile_shift, hipStream_t st);
 extern "C" hipError_t erd_launch_adj_wavefront(const DevParams* p, unsigned int* counts, const void* jobs, const void* events,
@@ -77,7 +78,7 @@ extern "C" hipError_t erd_launch_adj_wavefront(const DevParams* p, unsigned int*
 extern "C" hipError_t erd_launch_adj_reset(unsigned int* counts, unsigned int* lcount, hipStream_t st);
 extern "C" size_t erd_autofocus_work_size(void);
 extern "C" size_t erd_autofocus_out_offset(void);
-extern "C" hipError_t erd_launch_autofocus(const DevParams* p, int u, int v, uint32_t s0, uint32_t s1, void* work, int full,
+extern "C" hipError_t erd_launch_autofocus(const DevParams* p, int u, int v, uint32_t s0, uint32_t s1, void* work, int plain,
                                            int serial, int lut_lds, size_t lds_bytes, hipStream_t st);
 extern "C" hipError_t erd_launch_adjoint(const DevParams* p, int mode, const float* lut_eval, const float* sigma_eval,
                                          const float4* adj, float4* value, float* partials, uint32_t* s1, uint32_t* s2,
@@ -431,6 +432,8 @@ struct Tracer {
     DevBuf<uint8_t> group_tmp;
     size_t lds_bytes = 0;
     int lut_lds = 0;
+    int lut_nonneg = 0;              /* no entry of the opacity table is negative or NaN */
+    int plain = 0;                   /* the marches may take their plain form (ER_MARCH_PLAIN) */
     DevBuf<DevParams> params;
     DevParams* params_pinned = nullptr;   /* the copy the upload reads */
     /* what the tables above (opacity, occupancy, radii, majorants) were built from, by value:
@@ -927,7 +930,7 @@ int build_params(Tracer& t)
     P.shading_type = s.shading_type;
     P.opacity_modulated = s.opacity_modulated;
     P.gradient_mode = s.gradient_computation;
-    P.sampler = s.sampler;
+    P.sampler = s.estimator == ER_ESTIMATOR_FULL ? s.sampler : ER_SAMPLER_RAYMARCH;   /* compat has no other */
 
     /* Volume::operator=(ErVolume) (Source/volume.h:100-129) */
     const er_volume_desc& vd = vol->desc;
@@ -1146,6 +1149,8 @@ int build_params(Tracer& t)
                                              : erd::tf_lut_eval(t.tf_lut.data(), t.tf_scale, (float)i, 0);
             lut[i] = s.density_scale * o;
         }
+        t.lut_nonneg = 1;
+        for (int i = 0; i < lut_n; ++i) t.lut_nonneg = t.lut_nonneg && lut[i] >= 0.0f;
         uint32_t following = 0xffffffffu;
         for (int i = lut_n - 1; i >= 0; --i) next[i] = following = lut[i] > 0.0f ? (uint32_t)i : following;
         HIP_TRY(hipMemcpyAsync(t.lut.ptr, lut.data(), lut_n * sizeof(float), hipMemcpyHostToDevice, t.stream));
@@ -1153,6 +1158,7 @@ int build_params(Tracer& t)
     }
     P.sigma_lut = t.lut.ptr;
     P.lut_max = lut_n - 1;
+    t.plain = t.lut_nonneg && P.clip_count == 0 && !woodcock;
     const int nmc = grid->mc[0] * grid->mc[1] * grid->mc[2];
     P.mc_shift = mc_shift;
     /* Woodcock majorants on their own fixed grid of 2^ER_WC_SHIFT-cell macrocells */
@@ -1304,7 +1310,7 @@ int enqueue_pass(Tracer& t, hipEvent_t* e)
 #endif
     const bool reorder = !order_valid || (t.desc.no_iterations & ER_REORDER_MASK) == 0;
     HIP_TRY(erd_launch_trace(t.params.ptr, S.frame.ptr, t.seeds1.ptr, t.seeds2.ptr, S.queue.ptr, S.qcount.ptr,
-                             S.events.ptr, S.jobs.ptr, S.vis.ptr, t.counters.ptr, t.W, t.H, full, t.counting, t.lut_lds,
+                             S.events.ptr, S.jobs.ptr, S.vis.ptr, t.counters.ptr, t.W, t.H, full, t.plain, t.counting, t.lut_lds,
                              t.lds_bytes, shade_blocks, primary_blocks(t), shadow_blocks(t), t.tile_shift, t.stream,
                              t.stream2, S.shaded, e ? e[1] : nullptr, order_valid ? t.tile_order.ptr : nullptr,
                              t.tile_cost.ptr, reorder ? t.tile_order.ptr : nullptr, t.heavy_tiles,
@@ -2126,6 +2132,8 @@ static int render_batch_chunk(std::vector<std::pair<int, Tracer*>>& jobs, int fu
     if (!all_lds) lds_words = 0;
     /* lanes per primary and shadow march, for the whole batch: the jobs' common rays per wave
      * (one lane per ray when they differ, or when a job uses Woodcock tracking) */
+    int plain = 1;   /* the marches' plain form, when every job's scene allows it */
+    for (auto& j : jobs) plain = plain && j.second->plain;
     int lpr = 64 / jobs[0].second->rays_per_wave, slpr = 64 / jobs[0].second->shadow_rays_per_wave;
     for (auto& j : jobs) {
         const Tracer& t = *j.second;
@@ -2137,7 +2145,7 @@ static int render_batch_chunk(std::vector<std::pair<int, Tracer*>>& jobs, int fu
     /* the graph's key: the job tables without their first pass numbers, and the launch shape */
     std::string key;
     {
-        const int hdr[7] = {nj, full, batch_blocks, lds_words, shade_blocks, lpr, slpr};
+        const int hdr[8] = {nj, full, plain, batch_blocks, lds_words, shade_blocks, lpr, slpr};
         key.append((const char*)hdr, sizeof(hdr));
         for (int b = 0; b < 2; ++b)
             for (int k = 0; k < nj; ++k) {
@@ -2189,7 +2197,7 @@ static int render_batch_chunk(std::vector<std::pair<int, Tracer*>>& jobs, int fu
             hipEvent_t shaded = nullptr;
             if (ec == hipSuccess) ec = new_event(shaded);
             if (ec == hipSuccess)
-                ec = erd_launch_batch_trace(dJ[b].ptr, na, full, batch_blocks, lds_words, shade_blocks, bs, bs2, shaded, lpr,
+                ec = erd_launch_batch_trace(dJ[b].ptr, na, full, plain, batch_blocks, lds_words, shade_blocks, bs, bs2, shaded, lpr,
                                             slpr);
             if (ec == hipSuccess) ec = erd_launch_batch_post(dJ[b].ptr, na, (unsigned int)r, active_tiles, bs2);
             if (ec == hipSuccess) ec = erd_launch_round_end(dJ[b].ptr, nj, bs2);
@@ -2354,7 +2362,7 @@ ER_API int er_adjoint_lut(int tracer_id, const uint32_t* seeds1, const uint32_t*
         }
         /* the forward pass's primary and shading kernels: decisions, queues, final seeds */
         HIP_TRY(erd_launch_primary_shade(t->params.ptr, A.frame.ptr, W.d1.ptr, W.d2.ptr, A.queue.ptr, A.counts.ptr, A.events.ptr,
-                                         A.jobs.ptr, t->W, t->H, t->lut_lds, t->lds_bytes, shade_blocks,
+                                         A.jobs.ptr, t->W, t->H, t->plain, t->lut_lds, t->lds_bytes, shade_blocks,
                                          primary_blocks(*t), t->tile_shift, s));
         HIP_TRY(hipEventRecord(A.shaded, s));
         HIP_TRY(hipStreamWaitEvent(s2, A.shaded, 0));
@@ -2434,7 +2442,7 @@ ER_API int er_adjoint_lut_noalloc(int tracer_id, const uint32_t* seeds1, const u
             HIP_TRY(hipMemcpyAsync(s1s, d1, n * 4, hipMemcpyDeviceToDevice, s));
             HIP_TRY(hipMemcpyAsync(s2s, d2, n * 4, hipMemcpyDeviceToDevice, s));
         }
-        HIP_TRY(erd_launch_primary_shade(t->params.ptr, frame, d1, d2, queue, counts, events, jobs, t->W, t->H, t->lut_lds,
+        HIP_TRY(erd_launch_primary_shade(t->params.ptr, frame, d1, d2, queue, counts, events, jobs, t->W, t->H, t->plain, t->lut_lds,
                                          t->lds_bytes, shade_blocks, primary_blocks(*t), t->tile_shift, s));
         if (w != 0.0f) {
             if (w != cur_w) {
@@ -2573,7 +2581,7 @@ ER_API int er_get_autofocus_distance(int tracer_id, int film_u, int film_v, floa
     }
     const int full = t->desc.settings.estimator == ER_ESTIMATOR_FULL;
     const int serial = full && t->desc.settings.sampler == ER_SAMPLER_WOODCOCK;
-    HIP_TRY(erd_launch_autofocus(t->params.ptr, film_u, film_v, s0, s1, t->focus.ptr, full, serial, t->lut_lds, t->lds_bytes,
+    HIP_TRY(erd_launch_autofocus(t->params.ptr, film_u, film_v, s0, s1, t->focus.ptr, t->plain, serial, t->lut_lds, t->lds_bytes,
                                  t->stream));
     HIP_TRY(hipMemcpyAsync(distance, t->focus.ptr + erd_autofocus_out_offset(), sizeof(float), hipMemcpyDeviceToHost, t->stream));
     HIP_TRY(hipStreamSynchronize(t->stream));

@@ -16,8 +16,9 @@
  * shadow march takes the RNG state it starts from along and the shading kernel advances past
  * its two draws, so every path consumes exactly the reference draw sequence.
  *
- * Template parameters: FULL selects the full estimator (shading-mode selection, both halves
- * of MIS, clipping objects, Woodcock sampler); COUNT adds the sample counters.
+ * Template parameters: in the shading kernels FULL selects the full estimator (shading-mode
+ * selection, both halves of MIS); in the march kernels it is the march functions' mode
+ * (ER_MARCH_ANY, ER_MARCH_PLAIN). COUNT adds the sample counters.
  */
 #include "er_path.h"
 
@@ -27,9 +28,10 @@
 
 namespace erd {
 
-/* Stage the macrocell bits (always) and the opacity LUT (when LUT_LDS) in LDS. */
-template<int LUT_LDS>
-__device__ __forceinline__ Tables stage_tables(const DevParams& p, uint32_t* lds)
+/* Stage the macrocell bits (always) and the opacity LUT (when LUT_LDS; times step for the plain
+ * marches, see Tables) in LDS. */
+template<int FULL, int LUT_LDS>
+__device__ __forceinline__ Tables stage_tables(const DevParams& p, uint32_t* lds, float step)
 {
     const int nw = p.mc_words;
     for (int k = threadIdx.x; k < nw; k += blockDim.x) lds[k] = gmem(p.mc_bits)[k];
@@ -38,7 +40,10 @@ __device__ __forceinline__ Tables stage_tables(const DevParams& p, uint32_t* lds
     T.bits_glb = nullptr;
     if (LUT_LDS) {
         float* lut = (float*)(lds + nw);
-        for (int k = threadIdx.x; k <= p.lut_max; k += blockDim.x) lut[k] = gmem(p.sigma_lut)[k];
+        for (int k = threadIdx.x; k <= p.lut_max; k += blockDim.x) {
+            const float s = gmem(p.sigma_lut)[k];
+            lut[k] = FULL == ER_MARCH_PLAIN ? s * step : s;
+        }
         T.lut_lds = lut;
         T.lut_glb = nullptr;
     } else {
@@ -120,7 +125,7 @@ __device__ __forceinline__ void primary_tile(const DevParams& p, const Tables& T
         rng.s1 = seeds2[i];
         r = camera_ray(p, px, py, rng, smp);
         D = r.D;
-        if (FULL && p.sampler == ER_SAMPLER_WOODCOCK) {
+        if (FULL == ER_MARCH_ANY && p.sampler == ER_SAMPLER_WOODCOCK) {
             vol = march<FULL, COUNT, ER_BATCH_PRIMARY>(p, T, r, true, rng, Tv, Pv, cnt);
         } else {
             /* march_v's set-up; its loop follows, wave by wave */
@@ -390,7 +395,7 @@ __global__ __launch_bounds__(ER_PRIMARY_WG) __attribute__((amdgpu_waves_per_eu(E
 {
     extern __shared__ uint32_t lds[];
     const DevParams& p = *pp;
-    const Tables T = stage_tables<LUT_LDS>(p, lds);
+    const Tables T = stage_tables<FULL, LUT_LDS>(p, lds, p.step_primary * p.minstep);
     const int lane = threadIdx.x & 63;
     Cnt cnt = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     int paths = 0;
@@ -400,7 +405,7 @@ __global__ __launch_bounds__(ER_PRIMARY_WG) __attribute__((amdgpu_waves_per_eu(E
      * order */
     const unsigned int HL = heavy_lanes == 4 || heavy_lanes == 16 ? (unsigned int)heavy_lanes : 64u;
     unsigned int hc = order ? min((unsigned int)__builtin_amdgcn_readfirstlane(order[ntiles]), (unsigned int)ntiles) : 0u;
-    if ((FULL && p.sampler == ER_SAMPLER_WOODCOCK) || LPR > 1) hc = 0u;
+    if ((FULL == ER_MARCH_ANY && p.sampler == ER_SAMPLER_WOODCOCK) || LPR > 1) hc = 0u;
     const unsigned int nclaims = LPR > 1 ? (unsigned int)ntiles * (unsigned int)LPR : hc * HL + ((unsigned int)ntiles - hc);
     for (;;) {
         unsigned int claim = 0;
@@ -643,7 +648,7 @@ __device__ __forceinline__ void shadow_marches(const DevParams& p, const Tables&
                                                unsigned char* __restrict__ vis, unsigned int* claim, unsigned int n,
                                                unsigned int j, unsigned int claim_base, bool drained, int lane, Cnt& cnt)
 {
-    if (FULL && p.sampler == ER_SAMPLER_WOODCOCK) {
+    if (FULL == ER_MARCH_ANY && p.sampler == ER_SAMPLER_WOODCOCK) {
         shadow_marches_wc<FULL, COUNT>(p, T, jobq, vis, claim, n, j, claim_base, drained, lane, cnt);
         return;
     }
@@ -786,7 +791,7 @@ __global__ __launch_bounds__(256) void k_shadow(const DevParams* __restrict__ pp
     const unsigned int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const unsigned int static_end = ((gridDim.x * blockDim.x) >> 6) * R;
     if ((blockIdx.x * blockDim.x >> 6) * R >= n) return;   /* no static chunk in the workgroup (workgroup-uniform) */
-    const Tables T = stage_tables<LUT_LDS>(p, lds);
+    const Tables T = stage_tables<FULL, LUT_LDS>(p, lds, p.step_shadow * p.minstep);
     const int lane = threadIdx.x & 63;
     Cnt cnt = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     if constexpr (LPR > 1)
@@ -900,7 +905,7 @@ __global__ __launch_bounds__(256) void k_autofocus(const DevParams* __restrict__
         uint32_t s = s1;
         for (int k = 0; k < 4 * ER_FOCUS_RAYS; ++k) { s = 18000u * (s & 65535u) + (s >> 16); st1[k] = s; }
     }
-    const Tables T = stage_tables<LUT_LDS>(p, lds);   /* ends with a barrier */
+    const Tables T = stage_tables<FULL, LUT_LDS>(p, lds, p.step_primary * p.minstep);   /* ends with a barrier */
     auto draw = [&](int k) { return (float)(((st0[k] << 16) + st1[k]) & 0x007fffffu) * 1.1920928955078125e-07f; };
     const int t = threadIdx.x;
     int at = 4 * t;
@@ -994,14 +999,17 @@ __constant__ DevParams c_batch_params[ER_BATCH_CONST_JOBS];
  * into the workgroup's LDS (the host launches this form only when every job's tables fit),
  * LDS = 0 reads both from global memory. Called by the whole workgroup after every wave has
  * finished with the previous job's tables. */
-template<int LDS>
-__device__ __forceinline__ Tables stage_job_tables(const DevParams& p, uint32_t* lds)
+template<int FULL, int LDS>
+__device__ __forceinline__ Tables stage_job_tables(const DevParams& p, uint32_t* lds, float step)
 {
     if (!LDS) return global_tables(p);
     const int nw = p.mc_words;
     for (int k = threadIdx.x; k < nw; k += blockDim.x) lds[k] = gmem(p.mc_bits)[k];
     float* lut = (float*)(lds + nw);
-    for (int k = threadIdx.x; k <= p.lut_max; k += blockDim.x) lut[k] = gmem(p.sigma_lut)[k];
+    for (int k = threadIdx.x; k <= p.lut_max; k += blockDim.x) {
+        const float s = gmem(p.sigma_lut)[k];
+        lut[k] = FULL == ER_MARCH_PLAIN ? s * step : s;
+    }
     __syncthreads();
     Tables T;
     T.bits = lds;
@@ -1050,7 +1058,7 @@ __global__ __launch_bounds__(256) void k_primary_b(const BatchJob* __restrict__ 
     for (;;) {
         const BatchJob& B = J[j];
         const DevParams& p = c_batch_params[j];
-        const Tables T = stage_job_tables<LDS>(p, lds);
+        const Tables T = stage_job_tables<FULL, LDS>(p, lds, p.step_primary * p.minstep);
         for (;;) {
             unsigned int claim = 0;
             if (lane == 0) claim = atomicAdd(&B.counts[2], 1u);
@@ -1159,7 +1167,7 @@ __global__ __launch_bounds__(256) void k_shadow_b(const BatchJob* __restrict__ J
     for (;;) {
         const BatchJob& B = J[j];
         const DevParams& p = c_batch_params[j];
-        const Tables T = stage_job_tables<LDS>(p, lds);
+        const Tables T = stage_job_tables<FULL, LDS>(p, lds, p.step_shadow * p.minstep);
         const unsigned int n = __builtin_amdgcn_readfirstlane(B.counts[1]);
         if constexpr (LPR > 1)
             shadow_marches_g<FULL, 0, LPR>(p, T, B.jobs, B.vis, &B.counts[3], n, n, 0u, false, lane, cnt);
@@ -1209,15 +1217,16 @@ extern "C" void erd_pass_record_sizes(size_t* scatter, size_t* event, size_t* jo
     *job = sizeof(erd::ShadowJob);
 }
 
-template<int FULL, int COUNT, int LUT_LDS>
-static void launch_all(const erd::DevParams* p, float4* frame, uint32_t* s1, uint32_t* s2, erd::ScatterRec* queue,
+/* M: the march functions' mode (ER_MARCH_ANY or ER_MARCH_PLAIN) */
+template<int M, int COUNT, int LUT_LDS>
+static void launch_all(int full, const erd::DevParams* p, float4* frame, uint32_t* s1, uint32_t* s2, erd::ScatterRec* queue,
                        unsigned int* counts, erd::EventRec* events, erd::ShadowJob* jobs, unsigned char* vis,
                        unsigned long long* counters, int tiles_x, int ntiles, int nblocks, int shade_blocks,
                        int shadow_blocks, size_t lds, hipStream_t st, hipStream_t st2,
                        hipEvent_t shaded, hipEvent_t after_primary, const uint32_t* order_in, uint32_t* cost,
                        uint32_t* order_out, int heavy_cap, int lpr, int shadow_lpr, int heavy_lanes)
 {
-#define ER_PRIMARY(G) hipLaunchKernelGGL((erd::k_primary<FULL, COUNT, LUT_LDS, G>), dim3(nblocks), dim3(ER_PRIMARY_WG), lds, st, p, \
+#define ER_PRIMARY(G) hipLaunchKernelGGL((erd::k_primary<M, COUNT, LUT_LDS, G>), dim3(nblocks), dim3(ER_PRIMARY_WG), lds, st, p, \
                                          frame, s1, s2, queue, counts, counters, tiles_x, ntiles, order_in, cost, heavy_lanes)
     if (lpr == 4) ER_PRIMARY(4);
     else if (lpr == 16) ER_PRIMARY(16);
@@ -1225,11 +1234,15 @@ static void launch_all(const erd::DevParams* p, float4* frame, uint32_t* s1, uin
     else ER_PRIMARY(1);
 #undef ER_PRIMARY
     if (after_primary) (void)hipEventRecord(after_primary, st);
-    hipLaunchKernelGGL((erd::k_shade<FULL, COUNT>), dim3(shade_blocks), dim3(256), 0, st, p, s1, s2,
-                       (const erd::ScatterRec*)queue, counts, events, jobs, counters);
+    if (full)
+        hipLaunchKernelGGL((erd::k_shade<1, COUNT>), dim3(shade_blocks), dim3(256), 0, st, p, s1, s2,
+                           (const erd::ScatterRec*)queue, counts, events, jobs, counters);
+    else
+        hipLaunchKernelGGL((erd::k_shade<0, COUNT>), dim3(shade_blocks), dim3(256), 0, st, p, s1, s2,
+                           (const erd::ScatterRec*)queue, counts, events, jobs, counters);
     (void)hipEventRecord(shaded, st);
     (void)hipStreamWaitEvent(st2, shaded, 0);
-#define ER_SHADOW(G) hipLaunchKernelGGL((erd::k_shadow<FULL, COUNT, LUT_LDS, G>), dim3(shadow_blocks), dim3(256), lds, st2, \
+#define ER_SHADOW(G) hipLaunchKernelGGL((erd::k_shadow<M, COUNT, LUT_LDS, G>), dim3(shadow_blocks), dim3(256), lds, st2, \
                                     p, counts, (const erd::ShadowJob*)jobs, vis, counters)
     if (shadow_lpr == 4) ER_SHADOW(4);
     else if (shadow_lpr == 16) ER_SHADOW(16);
@@ -1244,11 +1257,13 @@ static void launch_all(const erd::DevParams* p, float4* frame, uint32_t* s1, uin
 }
 
 /* One pass's trace kernels: primary and shading on st; shadow marches and combine on st2
- * after the shading (event `shaded`). The caller runs post-processing on st2. */
+ * after the shading (event `shaded`). The caller runs post-processing on st2. plain: the marches
+ * may take their ER_MARCH_PLAIN form (the counting kernels never do). */
 extern "C" hipError_t erd_launch_trace(const erd::DevParams* p, float4* frame, uint32_t* s1, uint32_t* s2, void* queue,
                                        unsigned int* counts, void* events, void* jobs, unsigned char* vis,
-                                       unsigned long long* counters, int W, int H, int full, int count, int lut_lds,
-                                       size_t lds_bytes, int shade_blocks, int primary_blocks, int shadow_blocks, int tile_shift, hipStream_t st,
+                                       unsigned long long* counters, int W, int H, int full, int plain, int count,
+                                       int lut_lds, size_t lds_bytes, int shade_blocks, int primary_blocks,
+                                       int shadow_blocks, int tile_shift, hipStream_t st,
                                        hipStream_t st2, hipEvent_t shaded, hipEvent_t after_primary,
                                        const uint32_t* order_in, uint32_t* cost, uint32_t* order_out, int heavy_cap,
                                        int lanes_per_ray, int shadow_lanes_per_ray, int heavy_lanes_per_ray)
@@ -1264,18 +1279,14 @@ extern "C" hipError_t erd_launch_trace(const erd::DevParams* p, float4* frame, u
     erd::ScatterRec* q = (erd::ScatterRec*)queue;
     erd::EventRec* ev = (erd::EventRec*)events;
     erd::ShadowJob* jb = (erd::ShadowJob*)jobs;
-#define ER_ALL(F, C, L) launch_all<F, C, L>(p, frame, s1, s2, q, counts, ev, jb, vis, counters, tiles_x, ntiles, nblocks, \
+#define ER_ALL(M, C, L) launch_all<M, C, L>(full, p, frame, s1, s2, q, counts, ev, jb, vis, counters, tiles_x, ntiles, nblocks, \
                                             shade_blocks, std::max(1, shadow_blocks), lds_bytes, st, st2, \
                                             shaded, after_primary, order_in, cost, order_out, heavy_cap, lpr, \
                                             (shadow_lanes_per_ray == 4 || shadow_lanes_per_ray == 16) ? shadow_lanes_per_ray : 1, \
                                             heavy_lanes_per_ray)
-    if (full) {
-        if (count) { if (lut_lds) ER_ALL(1, 1, 1); else ER_ALL(1, 1, 0); }
-        else { if (lut_lds) ER_ALL(1, 0, 1); else ER_ALL(1, 0, 0); }
-    } else {
-        if (count) { if (lut_lds) ER_ALL(0, 1, 1); else ER_ALL(0, 1, 0); }
-        else { if (lut_lds) ER_ALL(0, 0, 1); else ER_ALL(0, 0, 0); }
-    }
+    if (count) { if (lut_lds) ER_ALL(ER_MARCH_ANY, 1, 1); else ER_ALL(ER_MARCH_ANY, 1, 0); }
+    else if (plain) { if (lut_lds) ER_ALL(ER_MARCH_PLAIN, 0, 1); else ER_ALL(ER_MARCH_PLAIN, 0, 0); }
+    else { if (lut_lds) ER_ALL(ER_MARCH_ANY, 0, 1); else ER_ALL(ER_MARCH_ANY, 0, 0); }
 #undef ER_ALL
     return hipGetLastError();
 }
@@ -1302,27 +1313,24 @@ static void launch_shadow_b(const erd::BatchJob* J, int na, int lpr, int blocks,
 
 /* na: the jobs taking part in this round, the first na of the job table (the table is ordered
  * by pass count, largest first) */
-extern "C" hipError_t erd_launch_batch_trace(const erd::BatchJob* J, int na, int full, int primary_blocks,
+extern "C" hipError_t erd_launch_batch_trace(const erd::BatchJob* J, int na, int full, int plain, int primary_blocks,
                                              int lds_words, int shade_blocks, hipStream_t stream,
                                              hipStream_t stream2, hipEvent_t shaded, int lpr, int shadow_lpr)
 {
     /* lds_words > 0: every job's tables fit in that many words of LDS */
     const size_t lds = (size_t)lds_words * 4;
 #define ER_PRIMARY_B(F, L) launch_primary_b<F, L>(J, na, lpr, primary_blocks, lds, stream)
-    if (full) {
-        if (lds_words > 0) ER_PRIMARY_B(1, 1); else ER_PRIMARY_B(1, 0);
-        hipLaunchKernelGGL(erd::k_shade_b<1>, dim3(shade_blocks), dim3(256), 0, stream, J, na);
-    } else {
-        if (lds_words > 0) ER_PRIMARY_B(0, 1); else ER_PRIMARY_B(0, 0);
-        hipLaunchKernelGGL(erd::k_shade_b<0>, dim3(shade_blocks), dim3(256), 0, stream, J, na);
-    }
+    if (plain) { if (lds_words > 0) ER_PRIMARY_B(ER_MARCH_PLAIN, 1); else ER_PRIMARY_B(ER_MARCH_PLAIN, 0); }
+    else { if (lds_words > 0) ER_PRIMARY_B(ER_MARCH_ANY, 1); else ER_PRIMARY_B(ER_MARCH_ANY, 0); }
+    if (full) hipLaunchKernelGGL(erd::k_shade_b<1>, dim3(shade_blocks), dim3(256), 0, stream, J, na);
+    else hipLaunchKernelGGL(erd::k_shade_b<0>, dim3(shade_blocks), dim3(256), 0, stream, J, na);
 #undef ER_PRIMARY_B
     hipError_t e = hipEventRecord(shaded, stream);
     if (e == hipSuccess) e = hipStreamWaitEvent(stream2, shaded, 0);
     if (e != hipSuccess) return e;
 #define ER_SHADOW_B(F, L) launch_shadow_b<F, L>(J, na, shadow_lpr, primary_blocks, lds, stream2)
-    if (full) { if (lds_words > 0) ER_SHADOW_B(1, 1); else ER_SHADOW_B(1, 0); }
-    else { if (lds_words > 0) ER_SHADOW_B(0, 1); else ER_SHADOW_B(0, 0); }
+    if (plain) { if (lds_words > 0) ER_SHADOW_B(ER_MARCH_PLAIN, 1); else ER_SHADOW_B(ER_MARCH_PLAIN, 0); }
+    else { if (lds_words > 0) ER_SHADOW_B(ER_MARCH_ANY, 1); else ER_SHADOW_B(ER_MARCH_ANY, 0); }
 #undef ER_SHADOW_B
     hipLaunchKernelGGL(erd::k_finish_b, dim3(shade_blocks), dim3(256), 0, stream2, J, na);
     return hipGetLastError();
@@ -1346,7 +1354,7 @@ extern "C" hipError_t erd_launch_round_end(const erd::BatchJob* J, int njobs, hi
  * follows them with its own kernels) */
 extern "C" hipError_t erd_launch_primary_shade(const erd::DevParams* p, float4* frame, uint32_t* s1, uint32_t* s2,
                                                void* queue, unsigned int* counts, void* events, void* jobs, int W, int H,
-                                               int lut_lds, size_t lds_bytes, int shade_blocks,
+                                               int plain, int lut_lds, size_t lds_bytes, int shade_blocks,
                                                int primary_blocks, int tile_shift, hipStream_t st)
 {
     const int tw = 1 << tile_shift, th = 64 >> tile_shift;
@@ -1355,12 +1363,12 @@ extern "C" hipError_t erd_launch_primary_shade(const erd::DevParams* p, float4* 
     constexpr int wpb = ER_PRIMARY_WG / 64;   /* waves per workgroup */
     const int nblocks = std::max(1, std::min((ntiles + wpb - 1) / wpb, primary_blocks));
     erd::ScatterRec* q = (erd::ScatterRec*)queue;
-    if (lut_lds)
-        hipLaunchKernelGGL((erd::k_primary<1, 0, 1, 1>), dim3(nblocks), dim3(ER_PRIMARY_WG), lds_bytes, st, p, frame, s1, s2, q, counts,
-                           (unsigned long long*)nullptr, tiles_x, ntiles, (const uint32_t*)nullptr, (uint32_t*)nullptr, 64);
-    else
-        hipLaunchKernelGGL((erd::k_primary<1, 0, 0, 1>), dim3(nblocks), dim3(ER_PRIMARY_WG), lds_bytes, st, p, frame, s1, s2, q, counts,
-                           (unsigned long long*)nullptr, tiles_x, ntiles, (const uint32_t*)nullptr, (uint32_t*)nullptr, 64);
+#define ER_PRIMARY(M, L) hipLaunchKernelGGL((erd::k_primary<M, 0, L, 1>), dim3(nblocks), dim3(ER_PRIMARY_WG), lds_bytes, st, p, \
+                                            frame, s1, s2, q, counts, (unsigned long long*)nullptr, tiles_x, ntiles, \
+                                            (const uint32_t*)nullptr, (uint32_t*)nullptr, 64)
+    if (plain) { if (lut_lds) ER_PRIMARY(ER_MARCH_PLAIN, 1); else ER_PRIMARY(ER_MARCH_PLAIN, 0); }
+    else { if (lut_lds) ER_PRIMARY(ER_MARCH_ANY, 1); else ER_PRIMARY(ER_MARCH_ANY, 0); }
+#undef ER_PRIMARY
     hipLaunchKernelGGL((erd::k_shade<1, 0>), dim3(shade_blocks), dim3(256), 0, st, p, s1, s2, (const erd::ScatterRec*)q, counts, (erd::EventRec*)events, (erd::ShadowJob*)jobs,
                        (unsigned long long*)nullptr);
     return hipGetLastError();
@@ -1372,19 +1380,19 @@ extern "C" size_t erd_autofocus_out_offset(void) { return offsetof(erd::FocusWor
 /* work: erd_autofocus_work_size() bytes, zero before the first call; the distance is left at
  * erd_autofocus_out_offset(). serial: the one-lane form (Woodcock tracking). */
 extern "C" hipError_t erd_launch_autofocus(const erd::DevParams* p, int u, int v, uint32_t s0, uint32_t s1, void* work,
-                                           int full, int serial, int lut_lds, size_t lds_bytes, hipStream_t st)
+                                           int plain, int serial, int lut_lds, size_t lds_bytes, hipStream_t st)
 {
     erd::FocusWork* w = (erd::FocusWork*)work;
     const dim3 grid((ER_FOCUS_RAYS + 3) / 4), block(256);
     if (serial)
         hipLaunchKernelGGL(erd::k_autofocus_serial, dim3(1), dim3(64), 0, st, p, u, v, s0, s1, &w->out);
-    else if (full && lut_lds)
-        hipLaunchKernelGGL((erd::k_autofocus<1, 1>), grid, block, lds_bytes, st, p, u, v, s0, s1, w);
-    else if (full)
-        hipLaunchKernelGGL((erd::k_autofocus<1, 0>), grid, block, lds_bytes, st, p, u, v, s0, s1, w);
+    else if (plain && lut_lds)
+        hipLaunchKernelGGL((erd::k_autofocus<ER_MARCH_PLAIN, 1>), grid, block, lds_bytes, st, p, u, v, s0, s1, w);
+    else if (plain)
+        hipLaunchKernelGGL((erd::k_autofocus<ER_MARCH_PLAIN, 0>), grid, block, lds_bytes, st, p, u, v, s0, s1, w);
     else if (lut_lds)
-        hipLaunchKernelGGL((erd::k_autofocus<0, 1>), grid, block, lds_bytes, st, p, u, v, s0, s1, w);
+        hipLaunchKernelGGL((erd::k_autofocus<ER_MARCH_ANY, 1>), grid, block, lds_bytes, st, p, u, v, s0, s1, w);
     else
-        hipLaunchKernelGGL((erd::k_autofocus<0, 0>), grid, block, lds_bytes, st, p, u, v, s0, s1, w);
+        hipLaunchKernelGGL((erd::k_autofocus<ER_MARCH_ANY, 0>), grid, block, lds_bytes, st, p, u, v, s0, s1, w);
     return hipGetLastError();
 }

@@ -306,27 +306,35 @@ __global__ __launch_bounds__(256) void k_macro_sigma(const uint32_t* __restrict_
  * next[i] is the smallest intensity >= i whose sigma is positive (0xffffffff: none), so the test
  * over the macrocell's range of intensities is one table read; gone (may be NULL) has bit m set
  * when every sample of macrocell m is clipped away (the host's conservative test; clipping
- * objects apply in the full estimator only). One lane per macrocell, a ballot for 64 bits. */
+ * objects apply in the full estimator only); with unclipped, whose bit m is set when no sample of
+ * macrocell m is, cut gets the macrocells that can hold such a sample and are not wholly
+ * unclipped. One lane per macrocell, a ballot for 64 bits. */
 __global__ __launch_bounds__(256) void k_macro_bits(const uint32_t* __restrict__ mm, const uint32_t* __restrict__ next,
                                                    int lut_max, const uint32_t* __restrict__ gone,
-                                                   uint32_t* __restrict__ bits, int n, int words)
+                                                   const uint32_t* __restrict__ unclipped, uint32_t* __restrict__ bits,
+                                                   uint32_t* __restrict__ cut, int n, int words)
 {
     const int m = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    bool occ = false;
+    bool occ = false, part = false;
     if (m < n) {
         int lo, hi;
         sample_range(mm[m], lut_max, lo, hi);
-        occ = next[lo] <= (uint32_t)hi && !(gone && ((gone[m >> 5] >> (m & 31)) & 1u));
+        occ = next[lo] <= (uint32_t)hi;
+        part = occ && unclipped && !((unclipped[m >> 5] >> (m & 31)) & 1u);
+        occ = occ && !(gone && ((gone[m >> 5] >> (m & 31)) & 1u));
     }
-    const unsigned long long v = __ballot(occ);
-    if ((threadIdx.x & 31) == 0 && (m >> 5) < words) bits[m >> 5] = (uint32_t)(v >> (threadIdx.x & 32));
+    const unsigned long long v = __ballot(occ), c = __ballot(part);
+    if ((threadIdx.x & 31) == 0 && (m >> 5) < words) {
+        bits[m >> 5] = (uint32_t)(v >> (threadIdx.x & 32));
+        if (cut) cut[m >> 5] = (uint32_t)(c >> (threadIdx.x & 32));
+    }
 }
 
 /* group bits: bit g set iff any macrocell of group g (2^ER_GROUP_SHIFT macrocells a side, clipped to the
  * grid) has its bit set, from word `occ_base` of the same array; the groups' clip-free bits
- * from word `free_base`: bit g set iff every occupied macrocell of group g is wholly unclipped
- * (bit m of `unclipped`, the host's conservative test; NULL: no clipping objects, every bit
- * clear), so the march need not test its samples against them. One lane per group, which reads
+ * from word `free_base`: bit g set iff no macrocell of group g has its bit in `cut` (k_macro_bits;
+ * NULL: no clipping objects, every bit clear), so the march need not test its samples against
+ * the clipping objects. One lane per group, which reads
  * its macrocells' bits a row of 4 at a time (one lane per 32 groups, bit by bit, took 340 us for
  * 16^3 groups; this takes 5). */
 __device__ __forceinline__ uint32_t bit_run(const uint32_t* __restrict__ w, int first, int count)
@@ -336,12 +344,12 @@ __device__ __forceinline__ uint32_t bit_run(const uint32_t* __restrict__ w, int 
     if (s + count > 32) v |= w[(first >> 5) + 1] << (32 - s);
     return v & ((1u << count) - 1u);
 }
-__global__ __launch_bounds__(256) void k_group_bits(uint32_t* __restrict__ bits, const uint32_t* __restrict__ unclipped,
+__global__ __launch_bounds__(256) void k_group_bits(uint32_t* __restrict__ bits, const uint32_t* __restrict__ cut,
                                                    int mx, int my, int mz, int gx, int gy, int gz, int occ_base,
                                                    int free_base, int words)
 {
     const int g = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    bool any = false, free = unclipped != nullptr;
+    bool any = false, free = cut != nullptr;
     if (g < gx * gy * gz) {
         const int E = 1 << ER_GROUP_SHIFT;
         const int x = g % gx, y = (g / gx) % gy, z = g / (gx * gy);
@@ -349,9 +357,8 @@ __global__ __launch_bounds__(256) void k_group_bits(uint32_t* __restrict__ bits,
         for (int k = E * z; k < min(E * z + E, mz); ++k)
             for (int j = E * y; j < min(E * y + E, my); ++j) {
                 const int m = (k * my + j) * mx + E * x;
-                const uint32_t o = bit_run(bits, m, nx);
-                any = any || o != 0u;
-                if (unclipped) free = free && (o & ~bit_run(unclipped, m, nx)) == 0u;
+                any = any || bit_run(bits, m, nx) != 0u;
+                if (cut) free = free && bit_run(cut, m, nx) == 0u;
             }
     } else {
         free = false;
@@ -537,15 +544,17 @@ extern "C" hipError_t erd_launch_macro_minmax(const uint16_t* vox, uint32_t* mm,
 }
 
 extern "C" hipError_t erd_launch_macro_bits(const uint32_t* mm, const uint32_t* next, int lut_max, const uint32_t* gone,
-                                            uint32_t* bits, int n, int words, hipStream_t st)
+                                            const uint32_t* unclipped, uint32_t* bits, uint32_t* cut, int n, int words,
+                                            hipStream_t st)
 {
-    hipLaunchKernelGGL(erd::k_macro_bits, dim3((n + 255) / 256), dim3(256), 0, st, mm, next, lut_max, gone, bits, n, words);
+    hipLaunchKernelGGL(erd::k_macro_bits, dim3((n + 255) / 256), dim3(256), 0, st, mm, next, lut_max, gone, unclipped, bits, cut,
+                       n, words);
     return hipGetLastError();
 }
 
 /* the groups' occupancy bits (from word occ_base), clip-free bits (free_base) and radii
  * (radii_base); tmp: two bytes a group */
-extern "C" hipError_t erd_launch_group_tables(uint32_t* bits, const uint32_t* unclipped, uint8_t* tmp, int mx, int my, int mz,
+extern "C" hipError_t erd_launch_group_tables(uint32_t* bits, const uint32_t* cut, uint8_t* tmp, int mx, int my, int mz,
                                               int gx, int gy, int gz, int occ_base, int free_base, int radii_base, int words,
                                               hipStream_t st)
 {
@@ -553,7 +562,7 @@ extern "C" hipError_t erd_launch_group_tables(uint32_t* bits, const uint32_t* un
     const dim3 grid((n + 255) / 256), block(256);
     uint8_t* tmp2 = tmp + n;
     const uint32_t* occ = bits + occ_base;
-    hipLaunchKernelGGL(erd::k_group_bits, grid, block, 0, st, bits, unclipped, mx, my, mz, gx, gy, gz, occ_base, free_base, words);
+    hipLaunchKernelGGL(erd::k_group_bits, grid, block, 0, st, bits, cut, mx, my, mz, gx, gy, gz, occ_base, free_base, words);
     hipLaunchKernelGGL(erd::k_group_radii<0>, grid, block, 0, st, occ, (const uint8_t*)nullptr, tmp, (uint32_t*)nullptr, gx, gy, gz);
     hipLaunchKernelGGL(erd::k_group_radii<1>, grid, block, 0, st, occ, (const uint8_t*)tmp, tmp2, (uint32_t*)nullptr, gx, gy, gz);
     hipLaunchKernelGGL(erd::k_group_radii<2>, grid, block, 0, st, occ, (const uint8_t*)tmp2, tmp, bits + radii_base, gx, gy, gz);

@@ -34,7 +34,7 @@ using erd::DevParams;
 
 extern "C" hipError_t erd_launch_trace(const DevParams* p, float4* frame, uint32_t* s1, uint32_t* s2, void* queue,
                                        unsigned int* counts, void* events, void* jobs, unsigned char* vis,
-                                       unsigned long long* counters, int W, int H, int full, int plain, int count,
+                                       unsigned long long* counters, int W, int H, int full, int march, int count,
                                        int lut_lds, size_t lds_bytes, int shade_blocks, int primary_blocks,
                                        int shadow_blocks, int tile_shift, hipStream_t st,
                                        hipStream_t st2, hipEvent_t shaded, hipEvent_t after_primary,
@@ -44,8 +44,9 @@ extern "C" void erd_pass_record_sizes(size_t* scatter, size_t* event, size_t* jo
 extern "C" hipError_t erd_launch_post(const DevParams* p, const float4* frame, float4* running, uchar4* display,
                                       int no_iterations, unsigned int* qcount, int W, int H, hipStream_t st);
 extern "C" hipError_t erd_launch_macro_bits(const uint32_t* mm, const uint32_t* next, int lut_max, const uint32_t* gone,
-                                            uint32_t* bits, int n, int words, hipStream_t st);
-extern "C" hipError_t erd_launch_group_tables(uint32_t* bits, const uint32_t* unclipped, uint8_t* tmp, int mx, int my, int mz,
+                                            const uint32_t* unclipped, uint32_t* bits, uint32_t* cut, int n, int words,
+                                            hipStream_t st);
+extern "C" hipError_t erd_launch_group_tables(uint32_t* bits, const uint32_t* cut, uint8_t* tmp, int mx, int my, int mz,
                                               int gx, int gy, int gz, int occ_base, int free_base, int radii_base, int words,
                                               hipStream_t st);
 extern "C" hipError_t erd_launch_bilateral(const void* bp, const uchar4* in, uchar4* tmp, uchar4* out, int W, int H,
@@ -59,7 +60,7 @@ extern "C" hipError_t erd_launch_macro_sigma(const uint32_t* mm, const float* lu
                                              hipStream_t st);
 extern "C" hipError_t erd_launch_gm_max(const DevParams* p, const uint16_t* vox, float* bounds, unsigned int* out, int rx,
                                         int ry, int rz, int prune, hipStream_t st);
-extern "C" hipError_t erd_launch_batch_trace(const erd::BatchJob* J, int na, int full, int plain, int primary_blocks,
+extern "C" hipError_t erd_launch_batch_trace(const erd::BatchJob* J, int na, int full, int march, int primary_blocks,
                                              int lds_words, int shade_blocks, hipStream_t stream,
                                              hipStream_t stream2, hipEvent_t shaded, int lpr, int shadow_lpr);
 extern "C" hipError_t erd_launch_batch_post(const erd::BatchJob* J, int na, unsigned int round, int active_tiles,
@@ -68,7 +69,7 @@ extern "C" hipError_t erd_launch_round_end(const erd::BatchJob* J, int njobs, hi
 extern "C" hipError_t erd_batch_params_upload(const erd::DevParams* host, int n);
 extern "C" size_t erd_adj_partials_per_block(void);
 extern "C" hipError_t erd_launch_primary_shade(const DevParams* p, float4* frame, uint32_t* s1, uint32_t* s2, void* queue,
-                                               unsigned int* counts, void* events, void* jobs, int W, int H, int plain, int lut_lds,
+                                               unsigned int* counts, void* events, void* jobs, int W, int H, int march, int lut_lds,
                                                size_t lds_bytes, int shade_blocks, int primary_blocks,
                                                int tile_shift, hipStream_t st);
 extern "C" hipError_t erd_launch_adj_wavefront(const DevParams* p, unsigned int* counts, const void* jobs, const void* events,
@@ -78,7 +79,7 @@ extern "C" hipError_t erd_launch_adj_wavefront(const DevParams* p, unsigned int*
 extern "C" hipError_t erd_launch_adj_reset(unsigned int* counts, unsigned int* lcount, hipStream_t st);
 extern "C" size_t erd_autofocus_work_size(void);
 extern "C" size_t erd_autofocus_out_offset(void);
-extern "C" hipError_t erd_launch_autofocus(const DevParams* p, int u, int v, uint32_t s0, uint32_t s1, void* work, int plain,
+extern "C" hipError_t erd_launch_autofocus(const DevParams* p, int u, int v, uint32_t s0, uint32_t s1, void* work, int march,
                                            int serial, int lut_lds, size_t lds_bytes, hipStream_t st);
 extern "C" hipError_t erd_launch_adjoint(const DevParams* p, int mode, const float* lut_eval, const float* sigma_eval,
                                          const float4* adj, float4* value, float* partials, uint32_t* s1, uint32_t* s2,
@@ -433,7 +434,7 @@ struct Tracer {
     size_t lds_bytes = 0;
     int lut_lds = 0;
     int lut_nonneg = 0;              /* no entry of the opacity table is negative or NaN */
-    int plain = 0;                   /* the marches may take their plain form (ER_MARCH_PLAIN) */
+    int march = ER_MARCH_ANY;        /* the marches' form for this scene */
     DevBuf<DevParams> params;
     DevParams* params_pinned = nullptr;   /* the copy the upload reads */
     /* what the tables above (opacity, occupancy, radii, majorants) were built from, by value:
@@ -1158,7 +1159,8 @@ int build_params(Tracer& t)
     }
     P.sigma_lut = t.lut.ptr;
     P.lut_max = lut_n - 1;
-    t.plain = t.lut_nonneg && P.clip_count == 0 && !woodcock;
+    t.march = !t.lut_nonneg ? ER_MARCH_ANY
+              : (woodcock ? ER_MARCH_WOODCOCK : (P.clip_count > 0 ? ER_MARCH_CLIP : ER_MARCH_PLAIN));
     const int nmc = grid->mc[0] * grid->mc[1] * grid->mc[2];
     P.mc_shift = mc_shift;
     /* Woodcock majorants on their own fixed grid of 2^ER_WC_SHIFT-cell macrocells */
@@ -1191,18 +1193,21 @@ int build_params(Tracer& t)
         /* macrocells wholly clipped away count as empty */
         const uint32_t* clipped = nullptr;
         const uint32_t* unclipped = nullptr;
+        uint32_t* cut = nullptr;
         if (P.clip_count > 0) {
             std::vector<uint32_t> free;
             clip_classes(P, nmc, edge_ext, classes, free);
             classes.insert(classes.end(), free.begin(), free.end());
-            if ((st = t.clip_bits.alloc(classes.size()))) return st;
+            if ((st = t.clip_bits.alloc(classes.size() + mc_words))) return st;
             HIP_TRY(hipMemcpyAsync(t.clip_bits.ptr, classes.data(), classes.size() * sizeof(uint32_t), hipMemcpyHostToDevice,
                                    t.stream));
             clipped = t.clip_bits.ptr;
             unclipped = t.clip_bits.ptr + mc_words;
+            cut = t.clip_bits.ptr + 2 * (size_t)mc_words;
         }
-        HIP_TRY(erd_launch_macro_bits(grid->mm.ptr, t.lut_next.ptr, P.lut_max, clipped, t.mc_bits.ptr, nmc, mc_words, t.stream));
-        HIP_TRY(erd_launch_group_tables(t.mc_bits.ptr, unclipped, t.group_tmp.ptr, grid->mc[0], grid->mc[1], grid->mc[2],
+        HIP_TRY(erd_launch_macro_bits(grid->mm.ptr, t.lut_next.ptr, P.lut_max, clipped, unclipped, t.mc_bits.ptr, cut, nmc,
+                                      mc_words, t.stream));
+        HIP_TRY(erd_launch_group_tables(t.mc_bits.ptr, cut, t.group_tmp.ptr, grid->mc[0], grid->mc[1], grid->mc[2],
                                         P.mc2_dim[0], P.mc2_dim[1], P.mc2_dim[2], occ_base, P.mc3_base, P.mc2_base, g_words,
                                         t.stream));
     }
@@ -1310,7 +1315,7 @@ int enqueue_pass(Tracer& t, hipEvent_t* e)
 #endif
     const bool reorder = !order_valid || (t.desc.no_iterations & ER_REORDER_MASK) == 0;
     HIP_TRY(erd_launch_trace(t.params.ptr, S.frame.ptr, t.seeds1.ptr, t.seeds2.ptr, S.queue.ptr, S.qcount.ptr,
-                             S.events.ptr, S.jobs.ptr, S.vis.ptr, t.counters.ptr, t.W, t.H, full, t.plain, t.counting, t.lut_lds,
+                             S.events.ptr, S.jobs.ptr, S.vis.ptr, t.counters.ptr, t.W, t.H, full, t.march, t.counting, t.lut_lds,
                              t.lds_bytes, shade_blocks, primary_blocks(t), shadow_blocks(t), t.tile_shift, t.stream,
                              t.stream2, S.shaded, e ? e[1] : nullptr, order_valid ? t.tile_order.ptr : nullptr,
                              t.tile_cost.ptr, reorder ? t.tile_order.ptr : nullptr, t.heavy_tiles,
@@ -2132,8 +2137,16 @@ static int render_batch_chunk(std::vector<std::pair<int, Tracer*>>& jobs, int fu
     if (!all_lds) lds_words = 0;
     /* lanes per primary and shadow march, for the whole batch: the jobs' common rays per wave
      * (one lane per ray when they differ, or when a job uses Woodcock tracking) */
-    int plain = 1;   /* the marches' plain form, when every job's scene allows it */
-    for (auto& j : jobs) plain = plain && j.second->plain;
+    /* the marches' form: the jobs' common one; ER_MARCH_CLIP renders scenes without clipping
+     * objects as well */
+    int march = jobs[0].second->march;
+    for (auto& j : jobs) {
+        const int m = j.second->march;
+        if (m == march) continue;
+        const bool clip = (m == ER_MARCH_CLIP || m == ER_MARCH_PLAIN) && (march == ER_MARCH_CLIP || march == ER_MARCH_PLAIN);
+        march = clip ? ER_MARCH_CLIP : ER_MARCH_ANY;
+        if (!clip) break;
+    }
     int lpr = 64 / jobs[0].second->rays_per_wave, slpr = 64 / jobs[0].second->shadow_rays_per_wave;
     for (auto& j : jobs) {
         const Tracer& t = *j.second;
@@ -2145,7 +2158,7 @@ static int render_batch_chunk(std::vector<std::pair<int, Tracer*>>& jobs, int fu
     /* the graph's key: the job tables without their first pass numbers, and the launch shape */
     std::string key;
     {
-        const int hdr[8] = {nj, full, plain, batch_blocks, lds_words, shade_blocks, lpr, slpr};
+        const int hdr[8] = {nj, full, march, batch_blocks, lds_words, shade_blocks, lpr, slpr};
         key.append((const char*)hdr, sizeof(hdr));
         for (int b = 0; b < 2; ++b)
             for (int k = 0; k < nj; ++k) {
@@ -2197,7 +2210,7 @@ static int render_batch_chunk(std::vector<std::pair<int, Tracer*>>& jobs, int fu
             hipEvent_t shaded = nullptr;
             if (ec == hipSuccess) ec = new_event(shaded);
             if (ec == hipSuccess)
-                ec = erd_launch_batch_trace(dJ[b].ptr, na, full, plain, batch_blocks, lds_words, shade_blocks, bs, bs2, shaded, lpr,
+                ec = erd_launch_batch_trace(dJ[b].ptr, na, full, march, batch_blocks, lds_words, shade_blocks, bs, bs2, shaded, lpr,
                                             slpr);
             if (ec == hipSuccess) ec = erd_launch_batch_post(dJ[b].ptr, na, (unsigned int)r, active_tiles, bs2);
             if (ec == hipSuccess) ec = erd_launch_round_end(dJ[b].ptr, nj, bs2);
@@ -2362,7 +2375,7 @@ ER_API int er_adjoint_lut(int tracer_id, const uint32_t* seeds1, const uint32_t*
         }
         /* the forward pass's primary and shading kernels: decisions, queues, final seeds */
         HIP_TRY(erd_launch_primary_shade(t->params.ptr, A.frame.ptr, W.d1.ptr, W.d2.ptr, A.queue.ptr, A.counts.ptr, A.events.ptr,
-                                         A.jobs.ptr, t->W, t->H, t->plain, t->lut_lds, t->lds_bytes, shade_blocks,
+                                         A.jobs.ptr, t->W, t->H, t->march, t->lut_lds, t->lds_bytes, shade_blocks,
                                          primary_blocks(*t), t->tile_shift, s));
         HIP_TRY(hipEventRecord(A.shaded, s));
         HIP_TRY(hipStreamWaitEvent(s2, A.shaded, 0));
@@ -2442,7 +2455,7 @@ ER_API int er_adjoint_lut_noalloc(int tracer_id, const uint32_t* seeds1, const u
             HIP_TRY(hipMemcpyAsync(s1s, d1, n * 4, hipMemcpyDeviceToDevice, s));
             HIP_TRY(hipMemcpyAsync(s2s, d2, n * 4, hipMemcpyDeviceToDevice, s));
         }
-        HIP_TRY(erd_launch_primary_shade(t->params.ptr, frame, d1, d2, queue, counts, events, jobs, t->W, t->H, t->plain, t->lut_lds,
+        HIP_TRY(erd_launch_primary_shade(t->params.ptr, frame, d1, d2, queue, counts, events, jobs, t->W, t->H, t->march, t->lut_lds,
                                          t->lds_bytes, shade_blocks, primary_blocks(*t), t->tile_shift, s));
         if (w != 0.0f) {
             if (w != cur_w) {
@@ -2581,7 +2594,7 @@ ER_API int er_get_autofocus_distance(int tracer_id, int film_u, int film_v, floa
     }
     const int full = t->desc.settings.estimator == ER_ESTIMATOR_FULL;
     const int serial = full && t->desc.settings.sampler == ER_SAMPLER_WOODCOCK;
-    HIP_TRY(erd_launch_autofocus(t->params.ptr, film_u, film_v, s0, s1, t->focus.ptr, t->plain, serial, t->lut_lds, t->lds_bytes,
+    HIP_TRY(erd_launch_autofocus(t->params.ptr, film_u, film_v, s0, s1, t->focus.ptr, t->march, serial, t->lut_lds, t->lds_bytes,
                                  t->stream));
     HIP_TRY(hipMemcpyAsync(distance, t->focus.ptr + erd_autofocus_out_offset(), sizeof(float), hipMemcpyDeviceToHost, t->stream));
     HIP_TRY(hipStreamSynchronize(t->stream));

@@ -42,7 +42,7 @@ __device__ __forceinline__ Tables stage_tables(const DevParams& p, uint32_t* lds
         float* lut = (float*)(lds + nw);
         for (int k = threadIdx.x; k <= p.lut_max; k += blockDim.x) {
             const float s = gmem(p.sigma_lut)[k];
-            lut[k] = FULL == ER_MARCH_PLAIN ? s * step : s;
+            lut[k] = ER_MARCH_IS_PLAIN(FULL) ? s * step : s;
         }
         T.lut_lds = lut;
         T.lut_glb = nullptr;
@@ -117,6 +117,7 @@ __device__ __forceinline__ void primary_tile(const DevParams& p, const Tables& T
     Ray r;
     bool vol = false, marching = false;
     float Tv = 0.0f;
+    int it = 0;
     MarchState m;
     const float StepSize = p.step_primary * p.minstep;
     if (active) {
@@ -125,19 +126,19 @@ __device__ __forceinline__ void primary_tile(const DevParams& p, const Tables& T
         rng.s1 = seeds2[i];
         r = camera_ray(p, px, py, rng, smp);
         D = r.D;
-        if (FULL == ER_MARCH_ANY && p.sampler == ER_SAMPLER_WOODCOCK) {
-            vol = march<FULL, COUNT, ER_BATCH_PRIMARY>(p, T, r, true, rng, Tv, Pv, cnt);
-        } else {
+        float nearT, farT;
+        if (!intersect_box(r, ld3(p.minp), ld3(p.maxp), nearT, farT)) {
+        } else if (FULL == ER_MARCH_WOODCOCK || (FULL == ER_MARCH_ANY && p.sampler == ER_SAMPLER_WOODCOCK)) {
+            vol = woodcock_track<FULL, COUNT>(p, T, r, nearT, farT, true, rng, Tv, Pv, cnt);
+        } else if constexpr (FULL != ER_MARCH_WOODCOCK) {
             /* march_v's set-up; its loop follows, wave by wave */
-            float nearT, farT;
-            if (intersect_box(r, ld3(p.minp), ld3(p.maxp), nearT, farT) &&
-                march_begin(p, r, nearT, farT, StepSize, rng, -1.0f, m)) {
+            if (march_begin(p, r, nearT, farT, StepSize, rng, -1.0f, m)) {
                 if (!(m.Sum < m.S)) { vol = true; Tv = m.MinT; Pv = mk(0.0f, 0.0f, 0.0f); }
                 else marching = true;
             }
         }
     }
-    /* The march loop, in three stages: every lane steps its own march until at most 64 / GD
+    /* The march loop (Woodcock walks are done), in three stages: every lane steps its own march until at most 64 / GD
      * lanes (ER_COOP_LANES without group tails) are still marching; groups of GD lanes then
      * take those marches over; a march left after that (a single-ray wave's) is finished by the
      * whole wave (coop_march). A lone ray through kilo-samples of tissue would otherwise keep its
@@ -146,8 +147,8 @@ __device__ __forceinline__ void primary_tile(const DevParams& p, const Tables& T
      * it: the lane's march iterations (the group and wave stages count their equivalents), for
      * the tile cost. */
     NoVisit nv;
-    int it = 0;
-    if constexpr (G > 1) {
+    if constexpr (FULL == ER_MARCH_WOODCOCK) {
+    } else if constexpr (G > 1) {
         if (marching) {
             f3 P = mk(0.0f, 0.0f, 0.0f);
             const int st = group_march<FULL, COUNT, G>(p, T, m, StepSize, lane, cnt, P, it);
@@ -405,7 +406,7 @@ __global__ __launch_bounds__(ER_PRIMARY_WG) __attribute__((amdgpu_waves_per_eu(E
      * order */
     const unsigned int HL = heavy_lanes == 4 || heavy_lanes == 16 ? (unsigned int)heavy_lanes : 64u;
     unsigned int hc = order ? min((unsigned int)__builtin_amdgcn_readfirstlane(order[ntiles]), (unsigned int)ntiles) : 0u;
-    if ((FULL == ER_MARCH_ANY && p.sampler == ER_SAMPLER_WOODCOCK) || LPR > 1) hc = 0u;
+    if (FULL == ER_MARCH_WOODCOCK || (FULL == ER_MARCH_ANY && p.sampler == ER_SAMPLER_WOODCOCK) || LPR > 1) hc = 0u;
     const unsigned int nclaims = LPR > 1 ? (unsigned int)ntiles * (unsigned int)LPR : hc * HL + ((unsigned int)ntiles - hc);
     for (;;) {
         unsigned int claim = 0;
@@ -425,7 +426,9 @@ __global__ __launch_bounds__(ER_PRIMARY_WG) __attribute__((amdgpu_waves_per_eu(E
         const unsigned int idx = heavy ? claim / HL : hc + (claim - hc * HL);
         const unsigned int tile = order ? __builtin_amdgcn_readfirstlane(order[idx]) : idx;
         int steps = 0;
-        if (heavy && HL == 4u)
+        if constexpr (FULL == ER_MARCH_WOODCOCK)
+            primary_tile<FULL, COUNT>(p, T, tile, tiles_x, lane, frame, seeds1, seeds2, queue, &counts[0], cnt, paths, steps, -1);
+        else if (heavy && HL == 4u)
             primary_tile<FULL, COUNT, 4>(p, T, tile, tiles_x, lane, frame, seeds1, seeds2, queue, &counts[0], cnt, paths,
                                          steps, (int)(claim % HL));
         else if (heavy && HL == 16u)
@@ -648,10 +651,11 @@ __device__ __forceinline__ void shadow_marches(const DevParams& p, const Tables&
                                                unsigned char* __restrict__ vis, unsigned int* claim, unsigned int n,
                                                unsigned int j, unsigned int claim_base, bool drained, int lane, Cnt& cnt)
 {
-    if (FULL == ER_MARCH_ANY && p.sampler == ER_SAMPLER_WOODCOCK) {
+    if (FULL == ER_MARCH_WOODCOCK || (FULL == ER_MARCH_ANY && p.sampler == ER_SAMPLER_WOODCOCK)) {
         shadow_marches_wc<FULL, COUNT>(p, T, jobq, vis, claim, n, j, claim_base, drained, lane, cnt);
         return;
     }
+    if constexpr (FULL != ER_MARCH_WOODCOCK) {
     const float StepSize = p.step_shadow * p.minstep;
     NoVisit nv;
     MarchState m;
@@ -706,6 +710,7 @@ __device__ __forceinline__ void shadow_marches(const DevParams& p, const Tables&
             if (base + (unsigned int)nidle >= n) drained = true;
             if (!busy) j = base + (unsigned int)__popcll(idle & ((1ull << lane) - 1ull));
         }
+    }
     }
 }
 
@@ -1008,7 +1013,7 @@ __device__ __forceinline__ Tables stage_job_tables(const DevParams& p, uint32_t*
     float* lut = (float*)(lds + nw);
     for (int k = threadIdx.x; k <= p.lut_max; k += blockDim.x) {
         const float s = gmem(p.sigma_lut)[k];
-        lut[k] = FULL == ER_MARCH_PLAIN ? s * step : s;
+        lut[k] = ER_MARCH_IS_PLAIN(FULL) ? s * step : s;
     }
     __syncthreads();
     Tables T;
@@ -1217,7 +1222,7 @@ extern "C" void erd_pass_record_sizes(size_t* scatter, size_t* event, size_t* jo
     *job = sizeof(erd::ShadowJob);
 }
 
-/* M: the march functions' mode (ER_MARCH_ANY or ER_MARCH_PLAIN) */
+/* M: the march functions' mode */
 template<int M, int COUNT, int LUT_LDS>
 static void launch_all(int full, const erd::DevParams* p, float4* frame, uint32_t* s1, uint32_t* s2, erd::ScatterRec* queue,
                        unsigned int* counts, erd::EventRec* events, erd::ShadowJob* jobs, unsigned char* vis,
@@ -1228,7 +1233,8 @@ static void launch_all(int full, const erd::DevParams* p, float4* frame, uint32_
 {
 #define ER_PRIMARY(G) hipLaunchKernelGGL((erd::k_primary<M, COUNT, LUT_LDS, G>), dim3(nblocks), dim3(ER_PRIMARY_WG), lds, st, p, \
                                          frame, s1, s2, queue, counts, counters, tiles_x, ntiles, order_in, cost, heavy_lanes)
-    if (lpr == 4) ER_PRIMARY(4);
+    if constexpr (M == ER_MARCH_WOODCOCK) ER_PRIMARY(1);
+    else if (lpr == 4) ER_PRIMARY(4);
     else if (lpr == 16) ER_PRIMARY(16);
     else if (lpr == 64) ER_PRIMARY(64);
     else ER_PRIMARY(1);
@@ -1244,7 +1250,8 @@ static void launch_all(int full, const erd::DevParams* p, float4* frame, uint32_
     (void)hipStreamWaitEvent(st2, shaded, 0);
 #define ER_SHADOW(G) hipLaunchKernelGGL((erd::k_shadow<M, COUNT, LUT_LDS, G>), dim3(shadow_blocks), dim3(256), lds, st2, \
                                     p, counts, (const erd::ShadowJob*)jobs, vis, counters)
-    if (shadow_lpr == 4) ER_SHADOW(4);
+    if constexpr (M == ER_MARCH_WOODCOCK) ER_SHADOW(1);
+    else if (shadow_lpr == 4) ER_SHADOW(4);
     else if (shadow_lpr == 16) ER_SHADOW(16);
     else ER_SHADOW(1);
 #undef ER_SHADOW
@@ -1257,11 +1264,11 @@ static void launch_all(int full, const erd::DevParams* p, float4* frame, uint32_
 }
 
 /* One pass's trace kernels: primary and shading on st; shadow marches and combine on st2
- * after the shading (event `shaded`). The caller runs post-processing on st2. plain: the marches
- * may take their ER_MARCH_PLAIN form (the counting kernels never do). */
+ * after the shading (event `shaded`). The caller runs post-processing on st2. march: the marches'
+ * form for the scene (the counting kernels take the general one). */
 extern "C" hipError_t erd_launch_trace(const erd::DevParams* p, float4* frame, uint32_t* s1, uint32_t* s2, void* queue,
                                        unsigned int* counts, void* events, void* jobs, unsigned char* vis,
-                                       unsigned long long* counters, int W, int H, int full, int plain, int count,
+                                       unsigned long long* counters, int W, int H, int full, int march, int count,
                                        int lut_lds, size_t lds_bytes, int shade_blocks, int primary_blocks,
                                        int shadow_blocks, int tile_shift, hipStream_t st,
                                        hipStream_t st2, hipEvent_t shaded, hipEvent_t after_primary,
@@ -1285,7 +1292,9 @@ extern "C" hipError_t erd_launch_trace(const erd::DevParams* p, float4* frame, u
                                             (shadow_lanes_per_ray == 4 || shadow_lanes_per_ray == 16) ? shadow_lanes_per_ray : 1, \
                                             heavy_lanes_per_ray)
     if (count) { if (lut_lds) ER_ALL(ER_MARCH_ANY, 1, 1); else ER_ALL(ER_MARCH_ANY, 1, 0); }
-    else if (plain) { if (lut_lds) ER_ALL(ER_MARCH_PLAIN, 0, 1); else ER_ALL(ER_MARCH_PLAIN, 0, 0); }
+    else if (march == ER_MARCH_PLAIN) { if (lut_lds) ER_ALL(ER_MARCH_PLAIN, 0, 1); else ER_ALL(ER_MARCH_PLAIN, 0, 0); }
+    else if (march == ER_MARCH_CLIP) { if (lut_lds) ER_ALL(ER_MARCH_CLIP, 0, 1); else ER_ALL(ER_MARCH_CLIP, 0, 0); }
+    else if (march == ER_MARCH_WOODCOCK) { if (lut_lds) ER_ALL(ER_MARCH_WOODCOCK, 0, 1); else ER_ALL(ER_MARCH_WOODCOCK, 0, 0); }
     else { if (lut_lds) ER_ALL(ER_MARCH_ANY, 0, 1); else ER_ALL(ER_MARCH_ANY, 0, 0); }
 #undef ER_ALL
     return hipGetLastError();
@@ -1313,14 +1322,15 @@ static void launch_shadow_b(const erd::BatchJob* J, int na, int lpr, int blocks,
 
 /* na: the jobs taking part in this round, the first na of the job table (the table is ordered
  * by pass count, largest first) */
-extern "C" hipError_t erd_launch_batch_trace(const erd::BatchJob* J, int na, int full, int plain, int primary_blocks,
+extern "C" hipError_t erd_launch_batch_trace(const erd::BatchJob* J, int na, int full, int march, int primary_blocks,
                                              int lds_words, int shade_blocks, hipStream_t stream,
                                              hipStream_t stream2, hipEvent_t shaded, int lpr, int shadow_lpr)
 {
     /* lds_words > 0: every job's tables fit in that many words of LDS */
     const size_t lds = (size_t)lds_words * 4;
 #define ER_PRIMARY_B(F, L) launch_primary_b<F, L>(J, na, lpr, primary_blocks, lds, stream)
-    if (plain) { if (lds_words > 0) ER_PRIMARY_B(ER_MARCH_PLAIN, 1); else ER_PRIMARY_B(ER_MARCH_PLAIN, 0); }
+    if (march == ER_MARCH_PLAIN) { if (lds_words > 0) ER_PRIMARY_B(ER_MARCH_PLAIN, 1); else ER_PRIMARY_B(ER_MARCH_PLAIN, 0); }
+    else if (march == ER_MARCH_CLIP) { if (lds_words > 0) ER_PRIMARY_B(ER_MARCH_CLIP, 1); else ER_PRIMARY_B(ER_MARCH_CLIP, 0); }
     else { if (lds_words > 0) ER_PRIMARY_B(ER_MARCH_ANY, 1); else ER_PRIMARY_B(ER_MARCH_ANY, 0); }
     if (full) hipLaunchKernelGGL(erd::k_shade_b<1>, dim3(shade_blocks), dim3(256), 0, stream, J, na);
     else hipLaunchKernelGGL(erd::k_shade_b<0>, dim3(shade_blocks), dim3(256), 0, stream, J, na);
@@ -1329,7 +1339,8 @@ extern "C" hipError_t erd_launch_batch_trace(const erd::BatchJob* J, int na, int
     if (e == hipSuccess) e = hipStreamWaitEvent(stream2, shaded, 0);
     if (e != hipSuccess) return e;
 #define ER_SHADOW_B(F, L) launch_shadow_b<F, L>(J, na, shadow_lpr, primary_blocks, lds, stream2)
-    if (plain) { if (lds_words > 0) ER_SHADOW_B(ER_MARCH_PLAIN, 1); else ER_SHADOW_B(ER_MARCH_PLAIN, 0); }
+    if (march == ER_MARCH_PLAIN) { if (lds_words > 0) ER_SHADOW_B(ER_MARCH_PLAIN, 1); else ER_SHADOW_B(ER_MARCH_PLAIN, 0); }
+    else if (march == ER_MARCH_CLIP) { if (lds_words > 0) ER_SHADOW_B(ER_MARCH_CLIP, 1); else ER_SHADOW_B(ER_MARCH_CLIP, 0); }
     else { if (lds_words > 0) ER_SHADOW_B(ER_MARCH_ANY, 1); else ER_SHADOW_B(ER_MARCH_ANY, 0); }
 #undef ER_SHADOW_B
     hipLaunchKernelGGL(erd::k_finish_b, dim3(shade_blocks), dim3(256), 0, stream2, J, na);
@@ -1354,7 +1365,7 @@ extern "C" hipError_t erd_launch_round_end(const erd::BatchJob* J, int njobs, hi
  * follows them with its own kernels) */
 extern "C" hipError_t erd_launch_primary_shade(const erd::DevParams* p, float4* frame, uint32_t* s1, uint32_t* s2,
                                                void* queue, unsigned int* counts, void* events, void* jobs, int W, int H,
-                                               int plain, int lut_lds, size_t lds_bytes, int shade_blocks,
+                                               int march, int lut_lds, size_t lds_bytes, int shade_blocks,
                                                int primary_blocks, int tile_shift, hipStream_t st)
 {
     const int tw = 1 << tile_shift, th = 64 >> tile_shift;
@@ -1366,7 +1377,8 @@ extern "C" hipError_t erd_launch_primary_shade(const erd::DevParams* p, float4* 
 #define ER_PRIMARY(M, L) hipLaunchKernelGGL((erd::k_primary<M, 0, L, 1>), dim3(nblocks), dim3(ER_PRIMARY_WG), lds_bytes, st, p, \
                                             frame, s1, s2, q, counts, (unsigned long long*)nullptr, tiles_x, ntiles, \
                                             (const uint32_t*)nullptr, (uint32_t*)nullptr, 64)
-    if (plain) { if (lut_lds) ER_PRIMARY(ER_MARCH_PLAIN, 1); else ER_PRIMARY(ER_MARCH_PLAIN, 0); }
+    if (march == ER_MARCH_PLAIN) { if (lut_lds) ER_PRIMARY(ER_MARCH_PLAIN, 1); else ER_PRIMARY(ER_MARCH_PLAIN, 0); }
+    else if (march == ER_MARCH_CLIP) { if (lut_lds) ER_PRIMARY(ER_MARCH_CLIP, 1); else ER_PRIMARY(ER_MARCH_CLIP, 0); }
     else { if (lut_lds) ER_PRIMARY(ER_MARCH_ANY, 1); else ER_PRIMARY(ER_MARCH_ANY, 0); }
 #undef ER_PRIMARY
     hipLaunchKernelGGL((erd::k_shade<1, 0>), dim3(shade_blocks), dim3(256), 0, st, p, s1, s2, (const erd::ScatterRec*)q, counts, (erd::EventRec*)events, (erd::ShadowJob*)jobs,
@@ -1380,15 +1392,15 @@ extern "C" size_t erd_autofocus_out_offset(void) { return offsetof(erd::FocusWor
 /* work: erd_autofocus_work_size() bytes, zero before the first call; the distance is left at
  * erd_autofocus_out_offset(). serial: the one-lane form (Woodcock tracking). */
 extern "C" hipError_t erd_launch_autofocus(const erd::DevParams* p, int u, int v, uint32_t s0, uint32_t s1, void* work,
-                                           int plain, int serial, int lut_lds, size_t lds_bytes, hipStream_t st)
+                                           int march, int serial, int lut_lds, size_t lds_bytes, hipStream_t st)
 {
     erd::FocusWork* w = (erd::FocusWork*)work;
     const dim3 grid((ER_FOCUS_RAYS + 3) / 4), block(256);
     if (serial)
         hipLaunchKernelGGL(erd::k_autofocus_serial, dim3(1), dim3(64), 0, st, p, u, v, s0, s1, &w->out);
-    else if (plain && lut_lds)
+    else if (march == ER_MARCH_PLAIN && lut_lds)
         hipLaunchKernelGGL((erd::k_autofocus<ER_MARCH_PLAIN, 1>), grid, block, lds_bytes, st, p, u, v, s0, s1, w);
-    else if (plain)
+    else if (march == ER_MARCH_PLAIN)
         hipLaunchKernelGGL((erd::k_autofocus<ER_MARCH_PLAIN, 0>), grid, block, lds_bytes, st, p, u, v, s0, s1, w);
     else if (lut_lds)
         hipLaunchKernelGGL((erd::k_autofocus<ER_MARCH_ANY, 1>), grid, block, lds_bytes, st, p, u, v, s0, s1, w);

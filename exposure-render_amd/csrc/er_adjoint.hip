@@ -491,7 +491,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADJ_SHADOW_
     const DevParams& p = *pp;
     for (int k = threadIdx.x; k < ADJ_NODES; k += blockDim.x) hist[k] = 0.0f;
     const Tables T = adj_stage(p, lds);   /* ends with a barrier */
-    const unsigned int n = counts[1];
+    const unsigned int n = counts[ER_CNT_SHADOW];
     const float DS = p.density_scale;
     const float dts = p.step_shadow * p.minstep;
     const float k2 = (DS * DS) * dts;          /* d tau / d opacity per sample */
@@ -558,7 +558,7 @@ __global__ __launch_bounds__(256) void k_adj_finish(const DevParams* __restrict_
     const DevParams& p = *pp;
     for (int k = threadIdx.x; k < ADJ_NODES; k += blockDim.x) hist[k] = 0.0f;
     __syncthreads();
-    const unsigned int n = counts[0];
+    const unsigned int n = counts[ER_CNT_SCATTER];
     for (unsigned int q = blockIdx.x * blockDim.x + threadIdx.x; q < n; q += gridDim.x * blockDim.x) {
         const EventRec ev = events[q];
         const uint32_t s1 = ev.state & 3u, s2 = (ev.state >> 2) & 3u;
@@ -668,7 +668,7 @@ __global__ __launch_bounds__(256) void k_adj_primary(const DevParams* __restrict
 
 __global__ void k_adj_reset(unsigned int* __restrict__ counts, unsigned int* __restrict__ lcount)
 {
-    if (threadIdx.x < 4) counts[threadIdx.x] = 0u;
+    if (threadIdx.x < ER_CNT_LINES) counts[ER_CNT(threadIdx.x)] = 0u;
     if (threadIdx.x == 0) *lcount = 0u;
 }
 

@@ -54,6 +54,20 @@ __device__ __forceinline__ bool clipped(const DevParams& p, f3 P)
     return false;
 }
 
+/* A pass's counters, each on a 128-byte line of its own (operations on one line go one after the
+ * other, some 10 ns each from all XCDs): the scatter queue's length, the shadow jobs' length, the
+ * shadow jobs claimed, and the tiles claimed from each of ER_TILE_QUEUES queues. */
+#define ER_CNT(i) ((i) * 32)
+#define ER_CNT_SCATTER ER_CNT(0)
+#define ER_CNT_SHADOW ER_CNT(1)
+#define ER_CNT_CLAIM ER_CNT(2)
+#define ER_CNT_TILES ER_CNT(3)
+#ifndef ER_TILE_QUEUES
+#define ER_TILE_QUEUES 8
+#endif
+#define ER_CNT_LINES (3 + ER_TILE_QUEUES)
+#define ER_CNT_WORDS ER_CNT(ER_CNT_LINES)
+
 /* dense samples per march iteration (loads in flight together) in the primary and shadow kernels */
 #define ER_BATCH_CONST_JOBS 128   /* jobs per batch graph (parameter blocks in constant memory) */
 
@@ -1678,7 +1692,7 @@ struct BatchJob {
     EventRec* events;
     ShadowJob* jobs;
     unsigned char* vis;
-    unsigned int* counts;       /* [0] scatter queue, [1] shadow jobs, [2] primary tiles claimed */
+    unsigned int* counts;       /* ER_CNT_*; the tiles are claimed from the first queue's counter */
     int tiles_x, ntiles, tile_base;
     int post_tiles_x, post_ntiles, post_base;
     int passes, no_iter0;

@@ -88,8 +88,8 @@ __global__ __launch_bounds__(256) void k_post(const DevParams* __restrict__ pp, 
                                              float4* __restrict__ running, uchar4* __restrict__ display, int no_iterations,
                                              unsigned int* __restrict__ qcount)
 {
-    /* the scatter queue of this pass has been consumed: empty it for the next pass */
-    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 4) qcount[threadIdx.x] = 0u;
+    /* the queues of this pass have been consumed: empty them for the next pass */
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < ER_CNT_LINES) qcount[ER_CNT(threadIdx.x)] = 0u;
     __shared__ float4 tile[POST_TILE + 2][POST_TILE + 2];
     post_tile(*pp, frame, running, display, no_iterations, blockIdx.x * POST_TILE, blockIdx.y * POST_TILE, tile);
 }

@@ -122,7 +122,7 @@ static __host__ __device__ constexpr NoAllocLayout noalloc_layout(size_t n)
     L.events = o;   o += align256(n * sizeof(erd::EventRec));
     L.jobs = o;     o += align256(2 * n * sizeof(erd::ShadowJob));
     L.list = o;     o += align256(n * sizeof(uint2));
-    L.counts = o;   o += align256(4 * sizeof(uint32_t));
+    L.counts = o;   o += align256(ER_CNT_WORDS * sizeof(uint32_t));
     L.lcount = o;   o += align256(sizeof(uint32_t));
     L.partials = o; o += align256((size_t)3 * ER_ADJ_BLOCKS * ER_TF_LUT_NODES * 4 * sizeof(float));
     L.out = o;      o += align256((size_t)ER_TF_LUT_NODES * 4 * sizeof(double));
@@ -310,7 +310,6 @@ struct Volume {
     er_volume_desc desc{};
     DevBuf<uint16_t> vox;
     DevBuf<uint4> cells;
-    DevBuf<unsigned int> top;       /* the largest voxel, as the device finds it */
     std::map<int, MacroGrid> grids;
     int mc_shift = 3;               /* default brick: 8 cells, coarser for very large volumes */
     uint16_t vmax = 0;
@@ -320,7 +319,7 @@ struct Volume {
     uint64_t gm_upload = 0;
     ~Volume()
     {
-        vox.release(); cells.release(); top.release();
+        vox.release(); cells.release();
         for (auto& g : grids) g.second.mm.release();
     }
 };
@@ -349,7 +348,7 @@ bool brick_fits(const er_volume_desc& d, uint16_t vmax, int shift)
  * next pass's primary and shading kernels (first stream). */
 struct PassSet {
     DevBuf<float4> frame;
-    DevBuf<uint32_t> qcount;        /* [0] scatter queue, [1] shadow jobs, [2] primary tiles */
+    DevBuf<uint32_t> qcount;        /* ER_CNT_* */
     DevBuf<char> queue, events, jobs;
     DevBuf<unsigned char> vis;
     hipEvent_t shaded = nullptr;    /* first stream: primary + shading of this set's pass done */
@@ -397,7 +396,7 @@ struct AdjWork {
             (st = partials.alloc(3 * blocks * per_block)) || (st = out.alloc(per_block)))
             return st;
         for (Set& A : set) {
-            if ((st = A.s1s.alloc(n)) || (st = A.s2s.alloc(n)) || (st = A.counts.alloc(4)) || (st = A.lcount.alloc(1)) ||
+            if ((st = A.s1s.alloc(n)) || (st = A.s2s.alloc(n)) || (st = A.counts.alloc(ER_CNT_WORDS)) || (st = A.lcount.alloc(1)) ||
                 (st = A.tvis.alloc(2 * n)) || (st = A.frame.alloc(n)) || (st = A.queue.alloc(n * rs)) ||
                 (st = A.events.alloc(n * re)) || (st = A.jobs.alloc(2 * n * rj)) || (st = A.list.alloc(n)))
                 return st;
@@ -626,7 +625,7 @@ int tracer_resize(Tracer& t, int W, int H, int id)
     erd_pass_record_sizes(&rs, &re, &rj);
     for (PassSet& S : t.set) {
         if ((st = S.frame.alloc(n)) || (st = S.queue.alloc(n * rs)) || (st = S.events.alloc(n * re)) ||
-            (st = S.jobs.alloc(2 * n * rj)) || (st = S.vis.alloc(2 * n)) || (st = S.qcount.alloc(4)))
+            (st = S.jobs.alloc(2 * n * rj)) || (st = S.vis.alloc(2 * n)) || (st = S.qcount.alloc(ER_CNT_WORDS)))
             return st;
         if (!S.shaded) HIP_TRY(hipEventCreateWithFlags(&S.shaded, hipEventDisableTiming));
         if (!S.posted) HIP_TRY(hipEventCreateWithFlags(&S.posted, hipEventDisableTiming));
@@ -635,7 +634,7 @@ int tracer_resize(Tracer& t, int W, int H, int id)
         S.pending = false;
         if (n) {
             HIP_TRY(hipMemset(S.frame.ptr, 0, n * sizeof(float4)));
-            HIP_TRY(hipMemset(S.qcount.ptr, 0, 4 * sizeof(uint32_t)));
+            HIP_TRY(hipMemset(S.qcount.ptr, 0, ER_CNT_WORDS * sizeof(uint32_t)));
         }
     }
     t.cur = 0;
@@ -699,7 +698,8 @@ MacroGrid* volume_grid(Volume& v, int shift, int& st)
     const int E = 1 << shift;
     MacroGrid& g = v.grids[shift];
     for (int i = 0; i < 3; ++i) g.mc[i] = (d.resolution[i] + E - 1) / E;
-    if ((st = g.mm.alloc((size_t)g.mc[0] * g.mc[1] * g.mc[2]))) { v.grids.erase(shift); return nullptr; }
+    /* one word more, for the largest voxel (upload_volume) */
+    if ((st = g.mm.alloc((size_t)g.mc[0] * g.mc[1] * g.mc[2] + 1))) { v.grids.erase(shift); return nullptr; }
     hipError_t e = erd_launch_macro_minmax(v.vox.ptr, g.mm.ptr, d.resolution[0], d.resolution[1], d.resolution[2], g.mc[0],
                                            g.mc[1], g.mc[2], shift, 0);
     if (e == hipSuccess) e = hipStreamSynchronize(0);
@@ -728,16 +728,17 @@ int upload_volume(Volume& v)
     if ((st = v.vox.alloc(n))) return st;
     HIP_TRY(hipMemcpy(v.vox.ptr, d.voxels, n * sizeof(uint16_t), hipMemcpyHostToDevice));
     const size_t nc = (size_t)(rx + 1) * (ry + 1) * (rz + 1);
-    if ((st = v.cells.alloc(nc)) || (st = v.top.alloc(1))) return st;
+    if ((st = v.cells.alloc(nc))) return st;
     for (auto& g : v.grids) g.second.mm.release();
     v.grids.clear();
     HIP_TRY(erd_launch_build_cells(v.vox.ptr, v.cells.ptr, rx, ry, rz, 0));
     /* the largest voxel, from the ranges of the 8-cell macrocells (the usual default grid) */
     MacroGrid* grid = volume_grid(v, 3, st);
     if (!grid) return st;
-    HIP_TRY(erd_launch_range_top(grid->mm.ptr, grid->mc[0] * grid->mc[1] * grid->mc[2], v.top.ptr, 0));
+    const int ranges = grid->mc[0] * grid->mc[1] * grid->mc[2];
+    HIP_TRY(erd_launch_range_top(grid->mm.ptr, ranges, grid->mm.ptr + ranges, 0));
     unsigned int vmax = 0;
-    HIP_TRY(hipMemcpy(&vmax, v.top.ptr, sizeof(vmax), hipMemcpyDeviceToHost));
+    HIP_TRY(hipMemcpy(&vmax, grid->mm.ptr + ranges, sizeof(vmax), hipMemcpyDeviceToHost));
     v.vmax = (uint16_t)vmax;
     /* default macrocell edge: 8 cells, coarser when the occupancy bits and the opacity table
      * would not fit their 52.5 KB of LDS */
@@ -2175,7 +2176,7 @@ static int render_batch_chunk(std::vector<std::pair<int, Tracer*>>& jobs, int fu
     for (int b = 0; b < 2; ++b) {
         if ((st = dJ[b].alloc(nj))) { G.release(); g_batch_graphs.erase(key); return st; }
         HIP_TRY(hipMemcpy(dJ[b].ptr, table[b].data(), nj * sizeof(erd::BatchJob), hipMemcpyHostToDevice));
-        for (int k = 0; k < nj; ++k) HIP_TRY(hipMemset(table[b][k].counts, 0, 4 * sizeof(uint32_t)));
+        for (int k = 0; k < nj; ++k) HIP_TRY(hipMemset(table[b][k].counts, 0, ER_CNT_WORDS * sizeof(uint32_t)));
     }
     /* the jobs' parameter blocks, in table order, for the batch kernels */
     {
@@ -2491,7 +2492,7 @@ ER_API int er_adjoint_value(int tracer_id, const uint32_t* seeds1, const uint32_
     ScopedBuf<float> lut_e, sig_e;
     ScopedBuf<float4> frame, running;
     ScopedBuf<uchar4> display;
-    if ((st = d1.alloc(n)) || (st = d2.alloc(n)) || (st = qc.alloc(4)) || (st = lut_e.alloc(ER_TF_LUT_NODES * 4)) ||
+    if ((st = d1.alloc(n)) || (st = d2.alloc(n)) || (st = qc.alloc(ER_CNT_WORDS)) || (st = lut_e.alloc(ER_TF_LUT_NODES * 4)) ||
         (st = sig_e.alloc(sig.size())) || (st = frame.alloc(n)) || (st = running.alloc(n)) || (st = display.alloc(n)))
         return st;
     HIP_TRY(hipMemcpy(d1.ptr, seeds1, n * 4, hipMemcpyHostToDevice));

@@ -106,6 +106,7 @@ struct DevParams {
     int   res[3];
     float minp[3], maxp[3], size[3], invsize[3], resf[3], spacing[3], minstep;
     const uint4* cells;
+    const uint4* cells_inside;       /* the record of lattice cell (0, 0, 0) */
     int   cstride_y, cstride_z;      /* (Rx+1), (Rx+1)(Ry+1) */
     const float* sigma_lut;          /* DensityScale * Opacity(i), i in [0, lut_max] */
     int   lut_max;
@@ -317,6 +318,26 @@ __device__ __forceinline__ CellFetch cell_fetch(const DevParams& p, const Lattic
     const unsigned idx = __umul24((unsigned)cz, (unsigned)p.cstride_z) + __umul24((unsigned)cy, (unsigned)p.cstride_y) +
                          (unsigned)cx;
     const u32x4 v = gmem((const u32x4*)p.cells)[idx];
+    f.c = make_uint4(v.x, v.y, v.z, v.w);
+    return f;
+}
+
+/* whether the sample's eight corners are voxels of the volume, none of them clamped (not for NaN) */
+__device__ __forceinline__ bool lattice_inside(const DevParams& p, const Lattice& l)
+{
+    return fminf(l.Lx, fminf(l.Ly, l.Lz)) >= 0.0f && l.Lx < p.resf[0] && l.Ly < p.resf[1] && l.Lz < p.resf[2];
+}
+
+/* cell_fetch for such a sample: no clamps, and for coordinates that are not negative the
+ * truncation is the floor and the hardware's fraction the exact difference (one instruction each) */
+__device__ __forceinline__ CellFetch cell_fetch_inside(const DevParams& p, const Lattice& l)
+{
+    CellFetch f;
+    f.dx = __builtin_amdgcn_fractf(l.Lx); f.dy = __builtin_amdgcn_fractf(l.Ly); f.dz = __builtin_amdgcn_fractf(l.Lz);
+    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+    const unsigned idx = __umul24((unsigned)l.Lz, (unsigned)p.cstride_z) + __umul24((unsigned)l.Ly, (unsigned)p.cstride_y) +
+                         (unsigned)l.Lx;
+    const u32x4 v = gmem((const u32x4*)p.cells_inside)[idx];
     f.c = make_uint4(v.x, v.y, v.z, v.w);
     return f;
 }

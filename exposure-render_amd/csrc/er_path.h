@@ -71,8 +71,15 @@ __device__ __forceinline__ bool clipped(const DevParams& p, f3 P)
 /* dense samples per march iteration (loads in flight together) in the primary and shadow kernels */
 #define ER_BATCH_CONST_JOBS 128   /* jobs per batch graph (parameter blocks in constant memory) */
 
+/* A march iteration costs about 2000 cycles besides its samples (the look at the occupancy bits,
+ * the loads' latency, the skips of the wave's other lanes) and 300 per sample, so the primary
+ * march, whose longest rays end last, takes 10 samples at once: against 6, one pass of the 256^3
+ * CT volume at 640 x 480 0.75 -> 0.68 ms, the compat loop 4.6 -> 4.0, 16 passes of the CT workload
+ * 9.4 -> 8.7. 16 samples (2 waves per SIMD) gain 4 - 6% more where few tiles are in flight and
+ * lose 4 - 9% where passes overlap; the heavy tiles' lane groups make up for the former. Shadow
+ * marches refill their lanes: 12 or 16 samples instead of 8 lose up to 8% on the large workloads. */
 #ifndef ER_BATCH_PRIMARY
-#define ER_BATCH_PRIMARY 6
+#define ER_BATCH_PRIMARY 10
 #endif
 /* a primary wave finishes its marches together (coop_march) once this few lanes still march */
 #ifndef ER_COOP_LANES
@@ -386,6 +393,62 @@ __device__ __forceinline__ void march_skip(const DevParams& p, const Tables& T, 
     if (COUNT) { if (primary) cnt.primary += n; else cnt.shadow += n; cnt.skipped += n; }
 }
 
+/* the cell loads of K samples at lattice points lk; INSIDE: all of them lattice_inside */
+template<int K, bool INSIDE>
+__device__ __forceinline__ void batch_fetch(const DevParams& p, const Lattice (&lk)[K], CellFetch (&f)[K])
+{
+#pragma unroll
+    for (int k = 0; k < K; ++k) f[k] = INSIDE ? cell_fetch_inside(p, lk[k]) : cell_fetch(p, lk[k]);
+}
+
+/* K consecutive samples of a plain march whose first, at lattice point l, lies in an occupied
+ * macrocell: all cell loads are issued before the first value is used. The optical depth after
+ * each sample never falls, so the first sample that reached the threshold, te, is where the
+ * comparisons turn (the last sample if none did), and the march ended before te exactly when te
+ * lies past the end (t grows). Returns as march_step. */
+template<int FULL, int K>
+__device__ __forceinline__ int march_batch(const DevParams& p, const Tables& T, MarchState& m, bool primary, float StepSize,
+                                           const Lattice& l, f3& Pout)
+{
+    CellFetch f[K];
+    Lattice lk[K];
+    float tk[K], sum[K], c[K];
+    tk[0] = m.MinT;
+    lk[0] = l;
+#pragma unroll
+    for (int k = 1; k < K; ++k) {
+        tk[k] = tk[k - 1] + StepSize;
+        lk[k] = to_lattice(p, add(m.O, scl(tk[k], m.D)));
+    }
+    /* lattice coordinates are monotone along the ray, so the first and the last sample bound the
+     * others; the wave takes the shorter form when all its lanes can */
+    if (__ballot(!(lattice_inside(p, lk[0]) && lattice_inside(p, lk[K - 1]))) == 0ull) batch_fetch<K, true>(p, lk, f);
+    else batch_fetch<K, false>(p, lk, f);
+    uint32_t kept = 0xffffffffu;
+    if constexpr (FULL == ER_MARCH_CLIP) {
+        const int g = group_index(p, l);
+        if (clip_possible(p, T, g) || group_index(p, lk[K - 1]) != g)
+            kept = unclipped_samples<K, 1>(p, T, m.O, m.D, m.MinT, StepSize);
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        c[k] = T.step_sigma(cell_index(f[k]), StepSize);
+        if constexpr (FULL == ER_MARCH_CLIP) c[k] = (kept >> k) & 1u ? c[k] : 0.0f;
+    }
+    sum[0] = m.Sum + c[0];
+    float te = tk[0];
+#pragma unroll
+    for (int k = 1; k < K; ++k) {
+        sum[k] = sum[k - 1] + c[k];
+        te = sum[k - 1] < m.S ? tk[k] : te;
+    }
+    m.Sum = sum[K - 1];
+    m.MinT = te + StepSize;
+    if (primary ? (te >= m.MaxT) : (te > m.MaxT)) return -1;
+    if (!(m.Sum < m.S)) { Pout = add(m.O, scl(te, m.D)); return 1; }
+    return 0;
+}
+
 /* One iteration of the march loop: up to K consecutive samples in an occupied macrocell, or
  * the skip over the rest of an empty one. Returns 1 on an event (Pout = the sample, m.MinT one
  * step beyond it, Q13), -1 when the ray leaves the segment first (the primary march ends at
@@ -418,46 +481,7 @@ __device__ __forceinline__ int march_step(const DevParams& p, const Tables& T, M
         return 0;
     }
     if constexpr (ER_MARCH_IS_PLAIN(FULL) && K > 1 && !COUNT && IsNoVisit<Visit>::value) {
-        if (mc_occupied(T, mc)) {
-            /* K consecutive samples at once, as below, without the occupancy bits. The optical
-             * depth after each sample never falls, so the first sample that reached the
-             * threshold, te, is where the comparisons turn (the last sample if none did), and
-             * the march ended before te exactly when te lies past the end (t grows). */
-            CellFetch f[K];
-            float tk[K], sum[K], c[K];
-            tk[0] = m.MinT;
-            f[0] = cell_fetch(p, l);
-            Lattice le = l;
-#pragma unroll
-            for (int k = 1; k < K; ++k) {
-                tk[k] = tk[k - 1] + StepSize;
-                le = to_lattice(p, add(m.O, scl(tk[k], m.D)));
-                f[k] = cell_fetch(p, le);
-            }
-            uint32_t kept = 0xffffffffu;
-            if constexpr (FULL == ER_MARCH_CLIP) {
-                const int g = group_index(p, l);
-                if (clip_possible(p, T, g) || group_index(p, le) != g)
-                    kept = unclipped_samples<K, 1>(p, T, m.O, m.D, m.MinT, StepSize);
-            }
-#pragma unroll
-            for (int k = 0; k < K; ++k) {
-                c[k] = T.step_sigma(cell_index(f[k]), StepSize);
-                if constexpr (FULL == ER_MARCH_CLIP) c[k] = (kept >> k) & 1u ? c[k] : 0.0f;
-            }
-            sum[0] = m.Sum + c[0];
-            float te = tk[0];
-#pragma unroll
-            for (int k = 1; k < K; ++k) {
-                sum[k] = sum[k - 1] + c[k];
-                te = sum[k - 1] < m.S ? tk[k] : te;
-            }
-            m.Sum = sum[K - 1];
-            m.MinT = te + StepSize;
-            if (primary ? (te >= m.MaxT) : (te > m.MaxT)) return -1;
-            if (!(m.Sum < m.S)) { Pout = add(m.O, scl(te, m.D)); return 1; }
-            return 0;
-        }
+        if (mc_occupied(T, mc)) return march_batch<FULL, K>(p, T, m, primary, StepSize, l, Pout);
         march_skip<COUNT>(p, T, m, primary, StepSize, cnt, l, mxi, myi, mzi);
         return 0;
     }
@@ -754,11 +778,17 @@ __device__ int coop_march(const DevParams& p, const Tables& T, MarchState& m, fl
     }
 }
 
-/* samples each lane of a G-lane group loads per round trip in group_march */
+/* samples each lane of a G-lane group loads per round trip in group_march (3 or 4 for G = 16:
+ * within 2% of 2); observed marches (the adjoint's) hold more registers per sample */
 #ifndef ER_GROUP4_BATCH
-#define ER_GROUP4_BATCH 6
+#define ER_GROUP4_BATCH 8
 #endif
-template<int G> struct GroupBatch { static constexpr int value = G >= 16 ? 2 : ER_GROUP4_BATCH; };
+#ifndef ER_GROUP4_BATCH_VISIT
+#define ER_GROUP4_BATCH_VISIT 6
+#endif
+template<int G, bool VISIT> struct GroupBatch {
+    static constexpr int value = G >= 16 ? 2 : (VISIT ? ER_GROUP4_BATCH_VISIT : ER_GROUP4_BATCH);
+};
 
 /* lane Q's v within each aligned group of G lanes (Q a constant): a DPP quad permutation for
  * G = 4, a DPP row broadcast for G = 16, which the compiler folds into the instruction that uses
@@ -809,7 +839,7 @@ __device__ __forceinline__ void group_count(const float (&c)[KB], float Sum, flo
 /* One round of a march (SampleVolume's loop, raymarching.h:55-68, primary; the same loop with
  * the shadow end test, raymarching.h:95-113, otherwise) run by an aligned group of G lanes
  * (G = 4 or 16; 64 / G rays per wave): m is the same in every lane of the group. A round either
- * skips the empty macrocell at MinT (march_step's exact skip) or reads B = GroupBatch<G> x G
+ * skips the empty macrocell at MinT (march_step's exact skip) or reads B = GroupBatch x G
  * consecutive samples, lane k of the group taking samples k, k + G, ..., k + (B/G - 1) G, so a
  * ray advances B samples per memory round trip instead of ER_BATCH_PRIMARY / ER_BATCH_SHADOW.
  * As in coop_march every position is the sequential loop's (the same float additions of
@@ -829,7 +859,7 @@ template<int FULL, int COUNT, int G, bool PRIMARY, class Visit>
 __device__ __forceinline__ int group_step_v(const DevParams& p, const Tables& T, MarchState& m, float StepSize, int lane,
                                             Cnt& cnt, f3& Pout, int& iters, Visit& vis)
 {
-    constexpr int KB = GroupBatch<G>::value;
+    constexpr int KB = GroupBatch<G, !IsNoVisit<Visit>::value>::value;
     constexpr int NS = KB * G;
     const int k = lane & (G - 1);
     const int gb = lane & ~(G - 1);

@@ -955,6 +955,7 @@ int build_params(Tracer& t)
     P.cells = vol->cells.ptr;
     P.cstride_y = vd.resolution[0] + 1;
     P.cstride_z = (vd.resolution[0] + 1) * (vd.resolution[1] + 1);
+    P.cells_inside = vol->cells.ptr + (size_t)P.cstride_z + P.cstride_y + 1;
     P.neglog = g_neglog_dev;
     const int mc_shift = (t.mc_shift > 0 && brick_fits(vd, vol->vmax, t.mc_shift)) ? t.mc_shift : vol->mc_shift;
     MacroGrid* grid = volume_grid(*vol, mc_shift, st);

@@ -459,6 +459,7 @@ struct Tracer {
      * workgroups per CU (0: the library default) */
     int mc_shift = 0, tile_shift = 3, blocks_per_cu = 0, shadow_waves_per_cu = 4, heavy_tiles = 0, rays_per_wave = 64,
         shadow_rays_per_wave = 64, heavy_rays_per_wave = 4;
+    bool tuned = false;               /* set by er_set_tune / er_autotune; until then launch_for chooses */
     /* primary tiles: each pass records its tiles' march steps and orders the next pass's tiles
      * most expensive first; the order is valid for the tile shape and count it was built for */
     DevBuf<uint32_t> tile_cost, tile_order;
@@ -540,7 +541,6 @@ Registry<ObjectObj> g_objects;
 Registry<BitmapObj> g_bitmaps;
 bool g_device_ready = false;
 int g_list_capacity = ER_LIST_CAPACITY;   /* list.cuh:27 MaxSize; er_set_list_capacity */
-int g_primary_blocks = 2048;   /* persistent primary workgroups: 7 per CU (LDS and VGPR bound) */
 int g_cus = 256;
 
 /* Device address of `scratch` per device. In host code the array's name is only a stand-in
@@ -573,10 +573,7 @@ int ensure_device()
     if (e != hipSuccess || n <= 0) return set_error(ER_ERROR, "no HIP device available (%s)", hipGetErrorString(e));
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
-    {
         g_cus = cus;
-        g_primary_blocks = cus * 7;
-    }
     /* set-up of the no-allocation entry point's scratch on this device */
     unsigned char* sp = nullptr;
     int st = scratch_for_current_device(sp);
@@ -908,6 +905,19 @@ void clip_classes(const DevParams& P, int nmc, double edge_ext, std::vector<uint
     for (auto& x : th) x.join();
 }
 
+/* The brick (macrocell) edge of a tracer's marches, as a shift: the tuned one where it fits the
+ * volume, else 4 cells where that fits (against 8, with 768 heavy tiles: one frame of the CT
+ * volume 0.61 -> 0.59 ms, 16 passes 7.3 -> 7.0 ms, 8 with objects 3.08 -> 2.91), else the volume's
+ * default. Scenes with clipping objects keep the volume's: the host classifies every macrocell.
+ * Woodcock tracking reads no macrocells. */
+int brick_shift(const Tracer& t, const Volume& v, int clip_count)
+{
+    if (t.tuned) return t.mc_shift > 0 && brick_fits(v.desc, v.vmax, t.mc_shift) ? t.mc_shift : v.mc_shift;
+    const er_render_settings& s = t.desc.settings;
+    const bool woodcock = s.estimator == ER_ESTIMATOR_FULL && s.sampler == ER_SAMPLER_WOODCOCK;
+    return clip_count == 0 && !woodcock && brick_fits(v.desc, v.vmax, 2) ? 2 : v.mc_shift;
+}
+
 /* Rebuild the tracer's DevParams (and the LUT / macrocell maxima / gm_max that depend on it). */
 int build_params(Tracer& t)
 {
@@ -957,10 +967,6 @@ int build_params(Tracer& t)
     P.cstride_z = (vd.resolution[0] + 1) * (vd.resolution[1] + 1);
     P.cells_inside = vol->cells.ptr + (size_t)P.cstride_z + P.cstride_y + 1;
     P.neglog = g_neglog_dev;
-    const int mc_shift = (t.mc_shift > 0 && brick_fits(vd, vol->vmax, t.mc_shift)) ? t.mc_shift : vol->mc_shift;
-    MacroGrid* grid = volume_grid(*vol, mc_shift, st);
-    if (!grid) return st;
-    for (int i = 0; i < 3; ++i) P.mc_dim[i] = grid->mc[i];
     P.tile_shift = t.tile_shift;
 
     /* The tracer's lights, compacted into device slots in the order of its LightIDs, and the
@@ -1094,6 +1100,11 @@ int build_params(Tracer& t)
 
     P.opacity = d.opacity; P.glossiness = d.glossiness;
     P.diffuse = d.diffuse; P.specular = d.specular; P.emission = d.emission;
+
+    const int mc_shift = brick_shift(t, *vol, P.clip_count);
+    MacroGrid* grid = volume_grid(*vol, mc_shift, st);
+    if (!grid) return st;
+    for (int i = 0; i < 3; ++i) P.mc_dim[i] = grid->mc[i];
 
     /* what the tracer's tables depend on: the volume's contents and brick size, the opacity (by
      * node table or PLF), and - through the occupancy bits - the clipping objects with the
@@ -1283,17 +1294,43 @@ bool use_bilateral(const Tracer& t)
     return t.desc.settings.estimator == ER_ESTIMATOR_FULL && t.desc.settings.bilateral;
 }
 
-int primary_blocks(const Tracer& t) { return t.blocks_per_cu > 0 ? g_cus * t.blocks_per_cu : g_primary_blocks; }
-int shadow_blocks(const Tracer& t) { return std::max(1, g_cus * t.shadow_waves_per_cu / 4); }
+/* How a tracer's passes are launched. Tuned: as er_set_tune or er_autotune set it. Otherwise by the
+ * film's size and by whether the pass runs alone (er_render_estimate) or overlaps others:
+ *  - 64 rays per wave, the rays of the 768 most expensive tiles in groups of 4 lanes (their long
+ *    marches end the kernel): against no heavy tiles, one frame of the CT volume at 640 x 480
+ *    0.68 -> 0.61 ms, the compat loop 3.96 -> 3.61, 8 passes with objects 3.50 -> 3.08, 16 CT
+ *    passes 8.1 -> 7.3 ms; 256 or 2048 tiles are within 2% of 768 or worse, groups of 16 lanes
+ *    5 - 15% slower;
+ *  - a pass alone on a film of at most two tiles per SIMD cannot fill the device with a lane per
+ *    ray: 16 rays per wave, primary and shadow, and 16 shadow waves per CU (256 x 256: 0.31 ->
+ *    0.25 ms a frame). Overlapped passes do (16 passes: 2.5 ms with heavy tiles, 2.9 so); and on
+ *    larger films the groups' redundant skips cost more than the lanes gain (8 passes at 643 x 479
+ *    3.9 ms).
+ * 4 primary workgroups per CU, what the registers let in: the 7 of before only staged their
+ * tables to find no tile left. */
+struct Launch {
+    int blocks_per_cu, shadow_waves_per_cu, heavy_tiles, rays_per_wave, shadow_rays_per_wave, heavy_rays_per_wave;
+};
+Launch launch_for(const Tracer& t, bool alone)
+{
+    if (t.tuned)
+        return {t.blocks_per_cu, t.shadow_waves_per_cu, t.heavy_tiles, t.rays_per_wave, t.shadow_rays_per_wave,
+                t.heavy_rays_per_wave};
+    if (alone && (long long)t.W * t.H <= (long long)g_cus * 4 * 2 * 64) return {4, 16, 0, 16, 16, 4};
+    return {4, 4, 768, 64, 64, 16};
+}
+int primary_blocks(const Tracer& t) { return g_cus * launch_for(t, false).blocks_per_cu; }
 
-/* One pass on the tracer's two streams (no host synchronisation). Timing events, when given:
+/* One pass on the tracer's two streams (no host synchronisation). alone: no other pass of the
+ * call follows or precedes it. Timing events, when given:
  * e[0] first stream before the primary kernel, e[1] after it, e[2] second stream after the
  * combine kernel, e[3] after post. */
-int enqueue_pass(Tracer& t, hipEvent_t* e)
+int enqueue_pass(Tracer& t, hipEvent_t* e, bool alone = false)
 {
     if (t.W == 0 || t.H == 0) return ER_OK;
     const int b = 1 - t.cur;
     PassSet& S = t.set[b];
+    const Launch L = launch_for(t, alone);
     if (!e) e = S.marks;
     const int full = t.desc.settings.estimator == ER_ESTIMATOR_FULL;
     const int shade_blocks = std::max(1, std::min((t.W * t.H + 255) / 256, 2048));
@@ -1318,11 +1355,12 @@ int enqueue_pass(Tracer& t, hipEvent_t* e)
     const bool reorder = !order_valid || (t.desc.no_iterations & ER_REORDER_MASK) == 0;
     HIP_TRY(erd_launch_trace(t.params.ptr, S.frame.ptr, t.seeds1.ptr, t.seeds2.ptr, S.queue.ptr, S.qcount.ptr,
                              S.events.ptr, S.jobs.ptr, S.vis.ptr, t.counters.ptr, t.W, t.H, full, t.march, t.counting, t.lut_lds,
-                             t.lds_bytes, shade_blocks, primary_blocks(t), shadow_blocks(t), t.tile_shift, t.stream,
+                             t.lds_bytes, shade_blocks, g_cus * L.blocks_per_cu,
+                             std::max(1, g_cus * L.shadow_waves_per_cu / 4), t.tile_shift, t.stream,
                              t.stream2, S.shaded, e ? e[1] : nullptr, order_valid ? t.tile_order.ptr : nullptr,
-                             t.tile_cost.ptr, reorder ? t.tile_order.ptr : nullptr, t.heavy_tiles,
-                             woodcock ? 1 : 64 / t.rays_per_wave, woodcock ? 1 : 64 / t.shadow_rays_per_wave,
-                             64 / t.heavy_rays_per_wave));
+                             t.tile_cost.ptr, reorder ? t.tile_order.ptr : nullptr, L.heavy_tiles,
+                             woodcock ? 1 : 64 / L.rays_per_wave, woodcock ? 1 : 64 / L.shadow_rays_per_wave,
+                             64 / L.heavy_rays_per_wave));
     t.order_shift = t.tile_shift;
     t.order_tiles = ntiles;
     if (e) HIP_TRY(hipEventRecord(e[2], t.stream2));
@@ -1412,7 +1450,7 @@ void fill_tune(const Tracer& t, er_tune& r)
     r.brick = 1 << shift;
     r.tile_w = 1 << t.tile_shift;
     r.tile_h = 64 >> t.tile_shift;
-    r.blocks_per_cu = t.blocks_per_cu > 0 ? t.blocks_per_cu : g_primary_blocks / std::max(1, g_cus);
+    r.blocks_per_cu = t.blocks_per_cu > 0 ? t.blocks_per_cu : 7;
     r.shadow_waves_per_cu = t.shadow_waves_per_cu;
     r.heavy_tiles = t.heavy_tiles;
     r.rays_per_wave = t.rays_per_wave;
@@ -1450,6 +1488,7 @@ int apply_tune(Tracer& t, const er_tune& r)
     t.rays_per_wave = r.rays_per_wave;
     t.shadow_rays_per_wave = r.shadow_rays_per_wave;
     t.heavy_rays_per_wave = r.heavy_rays_per_wave;
+    t.tuned = true;
     t.built_version = 0;
     return ER_OK;
 }
@@ -1833,7 +1872,7 @@ ER_API int er_render_estimate(int tracer_id)
     Tracer* t = get_tracer(tracer_id, st);
     if (!t) return st;
     if ((st = build_params(*t))) return st;
-    if ((st = enqueue_pass(*t, nullptr))) return st;
+    if ((st = enqueue_pass(*t, nullptr, true))) return st;
     if ((st = sync_tracer(*t))) return st;
     return ER_OK;
 }
@@ -1848,7 +1887,7 @@ ER_API int er_render_passes(int tracer_id, int passes, er_timing* timing)
     if ((st = build_params(*t))) return st;
     if (timing && (st = timing_events(*t, (size_t)passes * 4))) return st;
     hipEvent_t* ev = t->timing_events.data();
-    for (int k = 0; k < passes && !st; ++k) st = enqueue_pass(*t, timing ? &ev[4 * k] : nullptr);
+    for (int k = 0; k < passes && !st; ++k) st = enqueue_pass(*t, timing ? &ev[4 * k] : nullptr, passes == 1);
     hipError_t se = hipStreamSynchronize(t->stream);
     hipError_t se2 = hipStreamSynchronize(t->stream2);
     if (se == hipSuccess) se = se2;
@@ -1895,6 +1934,7 @@ ER_API int er_autotune(int tracer_id, int passes, int flags, er_tune* out)
     if ((st = snap.save(t))) return st;
     const int mc0 = t.mc_shift, ts0 = t.tile_shift, bpc0 = t.blocks_per_cu, sw0 = t.shadow_waves_per_cu,
               ht0 = t.heavy_tiles, rw0 = t.rays_per_wave, srw0 = t.shadow_rays_per_wave, hrw0 = t.heavy_rays_per_wave;
+    const bool tuned0 = t.tuned;
     er_tune cur{};
     fill_tune(t, cur);
     int trials = 0;
@@ -1960,6 +2000,7 @@ ER_API int er_autotune(int tracer_id, int passes, int flags, er_tune* out)
     if (st) {
         t.mc_shift = mc0; t.tile_shift = ts0; t.blocks_per_cu = bpc0; t.shadow_waves_per_cu = sw0; t.heavy_tiles = ht0;
         t.rays_per_wave = rw0; t.shadow_rays_per_wave = srw0; t.heavy_rays_per_wave = hrw0;
+        t.tuned = tuned0;
         t.built_version = 0;
     }
     const int rst = snap.restore(t);
@@ -1995,7 +2036,9 @@ ER_API int er_autotune_batch(const er_batch_item* items, int n, int rounds, er_t
     }
     std::vector<std::unique_ptr<Snapshot>> snaps;
     std::vector<er_tune> orig(n);
+    std::vector<char> tuned0(n);
     for (int k = 0; k < n; ++k) {
+        tuned0[k] = ts[k]->tuned;
         snaps.emplace_back(new Snapshot());
         if ((st = snaps[k]->save(*ts[k]))) return st;
         fill_tune(*ts[k], orig[k]);
@@ -2040,7 +2083,11 @@ ER_API int er_autotune_batch(const er_batch_item* items, int n, int rounds, er_t
         }
     }
     if (!st) st = apply_all(cur);
-    if (st) for (int k = 0; k < n; ++k) (void)apply_tune(*ts[k], orig[k]);
+    if (st)
+        for (int k = 0; k < n; ++k) {
+            (void)apply_tune(*ts[k], orig[k]);
+            ts[k]->tuned = tuned0[k];
+        }
     for (int k = 0; k < n; ++k) {
         const int rst = snaps[k]->restore(*ts[k]);
         if (!st) st = rst;

@@ -375,6 +375,11 @@ ER_API int er_set_list_capacity(int capacity);
 
 /* A tracer's launch configuration. None of it changes the image: paths are per pixel and the
  * empty-space skipping is exact, so every configuration renders the same bits. */
+/* Until a tracer is tuned (er_set_tune, er_autotune) er_get_tune reports the configuration the
+ * tuner's search starts from, and the library chooses for itself per pass: 4-cell bricks where
+ * they fit, 4 workgroups per CU, 768 heavy tiles at 16 rays per wave; a pass rendered alone
+ * (er_render_estimate) on a film of at most two tiles per SIMD takes 16 rays per wave, primary and
+ * shadow, and 16 shadow waves per CU. */
 typedef struct er_tune {
     int   brick;                  /* macrocell (brick) edge in cells: 2, 4, 8, 16, 32 */
     int   tile_w, tile_h;         /* primary tile, 64 pixels: 4x16, 8x8, 16x4 or 32x2 */

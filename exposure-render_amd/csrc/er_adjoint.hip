@@ -92,6 +92,8 @@ struct VisSum {
         last_d = sigma;
         last_e = e;
     }
+    /* without a branch: adding 0 only folds the compensation into the sum */
+    __device__ __forceinline__ void maybe(bool take, int, float sigma) { kahan_add(sd, cd, take ? sigma : 0.0f); }
     __device__ __forceinline__ void event(int i, float sigma)
     {
         last_d = sigma;
@@ -132,6 +134,7 @@ struct VisGrad {
         a0 += w * (1.0f - f);
         a1 += w * f;
     }
+    __device__ __forceinline__ void maybe(bool take, int i, float sigma) { if (take) sample(i, sigma); }
     __device__ __forceinline__ void event(int i, float sigma)
     {
         last_i = i;
@@ -177,10 +180,10 @@ __device__ __forceinline__ MarchState adj_march_from(const MarchState& m, int sr
 
 /* the rest of the marching lanes' transmittance marches (sum of sigma, VisSum<0>): on return
  * busy is false everywhere and each marching lane's vs.sd holds its whole march's sum */
-template<bool PRIMARY>
+template<int M, bool PRIMARY>
 __device__ __forceinline__ void adj_drain_sum(const DevParams& p, const Tables& T, const MarchState& m, bool busy, VisSum<0>& vs,
                                            float StepSize, int lane);
-template<bool PRIMARY>
+template<int M, bool PRIMARY>
 __device__ __forceinline__ void adj_march_sum(const DevParams& p, const Tables& T, MarchState& m, bool busy, VisSum<0>& vs,
                                               float StepSize, int lane)
 {
@@ -191,12 +194,12 @@ __device__ __forceinline__ void adj_march_sum(const DevParams& p, const Tables& 
         if (nb <= 64 / ADJ_DRAIN_G) break;
         if (busy) {
             f3 P;
-            if (march_step<1, 0, ER_BATCH_SHADOW_ADJ, VisSum<0>>(p, T, m, PRIMARY, StepSize, cnt, vs, P) != 0) busy = false;
+            if (march_step<M, 0, ER_BATCH_SHADOW_ADJ, VisSum<0>>(p, T, m, PRIMARY, StepSize, cnt, vs, P) != 0) busy = false;
         }
     }
-    adj_drain_sum<PRIMARY>(p, T, m, busy, vs, StepSize, lane);
+    adj_drain_sum<M, PRIMARY>(p, T, m, busy, vs, StepSize, lane);
 }
-template<bool PRIMARY>
+template<int M, bool PRIMARY>
 __device__ __forceinline__ void adj_drain_sum(const DevParams& p, const Tables& T, const MarchState& m, bool busy, VisSum<0>& vs,
                                            float StepSize, int lane)
 {
@@ -217,7 +220,7 @@ __device__ __forceinline__ void adj_drain_sum(const DevParams& p, const Tables& 
         if (gb) {
             f3 P;
             int iters = 0;
-            if (group_step_v<1, 0, G, PRIMARY, VisSum<0>>(p, T, g, StepSize, lane, cnt, P, iters, gv) != 0) gb = false;
+            if (group_step_v<M, 0, G, PRIMARY, VisSum<0>>(p, T, g, StepSize, lane, cnt, P, iters, gv) != 0) gb = false;
         }
     }
     /* the group's sum: the lanes' compensated sums added across the group */
@@ -232,10 +235,10 @@ __device__ __forceinline__ void adj_drain_sum(const DevParams& p, const Tables& 
 /* the rest of the marching lanes' gradient marches (VisGrad into the LDS histogram): on return
  * each marching lane's vol is whether its march ended on an event, and vg.last_i / last_sigma
  * are the event sample's */
-template<bool PRIMARY>
+template<int M, bool PRIMARY>
 __device__ __forceinline__ void adj_drain_grad(const DevParams& p, const Tables& T, const MarchState& m, bool busy, bool& vol,
                                             VisGrad& vg, float StepSize, int lane);
-template<bool PRIMARY, int K>
+template<int M, bool PRIMARY, int K>
 __device__ __forceinline__ void adj_march_grad(const DevParams& p, const Tables& T, MarchState& m, bool busy, bool& vol,
                                                VisGrad& vg, float StepSize, int lane)
 {
@@ -246,13 +249,13 @@ __device__ __forceinline__ void adj_march_grad(const DevParams& p, const Tables&
         if (nb <= 64 / ADJ_DRAIN_G) break;
         if (busy) {
             f3 P;
-            const int st = march_step<1, 0, K, VisGrad>(p, T, m, PRIMARY, StepSize, cnt, vg, P);
+            const int st = march_step<M, 0, K, VisGrad>(p, T, m, PRIMARY, StepSize, cnt, vg, P);
             if (st != 0) { busy = false; vol = st > 0; }
         }
     }
-    adj_drain_grad<PRIMARY>(p, T, m, busy, vol, vg, StepSize, lane);
+    adj_drain_grad<M, PRIMARY>(p, T, m, busy, vol, vg, StepSize, lane);
 }
-template<bool PRIMARY>
+template<int M, bool PRIMARY>
 __device__ __forceinline__ void adj_drain_grad(const DevParams& p, const Tables& T, const MarchState& m, bool busy, bool& vol,
                                             VisGrad& vg, float StepSize, int lane)
 {
@@ -273,7 +276,7 @@ __device__ __forceinline__ void adj_drain_grad(const DevParams& p, const Tables&
         if (gb) {
             f3 P;
             int iters = 0;
-            const int st = group_step_v<1, 0, G, PRIMARY, VisGrad>(p, T, g, StepSize, lane, cnt, P, iters, gv);
+            const int st = group_step_v<M, 0, G, PRIMARY, VisGrad>(p, T, g, StepSize, lane, cnt, P, iters, gv);
             if (st != 0) { gst = st; gb = false; }
         }
     }
@@ -481,6 +484,8 @@ __device__ __forceinline__ void adj_flush_hist(const float* hist, float* __restr
 #ifndef ADJ_SHADOW_WAVES_PER_EU
 #define ADJ_SHADOW_WAVES_PER_EU 3
 #endif
+/* M: the marches' form, ER_MARCH_PLAIN or ER_MARCH_ANY */
+template<int M>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADJ_SHADOW_WAVES_PER_EU))) void k_adj_shadow(const DevParams* __restrict__ pp, const unsigned int* __restrict__ counts,
                                                    const ShadowJob* __restrict__ jobq, const EventRec* __restrict__ events,
                                                    const float4* __restrict__ adj, float* __restrict__ tvis,
@@ -521,7 +526,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADJ_SHADOW_
             inbox = intersect_box(r, ld3(p.minp), ld3(p.maxp), nearT, farT);
             if (inbox && march_begin(p, r, nearT, farT, dts, rng, cap, m)) busy = m.Sum < m.S;
         }
-        adj_march_sum<false>(p, T, m, busy, vs, dts, lane);
+        adj_march_sum<M, false>(p, T, m, busy, vs, dts, lane);
         float g = 0.0f;
         if (has) {
             const float Tr = erm::expf_(-((DS * dts) * vs.sd));
@@ -543,7 +548,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADJ_SHADOW_
             rr.s1 = job.s1;
             if (march_begin(p, r, nearT, farT, dts, rr, cap, m)) busy2 = m.Sum < m.S;
         }
-        adj_march_grad<false, ER_BATCH_SHADOW_ADJ>(p, T, m, busy2, vol, vg, dts, lane);
+        adj_march_grad<M, false, ER_BATCH_SHADOW_ADJ>(p, T, m, busy2, vol, vg, dts, lane);
         vg.flush();
     }
     adj_flush_hist(hist, partials);
@@ -588,13 +593,15 @@ __global__ __launch_bounds__(256) void k_adj_finish(const DevParams* __restrict_
     adj_flush_hist(hist, partials);
 }
 
-/* pixels whose smooth value has a non-zero adjoint, with g_total, into a list */
+/* pixels whose smooth value has a non-zero adjoint, with g_total, into a list (one atomic per
+ * workgroup: one per wave took 43 us for 512 x 512 pixels) */
 __global__ __launch_bounds__(256) void k_adj_list(const float4* __restrict__ frame, const float4* __restrict__ adj, int n,
                                                  uint2* __restrict__ list, unsigned int* __restrict__ count)
 {
-    const int lane = threadIdx.x & 63;
-    for (int base = blockIdx.x * blockDim.x + (threadIdx.x & ~63); base < n; base += gridDim.x * blockDim.x) {
-        const int i = base + lane;
+    __shared__ unsigned int part[4], first;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x) {
+        const int i = base + (int)threadIdx.x;
         float g = 0.0f;
         if (i < n) {
             const float4 v = frame[i], A = adj[i];
@@ -602,15 +609,21 @@ __global__ __launch_bounds__(256) void k_adj_list(const float4* __restrict__ fra
         }
         const bool has = g != 0.0f;
         const unsigned long long m = __ballot(has);
-        if (!m) continue;
-        const int leader = __ffsll((long long)m) - 1;
-        unsigned int slot = 0;
-        if (lane == leader) slot = atomicAdd(count, (unsigned int)__popcll(m));
-        slot = __shfl(slot, leader);
+        if (lane == 0) part[wave] = (unsigned int)__popcll(m);
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const unsigned int total = part[0] + part[1] + part[2] + part[3];
+            first = total ? atomicAdd(count, total) : 0u;
+        }
+        __syncthreads();
+        unsigned int slot = first;
+        for (int w = 0; w < wave; ++w) slot += part[w];
         if (has) list[slot + (unsigned int)__popcll(m & ((1ull << lane) - 1ull))] = make_uint2((unsigned int)i, __float_as_uint(g));
+        __syncthreads();
     }
 }
 
+template<int M>
 __global__ __launch_bounds__(256) void k_adj_primary(const DevParams* __restrict__ pp, const uint2* __restrict__ list,
                                                     const unsigned int* __restrict__ count,
                                                     const uint32_t* __restrict__ seeds1, const uint32_t* __restrict__ seeds2,
@@ -654,7 +667,7 @@ __global__ __launch_bounds__(256) void k_adj_primary(const DevParams* __restrict
                 else busy = true;
             }
         }
-        adj_march_grad<true, ER_BATCH_PRIMARY_ADJ>(p, T, m, busy, vol, vg, StepSize, lane);
+        adj_march_grad<M, true, ER_BATCH_PRIMARY_ADJ>(p, T, m, busy, vol, vg, StepSize, lane);
         vg.flush();
         if (has && vol && vg.last_sigma > 0.0f) {
             const float tau = kdt * vg.last_sigma;
@@ -746,17 +759,22 @@ extern "C" hipError_t erd_launch_adj_wavefront(const erd::DevParams* p, unsigned
                                                const void* events, const void* queue, const float4* adj, float* tvis,
                                                float4* frame, uint2* list, unsigned int* lcount, const uint32_t* s1start,
                                                const uint32_t* s2start, float* partials, int blocks, int n,
-                                               size_t lds_bytes, hipStream_t st)
+                                               int march, size_t lds_bytes, hipStream_t st)
 {
     const size_t per = (size_t)blocks * ADJ_NODES;
-    hipLaunchKernelGGL(erd::k_adj_shadow, dim3(blocks), dim3(256), lds_bytes, st, p, (const unsigned int*)counts,
-                       (const erd::ShadowJob*)jobs, (const erd::EventRec*)events, adj, tvis, partials);
+#define ER_ADJ_SHADOW(M) hipLaunchKernelGGL(erd::k_adj_shadow<M>, dim3(blocks), dim3(256), lds_bytes, st, p, \
+                                            (const unsigned int*)counts, (const erd::ShadowJob*)jobs, \
+                                            (const erd::EventRec*)events, adj, tvis, partials)
+    if (march == ER_MARCH_PLAIN) ER_ADJ_SHADOW(ER_MARCH_PLAIN); else ER_ADJ_SHADOW(ER_MARCH_ANY);
+#undef ER_ADJ_SHADOW
     hipLaunchKernelGGL(erd::k_adj_finish, dim3(blocks), dim3(256), 0, st, p, (const unsigned int*)counts,
                        (const erd::EventRec*)events, (const erd::ScatterRec*)queue, (const float*)tvis, adj, frame,
                        partials + per);
     hipLaunchKernelGGL(erd::k_adj_list, dim3(blocks), dim3(256), 0, st, (const float4*)frame, adj, n, list, lcount);
-    hipLaunchKernelGGL(erd::k_adj_primary, dim3(blocks), dim3(256), lds_bytes, st, p, (const uint2*)list,
-                       (const unsigned int*)lcount, s1start, s2start, partials + 2 * per);
+#define ER_ADJ_PRIMARY(M) hipLaunchKernelGGL(erd::k_adj_primary<M>, dim3(blocks), dim3(256), lds_bytes, st, p, (const uint2*)list, \
+                                             (const unsigned int*)lcount, s1start, s2start, partials + 2 * per)
+    if (march == ER_MARCH_PLAIN) ER_ADJ_PRIMARY(ER_MARCH_PLAIN); else ER_ADJ_PRIMARY(ER_MARCH_ANY);
+#undef ER_ADJ_PRIMARY
     return hipGetLastError();
 }
 

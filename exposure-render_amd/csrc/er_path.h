@@ -285,7 +285,9 @@ __device__ __forceinline__ uint32_t skip_additions(float& t, float b, float t_li
 struct NoVisit {
     __device__ __forceinline__ void begin(float) {}
     __device__ __forceinline__ void sample(int, float) {}
-    /* group marches (group_step_v): the event sample, reported to every lane of the group */
+    /* sample() if the condition holds */
+    __device__ __forceinline__ void maybe(bool, int, float) {}
+    /* the event sample (plain batches, and every lane of the group in group marches) */
     __device__ __forceinline__ void event(int, float) {}
 };
 template<class V> struct IsNoVisit { static constexpr bool value = false; };
@@ -449,6 +451,62 @@ __device__ __forceinline__ int march_batch(const DevParams& p, const Tables& T, 
     return 0;
 }
 
+/* march_batch for a march with an observer: the samples up to the event or the end of the segment
+ * are reported in order, those that add nothing excepted (observers ignore a sigma of 0), and
+ * the event's sample again as such. T.lut holds sigma itself. */
+template<int K, class Visit>
+__device__ __forceinline__ int march_batch_visit(const DevParams& p, const Tables& T, MarchState& m, bool primary, float StepSize,
+                                                 const Lattice& l, Visit& vis, f3& Pout)
+{
+    CellFetch f[K];
+    Lattice lk[K];
+    float tk[K], sig[K];
+    int iv[K];
+    tk[0] = m.MinT;
+    lk[0] = l;
+#pragma unroll
+    for (int k = 1; k < K; ++k) {
+        tk[k] = tk[k - 1] + StepSize;
+        lk[k] = to_lattice(p, add(m.O, scl(tk[k], m.D)));
+    }
+    if (__ballot(!(lattice_inside(p, lk[0]) && lattice_inside(p, lk[K - 1]))) == 0ull) batch_fetch<K, true>(p, lk, f);
+    else batch_fetch<K, false>(p, lk, f);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        iv[k] = (int)cell_index(f[k]);
+        sig[k] = T.lut(iv[k]);
+    }
+    /* the sums never fall: last = the first sample that reached the threshold, or the batch's
+     * last; then the samples past the segment's end are dropped */
+    float sum = m.Sum, te = tk[0];
+    int last = 0;
+    bool open = true;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        if (k > 0) { te = open ? tk[k] : te; last = open ? k : last; }
+        sum += sig[k] * StepSize;
+        open = sum < m.S;
+    }
+    const bool ended = primary ? (te >= m.MaxT) : (te > m.MaxT);
+    int li = iv[0];
+    float ls = sig[0];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const bool in = k == 0 || (k <= last && (primary ? (tk[k] < m.MaxT) : (tk[k] <= m.MaxT)));
+        vis.maybe(in && sig[k] > 0.0f, iv[k], sig[k]);
+        if (k > 0 && k == last) { li = iv[k]; ls = sig[k]; }
+    }
+    m.Sum = sum;
+    m.MinT = te + StepSize;
+    if (ended) return -1;
+    if (!open) {
+        vis.event(li, ls);
+        Pout = add(m.O, scl(te, m.D));
+        return 1;
+    }
+    return 0;
+}
+
 /* One iteration of the march loop: up to K consecutive samples in an occupied macrocell, or
  * the skip over the rest of an empty one. Returns 1 on an event (Pout = the sample, m.MinT one
  * step beyond it, Q13), -1 when the ray leaves the segment first (the primary march ends at
@@ -482,6 +540,11 @@ __device__ __forceinline__ int march_step(const DevParams& p, const Tables& T, M
     }
     if constexpr (ER_MARCH_IS_PLAIN(FULL) && K > 1 && !COUNT && IsNoVisit<Visit>::value) {
         if (mc_occupied(T, mc)) return march_batch<FULL, K>(p, T, m, primary, StepSize, l, Pout);
+        march_skip<COUNT>(p, T, m, primary, StepSize, cnt, l, mxi, myi, mzi);
+        return 0;
+    }
+    if constexpr (FULL == ER_MARCH_PLAIN && K > 1 && !COUNT && !IsNoVisit<Visit>::value) {
+        if (mc_occupied(T, mc)) return march_batch_visit<K, Visit>(p, T, m, primary, StepSize, l, vis, Pout);
         march_skip<COUNT>(p, T, m, primary, StepSize, cnt, l, mxi, myi, mzi);
         return 0;
     }
@@ -934,6 +997,52 @@ __device__ __forceinline__ int group_step_v(const DevParams& p, const Tables& T,
         m.MinT = te + StepSize;
         if (PRIMARY ? (te >= m.MaxT) : (te > m.MaxT)) return -1;
         if (hit) Pout = add(m.O, scl(te, m.D));
+        return hit ? 1 : 0;
+    } else if constexpr (FULL == ER_MARCH_PLAIN && !COUNT) {
+        /* the same with an observer: every lane passes its own samples up to the event or the end */
+#pragma unroll
+        for (int j = 0; j < KB; ++j) {
+            if (j > 0) {
+#pragma unroll
+                for (int s = 0; s < G; ++s) t += StepSize;
+            }
+            tk[j] = t;
+            f[j] = cell_fetch(p, to_lattice(p, add(m.O, scl(t, m.D))));
+        }
+        int ivs[KB];
+        float sg[KB];
+#pragma unroll
+        for (int j = 0; j < KB; ++j) {
+            ivs[j] = (int)cell_index(f[j]);
+            sg[j] = T.lut(ivs[j]);
+            c[j] = sg[j] * StepSize;
+        }
+        float Sum = m.Sum;
+        group_sum<G, KB>(c, Sum);
+        const bool hit = !(Sum < m.S);
+        int last = NS - 1;
+        if (hit) {
+            last = 0;
+            group_count<G, KB>(c, m.Sum, m.S, last);
+        }
+        const int je = last / G;
+        float te = tk[0];
+        int ei = ivs[0];
+        float es = sg[0];
+#pragma unroll
+        for (int j = 1; j < KB; ++j) if (j == je) { te = tk[j]; ei = ivs[j]; es = sg[j]; }
+        te = __shfl(te, last - je * G, G);
+#pragma unroll
+        for (int j = 0; j < KB; ++j)
+            vis.maybe(j * G + k <= last && (PRIMARY ? (tk[j] < m.MaxT) : (tk[j] <= m.MaxT)) && sg[j] > 0.0f, ivs[j], sg[j]);
+        iters = (last + ER_BATCH_PRIMARY) / ER_BATCH_PRIMARY;
+        m.Sum = Sum;
+        m.MinT = te + StepSize;
+        if (PRIMARY ? (te >= m.MaxT) : (te > m.MaxT)) return -1;
+        if (hit) {
+            vis.event(__shfl(ei, last - je * G, G), __shfl(es, last - je * G, G));
+            Pout = add(m.O, scl(te, m.D));
+        }
         return hit ? 1 : 0;
     } else {
     bool ins[KB], live[KB];

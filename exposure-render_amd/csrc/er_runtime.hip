@@ -75,7 +75,7 @@ extern "C" hipError_t erd_launch_primary_shade(const DevParams* p, float4* frame
 extern "C" hipError_t erd_launch_adj_wavefront(const DevParams* p, unsigned int* counts, const void* jobs, const void* events,
                                                const void* queue, const float4* adj, float* tvis, float4* frame, uint2* list,
                                                unsigned int* lcount, const uint32_t* s1start, const uint32_t* s2start,
-                                               float* partials, int blocks, int n, size_t lds_bytes, hipStream_t st);
+                                               float* partials, int blocks, int n, int march, size_t lds_bytes, hipStream_t st);
 extern "C" hipError_t erd_launch_adj_reset(unsigned int* counts, unsigned int* lcount, hipStream_t st);
 extern "C" size_t erd_autofocus_work_size(void);
 extern "C" size_t erd_autofocus_out_offset(void);
@@ -370,36 +370,45 @@ struct PassSet {
     }
 };
 
-/* The work buffers of er_adjoint_lut, kept with the tracer: two sets of one pass's queues, so
- * that pass k + 1's primary and shading kernels (first stream) overlap pass k's adjoint kernels
- * (second stream), as the forward passes do. Made by the first call and resized with the film. */
+/* The work buffers of er_adjoint_lut, kept with the tracer: ER_ADJ_SETS sets of one pass's queues,
+ * histograms and gradient sum. Pass k + 1's primary and shading kernels (the tracer's first
+ * stream) need only pass k's seeds, and the adjoint kernels of different passes nothing of each
+ * other, so each set's run on a stream of its own: a pass's marches end with a few long ones,
+ * which leave the device to the next passes'. 16 + 16 passes of a 128^3 volume at 512 x 512: 43 ms
+ * with one stream, two sets and the general marches, 29 - 31 ms so (three streams and the first are the device's four
+ * hardware queues). Made by the first call and resized with the film. */
+#ifndef ER_ADJ_SETS
+#define ER_ADJ_SETS 3
+#endif
 struct AdjWork {
     struct Set {
         DevBuf<uint32_t> s1s, s2s, counts, lcount;
-        DevBuf<float> tvis;
+        DevBuf<float> tvis, partials;
+        DevBuf<double> out;
         DevBuf<float4> frame;
         DevBuf<char> queue, events, jobs;
         DevBuf<uint2> list;
+        hipStream_t own = nullptr;   /* the adjoint kernels' stream; null: the tracer's second */
         hipEvent_t shaded = nullptr, done = nullptr;
         bool pending = false;
-    } set[2];
+    } set[ER_ADJ_SETS];
     DevBuf<uint32_t> d1, d2;
-    DevBuf<float> dldr, partials;
+    DevBuf<float> dldr;
     DevBuf<float4> adj;
-    DevBuf<double> out;
     int fit(size_t n, size_t blocks, size_t per_block)
     {
         int st;
         size_t rs = 0, re = 0, rj = 0;
         erd_pass_record_sizes(&rs, &re, &rj);
-        if ((st = d1.alloc(n)) || (st = d2.alloc(n)) || (st = dldr.alloc(n * 3)) || (st = adj.alloc(n)) ||
-            (st = partials.alloc(3 * blocks * per_block)) || (st = out.alloc(per_block)))
-            return st;
+        if ((st = d1.alloc(n)) || (st = d2.alloc(n)) || (st = dldr.alloc(n * 3)) || (st = adj.alloc(n))) return st;
         for (Set& A : set) {
-            if ((st = A.s1s.alloc(n)) || (st = A.s2s.alloc(n)) || (st = A.counts.alloc(ER_CNT_WORDS)) || (st = A.lcount.alloc(1)) ||
-                (st = A.tvis.alloc(2 * n)) || (st = A.frame.alloc(n)) || (st = A.queue.alloc(n * rs)) ||
+            if ((st = A.s1s.alloc(n)) || (st = A.s2s.alloc(n)) || (st = A.counts.alloc(ER_CNT_WORDS)) ||
+                (st = A.lcount.alloc(1)) || (st = A.tvis.alloc(2 * n)) || (st = A.partials.alloc(3 * blocks * per_block)) ||
+                (st = A.out.alloc(per_block)) || (st = A.frame.alloc(n)) || (st = A.queue.alloc(n * rs)) ||
                 (st = A.events.alloc(n * re)) || (st = A.jobs.alloc(2 * n * rj)) || (st = A.list.alloc(n)))
                 return st;
+            if (&A != &set[0] && !A.own) HIP_TRY(hipStreamCreateWithFlags(&A.own, hipStreamNonBlocking));
+            if (A.own) HIP_TRY(hipStreamSynchronize(A.own));   /* idle, unless a call before this one failed */
             if (!A.shaded) HIP_TRY(hipEventCreateWithFlags(&A.shaded, hipEventDisableTiming));
             if (!A.done) HIP_TRY(hipEventCreateWithFlags(&A.done, hipEventDisableTiming));
             A.pending = false;
@@ -410,12 +419,15 @@ struct AdjWork {
     {
         for (Set& A : set) {
             A.s1s.release(); A.s2s.release(); A.counts.release(); A.lcount.release(); A.tvis.release(); A.frame.release();
+            A.partials.release(); A.out.release();
+            if (A.own) (void)hipStreamDestroy(A.own);
+            A.own = nullptr;
             A.queue.release(); A.events.release(); A.jobs.release(); A.list.release();
             if (A.shaded) (void)hipEventDestroy(A.shaded);
             if (A.done) (void)hipEventDestroy(A.done);
             A.shaded = A.done = nullptr;
         }
-        d1.release(); d2.release(); dldr.release(); partials.release(); adj.release(); out.release();
+        d1.release(); d2.release(); dldr.release(); adj.release();
     }
 };
 
@@ -2404,21 +2416,25 @@ ER_API int er_adjoint_lut(int tracer_id, const uint32_t* seeds1, const uint32_t*
     const size_t per_block = erd_adj_partials_per_block();
     AdjWork& W = t->adjoint;
     if ((st = W.fit(n, blocks, per_block))) return st;
-    hipStream_t s = t->stream, s2 = t->stream2;
+    hipStream_t s = t->stream;
     HIP_TRY(hipMemcpyAsync(W.d1.ptr, seeds1, n * 4, hipMemcpyHostToDevice, s));
     HIP_TRY(hipMemcpyAsync(W.d2.ptr, seeds2, n * 4, hipMemcpyHostToDevice, s));
     HIP_TRY(hipMemcpyAsync(W.dldr.ptr, dL_drunning_xyz, n * 12, hipMemcpyHostToDevice, s));
-    HIP_TRY(erd_launch_zero_words((uint32_t*)W.out.ptr, per_block * sizeof(double) / 4, s));
-    for (AdjWork::Set& A : W.set) HIP_TRY(erd_launch_adj_reset(A.counts.ptr, A.lcount.ptr, s));
-    const int shade_blocks = std::max(1, std::min((int)((n + 255) / 256), 2048));
-    float cur_w = -1.0f;
+    for (AdjWork::Set& A : W.set) {
+        HIP_TRY(erd_launch_zero_words((uint32_t*)A.out.ptr, per_block * sizeof(double) / 4, s));
+        HIP_TRY(erd_launch_adj_reset(A.counts.ptr, A.lcount.ptr, s));
+    }
     /* the running estimate after N passes is the mean of the filtered frames of passes 2..N
      * (the first pass is discarded, Q1), or the first frame when N == 1 */
+    const float weight = passes == 1 ? 1.0f : 1.0f / (float)(passes - 1);
+    HIP_TRY(erd_launch_adj_filter_t(W.dldr.ptr, W.adj.ptr, t->W, t->H, weight, s));
+    const int shade_blocks = std::max(1, std::min((int)((n + 255) / 256), 2048));
     for (int k = 1; k <= passes; ++k) {
-        AdjWork::Set& A = W.set[k & 1];
-        const float w = passes == 1 ? 1.0f : (k >= 2 ? 1.0f / (float)(passes - 1) : 0.0f);
+        AdjWork::Set& A = W.set[k % ER_ADJ_SETS];
+        hipStream_t sa = A.own ? A.own : t->stream2;
+        const bool counts = passes == 1 || k >= 2;
         if (A.pending) HIP_TRY(hipStreamWaitEvent(s, A.done, 0));
-        if (w != 0.0f) {
+        if (counts) {
             HIP_TRY(hipMemcpyAsync(A.s1s.ptr, W.d1.ptr, n * 4, hipMemcpyDeviceToDevice, s));
             HIP_TRY(hipMemcpyAsync(A.s2s.ptr, W.d2.ptr, n * 4, hipMemcpyDeviceToDevice, s));
         }
@@ -2427,23 +2443,31 @@ ER_API int er_adjoint_lut(int tracer_id, const uint32_t* seeds1, const uint32_t*
                                          A.jobs.ptr, t->W, t->H, t->march, t->lut_lds, t->lds_bytes, shade_blocks,
                                          primary_blocks(*t), t->tile_shift, s));
         HIP_TRY(hipEventRecord(A.shaded, s));
-        HIP_TRY(hipStreamWaitEvent(s2, A.shaded, 0));
-        if (w != 0.0f) {
-            if (w != cur_w) {
-                HIP_TRY(erd_launch_adj_filter_t(W.dldr.ptr, W.adj.ptr, t->W, t->H, w, s2));
-                cur_w = w;
-            }
+        HIP_TRY(hipStreamWaitEvent(sa, A.shaded, 0));
+        if (counts) {
             HIP_TRY(erd_launch_adj_wavefront(t->params.ptr, A.counts.ptr, A.jobs.ptr, A.events.ptr, A.queue.ptr, W.adj.ptr,
                                              A.tvis.ptr, A.frame.ptr, A.list.ptr, A.lcount.ptr, A.s1s.ptr, A.s2s.ptr,
-                                             W.partials.ptr, blocks, (int)n, t->lds_bytes, s2));
-            HIP_TRY(erd_launch_adj_reduce(W.partials.ptr, 3 * blocks, W.out.ptr, s2));
+                                             A.partials.ptr, blocks, (int)n, t->march, t->lds_bytes, sa));
+            HIP_TRY(erd_launch_adj_reduce(A.partials.ptr, 3 * blocks, A.out.ptr, sa));
         }
-        HIP_TRY(erd_launch_adj_reset(A.counts.ptr, A.lcount.ptr, s2));
-        HIP_TRY(hipEventRecord(A.done, s2));
+        HIP_TRY(erd_launch_adj_reset(A.counts.ptr, A.lcount.ptr, sa));
+        HIP_TRY(hipEventRecord(A.done, sa));
         A.pending = true;
     }
-    HIP_TRY(hipMemcpyAsync(dL_dlut, W.out.ptr, per_block * sizeof(double), hipMemcpyDeviceToHost, s2));
-    HIP_TRY(hipStreamSynchronize(s2));
+    /* the sets' sums, added in a fixed order */
+    std::vector<double> part(per_block * ER_ADJ_SETS);
+    for (int j = 0; j < ER_ADJ_SETS; ++j) {
+        AdjWork::Set& A = W.set[j];
+        hipStream_t sa = A.own ? A.own : t->stream2;
+        if (!A.pending) HIP_TRY(hipStreamSynchronize(s));   /* no pass on this set: its sum was cleared on the first stream */
+        HIP_TRY(hipMemcpyAsync(part.data() + j * per_block, A.out.ptr, per_block * sizeof(double), hipMemcpyDeviceToHost, sa));
+        HIP_TRY(hipStreamSynchronize(sa));
+    }
+    for (size_t i = 0; i < per_block; ++i) {
+        double v = 0.0;
+        for (int j = 0; j < ER_ADJ_SETS; ++j) v += part[j * per_block + i];
+        dL_dlut[i] = v;
+    }
     if ((st = sync_tracer(*t))) return st;
     return ER_OK;
 }
@@ -2512,7 +2536,7 @@ ER_API int er_adjoint_lut_noalloc(int tracer_id, const uint32_t* seeds1, const u
                 cur_w = w;
             }
             HIP_TRY(erd_launch_adj_wavefront(t->params.ptr, counts, jobs, events, queue, adj, tvis, frame, list, lcount, s1s,
-                                             s2s, partials, blocks, (int)n, t->lds_bytes, s));
+                                             s2s, partials, blocks, (int)n, t->march, t->lds_bytes, s));
             HIP_TRY(erd_launch_adj_reduce(partials, 3 * blocks, out, s));
         }
         HIP_TRY(erd_launch_adj_reset(counts, lcount, s));

@@ -113,9 +113,8 @@ __device__ __forceinline__ bool clipped(const DevParams& p, f3 P)
  * code), while the loads of all of them are in flight. 512 x 512 x 460 with a clipping box at
  * 1080p, 16 passes: 27.5 -> 22.5 ms (33.7 -> 29.3 for another phantom). */
 #define ER_MARCH_CLIP 3
-/* ER_MARCH_WOODCOCK: Woodcock tracking with no negative opacity, nothing else compiled in (82
- * VGPRs in the primary kernel instead of 162, 61 in the shadow kernel; 0 - 3% faster: its walks
- * are bound by their serial chains) */
+/* ER_MARCH_WOODCOCK: Woodcock tracking with no negative opacity, nothing else compiled in; its
+ * walks go in rounds (wc_round) and the last of a wave in groups of lanes (wc_drain) */
 #define ER_MARCH_WOODCOCK 4
 /* no occupancy test per sample, table of products with the step size */
 #define ER_MARCH_IS_PLAIN(M) ((M) == ER_MARCH_PLAIN || (M) == ER_MARCH_CLIP)
@@ -738,6 +737,246 @@ __device__ __forceinline__ int wc_step(const DevParams& p, const Tables& T, WcWa
     }
     w.t = t_exit;
     return 0;
+}
+
+/* A round of a walk (ER_MARCH_WOODCOCK, nothing counted): up to ER_WC_ROUND_STEPS majorant segments or
+ * ER_WC_ROUND tentative collisions, whichever comes first, walked as if every collision were
+ * rejected; then the cells of all the collisions are loaded together and the first real one, if
+ * any, is where the walk ended. Draws do not depend on the volume's values, so the sequence is
+ * that of woodcock_track; the state after an accepted collision is drawn again from the round's
+ * start (the next optical depth is drawn already). w.tau must hold the first optical depth
+ * (wc_first). One cell load at a time and every lane waiting for the slowest one's next collision
+ * took 9.9 / 13.7 ms for 4 passes of the CT volume (two phantoms), four 9.1 / 10.3; longer rounds
+ * (12 steps: 10.0 / 11.9) wait again, more collisions (6 in 6 steps) are within 2%. Returns as
+ * wc_step. */
+#define ER_WC_ROUND 4
+#define ER_WC_ROUND_STEPS 4
+__device__ __forceinline__ void wc_first(WcWalk& w)
+{
+    w.tau = -erm::logf_(w.rng.u());
+    w.need_tau = false;
+}
+
+__device__ __forceinline__ int wc_round(const DevParams& p, const Tables& T, WcWalk& w, bool primary)
+{
+    constexpr int B = ER_WC_ROUND;
+    const int dx = p.wc_dim[0], dy = p.wc_dim[1], dz = p.wc_dim[2];
+    const float big = 3.402823466e+38f;
+    const Rng start = w.rng;
+    /* the latest collision first: distance, and what sigma is compared with */
+    float tc[B], th[B];
+#pragma unroll
+    for (int k = 0; k < B; ++k) { tc[k] = w.t; th[k] = big; }
+    int n = 0;
+    bool ended = false;
+#pragma unroll 1
+    for (int s = 0; s < ER_WC_ROUND_STEPS; ++s) {
+        const bool go = n < B && !ended;
+        if (__ballot(go) == 0ull) break;
+        if (go) {
+            if (++w.segments > ER_WC_MAX_SEGMENTS || !(w.t < w.MaxT)) {
+                ended = true;
+            } else {
+                const Lattice l = to_lattice(p, add(w.O, scl(w.t, w.D)));
+                const int mx = mc_axis(l.Lx, ER_WC_SHIFT, dx), my = mc_axis(l.Ly, ER_WC_SHIFT, dy), mz = mc_axis(l.Lz, ER_WC_SHIFT, dz);
+                const float mu = p.density_scale * gmem(p.wc_sigma)[__umul24(__umul24((unsigned)mz, (unsigned)dy) + (unsigned)my, (unsigned)dx) + (unsigned)mx];
+                const float ex = w.gx > 0.0f ? (mx == dx - 1 ? big : ((float)((mx + 1) << ER_WC_SHIFT) - l.Lx) * w.igx)
+                                             : (w.gx < 0.0f ? (mx == 0 ? big : ((float)(mx << ER_WC_SHIFT) - l.Lx) * w.igx) : big);
+                const float ey = w.gy > 0.0f ? (my == dy - 1 ? big : ((float)((my + 1) << ER_WC_SHIFT) - l.Ly) * w.igy)
+                                             : (w.gy < 0.0f ? (my == 0 ? big : ((float)(my << ER_WC_SHIFT) - l.Ly) * w.igy) : big);
+                const float ez = w.gz > 0.0f ? (mz == dz - 1 ? big : ((float)((mz + 1) << ER_WC_SHIFT) - l.Lz) * w.igz)
+                                             : (w.gz < 0.0f ? (mz == 0 ? big : ((float)(mz << ER_WC_SHIFT) - l.Lz) * w.igz) : big);
+                const float t_exit = fmaxf(fminf(w.t + fminf(ex, fminf(ey, ez)), w.MaxT), w.t + fmaxf(w.t * 1.0e-6f, 1.0e-7f));
+                bool hit = false;
+                if (mu > 0.0f) {
+                    const float t = w.t + w.tau / mu;
+                    hit = t < t_exit;
+                    if (hit) w.t = t;
+                    else w.tau = fmaxf(w.tau - mu * (t_exit - w.t), 0.0f);
+                }
+                if (!hit) {
+                    w.t = t_exit;
+                } else if (primary ? (w.t >= w.MaxT) : (w.t > w.MaxT)) {
+                    ended = true;
+                } else {
+#pragma unroll
+                    for (int k = B - 1; k > 0; --k) { tc[k] = tc[k - 1]; th[k] = th[k - 1]; }
+                    tc[0] = w.t;
+                    th[0] = w.rng.u() * mu;
+                    ++n;
+                    w.tau = -erm::logf_(w.rng.u());
+                }
+            }
+        }
+    }
+    if (n > 0) {
+        CellFetch f[B];
+        Lattice l[B];
+#pragma unroll
+        for (int k = 0; k < B; ++k) {
+            l[k] = to_lattice(p, add(w.O, scl(tc[k], w.D)));
+            f[k] = cell_fetch(p, l[k]);
+        }
+        uint32_t real = 0u;
+#pragma unroll
+        for (int k = 0; k < B; ++k)
+            if (k < n && th[k] < T.lut((int)cell_index(f[k])) * p.density_scale) real |= 1u << k;
+        while (real) {
+            const int k = 31 - __builtin_clz(real);
+            float t = tc[0];
+#pragma unroll
+            for (int j = 1; j < B; ++j) t = k == j ? tc[j] : t;
+            if (p.clip_count > 0) {
+                const f3 P = add(w.O, scl(t, w.D));
+                if (clip_possible(p, T, to_lattice(p, P)) && clipped(p, P)) { real &= ~(1u << k); continue; }
+            }
+            w.t = t;
+            w.rng = start;
+            for (int d = 2 * (n - 1 - k); d >= 0; --d) (void)w.rng.next_bits();
+            return 1;
+        }
+    }
+    return ended ? -1 : 0;
+}
+
+/* A wave walks its last ER_WC_DRAIN walks with 64 / ER_WC_DRAIN lanes each, and the last of those
+ * with ER_WC_LAST_G. 16 walks and 16 lanes: 8 or 32 walks are 3 - 15% slower, 4 or 32 lanes at the
+ * end 2 - 15%. */
+#define ER_WC_DRAIN 16
+#define ER_WC_LAST_G 16
+/* One walk in a group of G aligned lanes (G = 4 or 16), every lane with the same w: the next G
+ * collisions are taken as if each lay in the macrocell of the walk's position and were rejected.
+ * Lane j draws collision j (the draws do not depend on the volume), the distances are added up in
+ * the walk's order, and each lane tests its own: that it still starts in this macrocell, collides
+ * before leaving it, and whether it is real. The collisions before the first that fails the
+ * former tests count; there the walk goes on with a plain step. Walks of 256 to 1864 steps, one
+ * in eighteen, spend 90% of them on such collisions (macrocells whose majorant is a bone's), and
+ * the last of them kept whole waves: 17% of the shadow kernel's lanes were at work. 4 passes of
+ * the 256^3 CT volume at 1024 x 768, two phantoms: 9.1 / 10.3 ms with rounds alone, 5.6 / 8.3 so.
+ * Returns as wc_step. */
+template<int G>
+__device__ __forceinline__ int wc_group_step(const DevParams& p, const Tables& T, WcWalk& w, bool primary, int lane)
+{
+    const int dx = p.wc_dim[0], dy = p.wc_dim[1], dz = p.wc_dim[2];
+    const float big = 3.402823466e+38f;
+    const Lattice l0 = to_lattice(p, add(w.O, scl(w.t, w.D)));
+    const int mx = mc_axis(l0.Lx, ER_WC_SHIFT, dx), my = mc_axis(l0.Ly, ER_WC_SHIFT, dy), mz = mc_axis(l0.Lz, ER_WC_SHIFT, dz);
+    const float mu = p.density_scale * gmem(p.wc_sigma)[__umul24(__umul24((unsigned)mz, (unsigned)dy) + (unsigned)my, (unsigned)dx) + (unsigned)mx];
+    if (mu > 0.0f) {
+        const int j = lane & (G - 1), base = lane & ~(G - 1);
+        /* the state after collision j's optical depth was drawn, and that draw */
+        Rng mine = w.rng, r = w.rng;
+        uint32_t bits = 0u;
+#pragma unroll
+        for (int i = 1; i < G; ++i) {
+            (void)r.next_bits();
+            const uint32_t b = r.next_bits();
+            if (i == j) { mine = r; bits = b; }
+        }
+        const float tau = j == 0 ? w.tau : -erm::logf_((float)bits * 1.1920928955078125e-07f);
+        const float q = tau / mu;
+        float t = w.t;
+#pragma unroll
+        for (int i = 0; i < G - 1; ++i) {
+            const float qi = __shfl(q, base + i);
+            if (i < j) t = t + qi;
+        }
+        const float tc = t + q;
+        Rng after = mine;
+        const float u = after.u();
+        const Lattice l = to_lattice(p, add(w.O, scl(t, w.D)));
+        const bool same = mc_axis(l.Lx, ER_WC_SHIFT, dx) == mx && mc_axis(l.Ly, ER_WC_SHIFT, dy) == my &&
+                          mc_axis(l.Lz, ER_WC_SHIFT, dz) == mz;
+        const float ex = w.gx > 0.0f ? (mx == dx - 1 ? big : ((float)((mx + 1) << ER_WC_SHIFT) - l.Lx) * w.igx)
+                                     : (w.gx < 0.0f ? (mx == 0 ? big : ((float)(mx << ER_WC_SHIFT) - l.Lx) * w.igx) : big);
+        const float ey = w.gy > 0.0f ? (my == dy - 1 ? big : ((float)((my + 1) << ER_WC_SHIFT) - l.Ly) * w.igy)
+                                     : (w.gy < 0.0f ? (my == 0 ? big : ((float)(my << ER_WC_SHIFT) - l.Ly) * w.igy) : big);
+        const float ez = w.gz > 0.0f ? (mz == dz - 1 ? big : ((float)((mz + 1) << ER_WC_SHIFT) - l.Lz) * w.igz)
+                                     : (w.gz < 0.0f ? (mz == 0 ? big : ((float)(mz << ER_WC_SHIFT) - l.Lz) * w.igz) : big);
+        const float t_exit = fmaxf(fminf(t + fminf(ex, fminf(ey, ez)), w.MaxT), t + fmaxf(t * 1.0e-6f, 1.0e-7f));
+        const bool ok = same && w.segments + j < ER_WC_MAX_SEGMENTS && t < w.MaxT && tc < t_exit &&
+                        !(primary ? (tc >= w.MaxT) : (tc > w.MaxT));
+        bool real = false;
+        if (ok) {
+            Cnt cnt;
+            real = u * mu < sample_sigma<ER_MARCH_WOODCOCK, 0>(p, T, add(w.O, scl(tc, w.D)), primary, cnt) * p.density_scale;
+        }
+        const uint32_t all = (uint32_t)((1ull << G) - 1ull);
+        const uint32_t fails = ~(uint32_t)(__ballot(ok) >> base) & all, reals = (uint32_t)(__ballot(real) >> base) & all;
+        const int f = fails ? __ffs((int)fails) - 1 : G;          /* the first that does not count */
+        const int a = reals ? __ffs((int)reals) - 1 : G;          /* the first real one */
+        if (a < f || f == G) {
+            const int from = base + (a < f ? a : G - 1);
+            w.t = __shfl(tc, from);
+            w.rng.s0 = (uint32_t)__shfl((int)after.s0, from);
+            w.rng.s1 = (uint32_t)__shfl((int)after.s1, from);
+            if (a < f) return 1;
+            w.segments += G;
+            wc_first(w);
+            return 0;
+        }
+        w.t = __shfl(t, base + f);
+        w.tau = __shfl(tau, base + f);
+        w.rng.s0 = (uint32_t)__shfl((int)mine.s0, base + f);
+        w.rng.s1 = (uint32_t)__shfl((int)mine.s1, base + f);
+        w.segments += f;
+    }
+    Cnt cnt;
+    const int st = wc_step<ER_MARCH_WOODCOCK, 0>(p, T, w, primary, cnt);
+    if (w.need_tau) wc_first(w);
+    return st;
+}
+
+/* The last walks of a wave, at most 64 / G of them (the busy lanes'), each in a group of G lanes;
+ * the last 64 / ER_WC_LAST_G in groups of that many. On return the busy lanes' w.t and w.rng are their walks' ends'.
+ * Returns the walks' ends as wc_step (0 in the other lanes). Every lane of the wave calls it. */
+template<int G>
+__device__ __forceinline__ int wc_drain(const DevParams& p, const Tables& T, WcWalk& w, bool busy, bool primary, int lane)
+{
+    const unsigned long long bm = __ballot(busy);
+    unsigned long long x = bm;
+    for (int k = 0; k < lane / G; ++k) x &= x - 1ull;
+    bool gb = x != 0ull;
+    const int src = gb ? __ffsll((long long)x) - 1 : 0;
+    const bool first = (lane & (G - 1)) == 0;
+    WcWalk g;
+    g.O = mk(__shfl(w.O.x, src), __shfl(w.O.y, src), __shfl(w.O.z, src));
+    g.D = mk(__shfl(w.D.x, src), __shfl(w.D.y, src), __shfl(w.D.z, src));
+    g.t = __shfl(w.t, src);
+    g.MaxT = __shfl(w.MaxT, src);
+    g.tau = __shfl(w.tau, src);
+    g.gx = __shfl(w.gx, src); g.gy = __shfl(w.gy, src); g.gz = __shfl(w.gz, src);
+    g.igx = __shfl(w.igx, src); g.igy = __shfl(w.igy, src); g.igz = __shfl(w.igz, src);
+    g.segments = __shfl(w.segments, src);
+    g.need_tau = false;
+    g.rng.s0 = (uint32_t)__shfl((int)w.rng.s0, src);
+    g.rng.s1 = (uint32_t)__shfl((int)w.rng.s1, src);
+    int gst = 0;
+    for (;;) {
+        const unsigned long long left = __ballot(gb && first);
+        if (left == 0ull) break;
+        if constexpr (G < ER_WC_LAST_G) {
+            constexpr int NG = G * 4 < ER_WC_LAST_G ? G * 4 : ER_WC_LAST_G;
+            if (__popcll(left) <= 64 / NG) {
+                const int st = wc_drain<NG>(p, T, g, gb && first, primary, lane);
+                if (gb) gst = st;
+                break;
+            }
+        }
+        if (gb) {
+            gst = wc_group_step<G>(p, T, g, primary, lane);
+            gb = gst == 0;
+        }
+    }
+    const int from = busy ? __popcll(bm & ((1ull << lane) - 1ull)) * G : 0;
+    const int st = __shfl(gst, from);
+    const float t = __shfl(g.t, from);
+    const uint32_t s0 = (uint32_t)__shfl((int)g.rng.s0, from), s1 = (uint32_t)__shfl((int)g.rng.s1, from);
+    if (!busy) return 0;
+    w.t = t;
+    w.rng.s0 = s0;
+    w.rng.s1 = s1;
+    return st;
 }
 
 /* S_fixed >= 0: the threshold is still drawn (same draws) but S_fixed replaces it, so the march

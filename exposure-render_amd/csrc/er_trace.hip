@@ -119,6 +119,7 @@ __device__ __forceinline__ void primary_tile(const DevParams& p, const Tables& T
     float Tv = 0.0f;
     int it = 0;
     MarchState m;
+    WcWalk walk;
     const float StepSize = p.step_primary * p.minstep;
     if (active) {
         if (owner) paths++;
@@ -129,7 +130,13 @@ __device__ __forceinline__ void primary_tile(const DevParams& p, const Tables& T
         float nearT, farT;
         if (!intersect_box(r, ld3(p.minp), ld3(p.maxp), nearT, farT)) {
         } else if (FULL == ER_MARCH_WOODCOCK || (FULL == ER_MARCH_ANY && p.sampler == ER_SAMPLER_WOODCOCK)) {
-            vol = woodcock_track<FULL, COUNT>(p, T, r, nearT, farT, true, rng, Tv, Pv, cnt);
+            if constexpr (FULL == ER_MARCH_WOODCOCK && !COUNT) {
+                wc_begin(p, r, nearT, farT, rng, walk);
+                wc_first(walk);
+                marching = true;
+            } else {
+                vol = woodcock_track<FULL, COUNT>(p, T, r, nearT, farT, true, rng, Tv, Pv, cnt);
+            }
         } else if constexpr (FULL != ER_MARCH_WOODCOCK) {
             /* march_v's set-up; its loop follows, wave by wave */
             if (march_begin(p, r, nearT, farT, StepSize, rng, -1.0f, m)) {
@@ -138,7 +145,7 @@ __device__ __forceinline__ void primary_tile(const DevParams& p, const Tables& T
             }
         }
     }
-    /* The march loop (Woodcock walks are done), in three stages: every lane steps its own march until at most 64 / GD
+    /* The march loop (Woodcock walks: rounds, then wc_drain), in three stages: every lane steps its own march until at most 64 / GD
      * lanes (ER_COOP_LANES without group tails) are still marching; groups of GD lanes then
      * take those marches over; a march left after that (a single-ray wave's) is finished by the
      * whole wave (coop_march). A lone ray through kilo-samples of tissue would otherwise keep its
@@ -148,6 +155,29 @@ __device__ __forceinline__ void primary_tile(const DevParams& p, const Tables& T
      * the tile cost. */
     NoVisit nv;
     if constexpr (FULL == ER_MARCH_WOODCOCK) {
+        if constexpr (!COUNT) {
+            /* rounds, then the last walks in groups */
+            const bool walked = marching;
+            int end = 0;
+            for (;;) {
+                const int nm = __popcll(__ballot(marching));
+                if (nm <= ER_WC_DRAIN) break;
+                if (marching) {
+                    end = wc_round(p, T, walk, true);
+                    marching = end == 0;
+                }
+            }
+            if (__ballot(marching)) {
+                const int st = wc_drain<64 / ER_WC_DRAIN>(p, T, walk, marching, true, lane);
+                if (marching) end = st;
+            }
+            if (walked) {
+                rng = walk.rng;
+                vol = end > 0;
+                if (vol) { Tv = walk.t; Pv = add(walk.O, scl(walk.t, walk.D)); }
+            }
+            marching = false;
+        }
     } else if constexpr (G > 1) {
         if (marching) {
             f3 P = mk(0.0f, 0.0f, 0.0f);
@@ -613,13 +643,15 @@ __device__ __forceinline__ void shadow_drain(const DevParams& p, const Tables& T
 }
 
 /* shadow_marches for Woodcock tracking: each lane's walk advances one majorant segment per
- * loop iteration (wc_step) instead of running whole when its job starts, so that idle lanes
+ * loop iteration (wc_step; ER_MARCH_WOODCOCK: a round of them, and the wave's last walks in
+ * groups of lanes) instead of running whole when its job starts, so that idle lanes
  * refill while the others walk. */
 template<int FULL, int COUNT>
 __device__ __forceinline__ void shadow_marches_wc(const DevParams& p, const Tables& T, const ShadowJob* __restrict__ jobq,
                                                   unsigned char* __restrict__ vis, unsigned int* claim, unsigned int n,
                                                   unsigned int j, unsigned int claim_base, bool drained, int lane, Cnt& cnt)
 {
+    constexpr bool ROUNDS = FULL == ER_MARCH_WOODCOCK && !COUNT;
     WcWalk w;
     unsigned int slot = 0;
     bool busy = false;
@@ -640,12 +672,15 @@ __device__ __forceinline__ void shadow_marches_wc(const DevParams& p, const Tabl
                 vis[slot] = 1;
             } else {
                 wc_begin(p, r, nearT, farT, rng, w);
+                if constexpr (ROUNDS) wc_first(w);
                 busy = true;
             }
             j = n;
         }
         if (busy) {
-            const int st = wc_step<FULL, COUNT>(p, T, w, false, cnt);
+            int st;
+            if constexpr (ROUNDS) st = wc_round(p, T, w, false);
+            else st = wc_step<FULL, COUNT>(p, T, w, false, cnt);
             if (st != 0) {
                 vis[slot] = st > 0 ? 0 : 1;
                 busy = false;
@@ -655,6 +690,13 @@ __device__ __forceinline__ void shadow_marches_wc(const DevParams& p, const Tabl
         const int nidle = __popcll(idle);
         if (drained) {
             if (nidle == 64) break;
+            if constexpr (ROUNDS) {
+                if (64 - nidle <= ER_WC_DRAIN) {
+                    const int st = wc_drain<64 / ER_WC_DRAIN>(p, T, w, busy, false, lane);
+                    if (busy) vis[slot] = st > 0 ? 0 : 1;
+                    break;
+                }
+            }
         } else if (nidle >= ER_SHADOW_REFILL) {
             const int leader = __ffsll((long long)idle) - 1;
             unsigned int base = 0;

@@ -10,10 +10,10 @@
  *   mc_*    : macrocells of 8^3 cells (16^3 or 32^3 for volumes whose occupancy bits and
  *             opacity table would not fit 52.5 KB of LDS). For each, the
  *             min/max voxel over the voxels its samples can
- *             read, and (per tracer) the max of DensityScale * Opacity over the intensities a
- *             truncating trilinear sample can produce from that range ([min-3, max]). A sample
- *             whose macrocell maximum is 0 contributes exactly 0 to the optical depth, so the
- *             march skips its fetch and keeps the exact sequence of MinT additions.
+ *             read, and (per tracer) a bit: whether DensityScale * Opacity is positive for one of
+ *             the intensities a truncating trilinear sample can produce from that range
+ *             ([min-3, max]). Samples in a macrocell without it contribute exactly 0 to the optical
+ *             depth, so the march skips them and keeps the exact sequence of MinT additions.
  * Per tracer: XYZA float4 frame / running estimates, RGBA8 display (+ bilateral temporaries),
  * two uint32 seed planes (SoA), all row-major y * W + x.
  *

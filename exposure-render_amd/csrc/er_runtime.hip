@@ -375,11 +375,10 @@ struct PassSet {
  * stream) need only pass k's seeds, and the adjoint kernels of different passes nothing of each
  * other, so each set's run on a stream of its own: a pass's marches end with a few long ones,
  * which leave the device to the next passes'. 16 + 16 passes of a 128^3 volume at 512 x 512: 43 ms
- * with one stream, two sets and the general marches, 29 - 31 ms so (three streams and the first are the device's four
- * hardware queues). Made by the first call and resized with the film. */
-#ifndef ER_ADJ_SETS
+ * with one stream, two sets and the general marches; with the plain ones and 3 / 4 / 5 sets
+ * 33.6 / 31.9 / 35.1 ms (another phantom 31.1 / 30.0 / 30.1), but a tracer's first call, which makes
+ * the sets, 34 ms with 3 and 39 with 4. Resized with the film. */
 #define ER_ADJ_SETS 3
-#endif
 struct AdjWork {
     struct Set {
         DevBuf<uint32_t> s1s, s2s, counts, lcount;

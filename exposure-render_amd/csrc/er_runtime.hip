@@ -313,7 +313,7 @@ struct Volume {
     std::map<int, MacroGrid> grids;
     int mc_shift = 3;               /* default brick: 8 cells, coarser for very large volumes */
     uint16_t vmax = 0;
-    uint64_t upload = 0;            /* upload serial number (key of what is derived from the voxels) */
+    uint64_t upload = 0;            /* upload serial number (key of what is derived from the voxels); 0: no contents */
     /* the gradient-magnitude maximum of this upload, and the geometry it was taken with */
     float gm_max = 0.0f, gm_geometry[6] = {0, 0, 0, 0, 0, 0};
     uint64_t gm_upload = 0;
@@ -720,19 +720,34 @@ MacroGrid* volume_grid(Volume& v, int shift, int& st)
     return &g;
 }
 
-int upload_volume(Volume& v)
+/* whether the kernels can take the volume; needs no device */
+int check_volume(const er_volume_desc& d)
 {
-    const er_volume_desc& d = v.desc;
     const int rx = d.resolution[0], ry = d.resolution[1], rz = d.resolution[2];
-    const size_t n = (size_t)rx * ry * rz;
     if (rx <= 0 || ry <= 0 || rz <= 0) return set_error(ER_ERROR, "invalid volume resolution %d x %d x %d", rx, ry, rz);
     /* the cell records are indexed with 24-bit factors and a 32-bit index (er_device.h) */
-    if ((size_t)(rx + 1) * (ry + 1) >= ((size_t)1 << 24) || (size_t)(rz + 1) >= ((size_t)1 << 24) ||
-        (size_t)(rx + 1) * (ry + 1) * (rz + 1) >= ((size_t)1 << 32))
+    const size_t sx = (size_t)rx + 1, sy = (size_t)ry + 1, sz = (size_t)rz + 1;
+    if (sx * sy >= ((size_t)1 << 24) || sz >= ((size_t)1 << 24) || sx * sy * sz >= ((size_t)1 << 32))
         return set_error(ER_ERROR, "volume %d x %d x %d too large: (Rx+1)(Ry+1) and Rz+1 must stay below 2^24 and the "
                                    "cell count below 2^32", rx, ry, rz);
     if (!d.voxels) return set_error(ER_ERROR, "volume voxels pointer is NULL");
+    return ER_OK;
+}
+
+/* The descriptor and its voxels into v. A volume that check_volume refuses leaves v as it was. From
+ * the first buffer touched to the end v has no contents (upload 0), so that after a failure in
+ * between (out of memory) no tracer renders from buffers of two sizes: the scene's new version
+ * makes every tracer look at its volume again, and build_params refuses one without contents. */
+int upload_volume(Volume& v, const er_volume_desc& d)
+{
     int st;
+    if ((st = check_volume(d))) return st;
+    const int rx = d.resolution[0], ry = d.resolution[1], rz = d.resolution[2];
+    const size_t n = (size_t)rx * ry * rz;
+    g_scene_version++;
+    v.upload = 0;
+    v.desc = d;
+    v.desc.voxels = nullptr;
     if ((st = v.vox.alloc(n))) return st;
     HIP_TRY(hipMemcpy(v.vox.ptr, d.voxels, n * sizeof(uint16_t), hipMemcpyHostToDevice));
     const size_t nc = (size_t)(rx + 1) * (ry + 1) * (rz + 1);
@@ -938,6 +953,8 @@ int build_params(Tracer& t)
     const er_tracer_desc& d = t.desc;
     Volume* vol = g_volumes.find(d.volume_id);
     if (!vol) return set_error(ER_WARNING, "volume with ID:%d does not exist", d.volume_id);
+    if (!vol->upload)
+        return set_error(ER_ERROR, "volume with ID:%d has no voxels on the device: its last bind failed", d.volume_id);
     DevParams& P = t.host_params;
     memset(&P, 0, sizeof(P));
     camera_update(P, d.camera);
@@ -1799,18 +1816,18 @@ ER_API int er_bind_volume(er_volume_desc* d, int bind)
     if (bind) { int st = ensure_device(); if (st) return st; }
     return bind_generic(g_volumes, d, bind, [](Volume*& v, er_volume_desc& desc, bool fresh) -> int {
         if (fresh) v = new Volume();
-        const bool upload = fresh || desc.voxels_dirty;
+        const bool upload = fresh || desc.voxels_dirty || v->upload == 0;
         /* without new voxels the device buffers keep their size: the volume keeps its own
          * resolution and takes the rest (spacing, normalisation) from the descriptor, as
          * Buffer3D::operator= skips a source that is not Dirty (buffer3d.h:52-65) */
-        int res[3] = {v->desc.resolution[0], v->desc.resolution[1], v->desc.resolution[2]};
-        v->desc = desc;
-        if (!upload)
-            for (int i = 0; i < 3; ++i) v->desc.resolution[i] = res[i];
         if (upload) {
-            int st = upload_volume(*v);
+            int st = upload_volume(*v, desc);
             if (st) { if (fresh) { delete v; v = nullptr; } return st; }
             desc.voxels_dirty = 0;   /* Buffer3D dirty-gated copy (buffer3d.h:52-65) */
+        } else {
+            const int res[3] = {v->desc.resolution[0], v->desc.resolution[1], v->desc.resolution[2]};
+            v->desc = desc;
+            for (int i = 0; i < 3; ++i) v->desc.resolution[i] = res[i];
         }
         v->desc.voxels = nullptr;
         return ER_OK;

@@ -154,3 +154,52 @@ def test_adjoint_workspace_follows_the_film(fresh):
             got = gradient(r, w, h)
             assert np.abs(got - want[(w, h)]).max() <= 2e-5 * np.abs(want[(w, h)]).max()
     r.close()
+
+
+def _nothing(v):
+    v.resolution[0], v.resolution[2] = 4 * v.resolution[0], 3 * v.resolution[2]
+    v.voxels = None
+
+
+def _empty(v):
+    v.resolution[1] = 0
+
+
+def _too_large(v):
+    v.resolution[0] = v.resolution[1] = 1 << 13
+    v.resolution[2] = 1
+
+
+@pytest.mark.parametrize("edit", [_nothing, _empty, _too_large])
+def test_a_refused_volume_leaves_the_bound_one(fresh, edit):
+    """A rebind that is refused changes nothing: the next binds and passes see the volume as it was,
+    its size with its buffers, and a later good rebind takes its place."""
+    print(f"[rebind] refused: {edit.__name__}", flush=True)
+    sc = _scene()
+    r = er.Renderer(sc)
+    base = _passes(r)
+    v = r.volume
+    kept = [v.resolution[i] for i in range(3)]
+    v.spacing[0] = 3.0
+    edit(v)
+    v.voxels_dirty = 1
+    assert r.lib.er_bind_volume(C.byref(v), 1) == capi.ER_ERROR
+    r.rebind()
+    again = _passes(r)
+    for i in range(3):
+        v.resolution[i] = kept[i]
+    v.spacing[0] = 1.0
+    other = np.ascontiguousarray(sc.voxels[::-1, :, ::-1] // 2)
+    v.voxels = other.ctypes.data_as(C.POINTER(C.c_uint16))
+    _bind(r, "volume")
+    r.rebind()
+    got = _passes(r)
+    r.close()
+    sc.voxels[:] = other
+    f = er.Renderer(sc)
+    want = _passes(f)
+    f.close()
+    for x, y in ((again, base), (got, want)):
+        assert np.array_equal(x[0], y[0]) and np.array_equal(x[2], y[2])
+        assert np.array_equal(x[1][0], y[1][0]) and np.array_equal(x[1][1], y[1][1])
+    assert not np.array_equal(base[2], want[2])

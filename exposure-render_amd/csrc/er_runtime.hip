@@ -2675,7 +2675,8 @@ ER_API int er_get_autofocus_distance(int tracer_id, int film_u, int film_v, floa
     const size_t work = erd_autofocus_work_size();
     if (!t->focus.ptr) {
         if ((st = t->focus.alloc(work))) return st;
-        const hipError_t e = hipMemset(t->focus.ptr, 0, work);
+        /* on the kernel's own stream: the null stream is not ordered before it */
+        const hipError_t e = erd_launch_zero_words((uint32_t*)t->focus.ptr, work / sizeof(uint32_t), t->stream);
         if (e != hipSuccess) {
             t->focus.release();
             return set_error(ER_ERROR, "%s (autofocus workspace)", hipGetErrorString(e));

@@ -42,3 +42,19 @@ def test_autofocus_matches_the_sequential_rays(fresh, kind):
         assert d == ref, (kind, u, v, d, ref)
         assert r.autofocus_distance(u, v) == d
     r.close()
+
+
+def test_first_call_of_a_tracer(fresh):
+    """The call that makes a tracer's workspace, in memory that earlier tracers gave back: its
+    arrival count has to be cleared before the kernel counts in it."""
+    sc = _scene("full")
+    orc = O.Oracle(sc)
+    W, H = sc.film
+    for k in range(12):
+        r = er.Renderer(sc)
+        if k % 2:
+            r.render_passes(2)      # tables already built, nothing else waits for the device
+        d = r.autofocus_distance(W // 2 + k, H // 2)
+        assert d == orc.autofocus(W // 2 + k, H // 2, *r.autofocus_seeds(W // 2 + k, H // 2)), k
+        assert r.autofocus_distance(W // 2 + k, H // 2) == d
+        r.close()

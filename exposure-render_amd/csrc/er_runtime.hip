@@ -1305,7 +1305,10 @@ int build_params(Tracer& t)
             for (int k = -R; k <= R; ++k) kd[k + R] = erm::expf_(-((float)(k * k)) / (2.0f * ss * ss));
             for (int q = 0; q < 256; ++q) gs[q] = erm::expf_(-((float)(q * q)) / (2.0f * sr * sr));
             if ((st = t.bilateral.alloc(bp.size()))) return st;
-            HIP_TRY(hipMemcpy(t.bilateral.ptr, bp.data(), bp.size(), hipMemcpyHostToDevice));
+            /* on the tracer's stream (the null stream is not ordered before it), and there until bp goes */
+            const hipError_t e = hipMemcpyAsync(t.bilateral.ptr, bp.data(), bp.size(), hipMemcpyHostToDevice, t.stream);
+            HIP_TRY(hipStreamSynchronize(t.stream));
+            HIP_TRY(e);
             t.bilateral_key = filter;
         }
     }

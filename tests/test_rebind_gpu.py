@@ -203,3 +203,22 @@ def test_a_refused_volume_leaves_the_bound_one(fresh, edit):
         assert np.array_equal(x[0], y[0]) and np.array_equal(x[2], y[2])
         assert np.array_equal(x[1][0], y[1][0]) and np.array_equal(x[1][1], y[1][1])
     assert not np.array_equal(base[2], want[2])
+
+
+def test_display_filter_follows_each_bind(fresh):
+    """The filter's tables are rebuilt by the bind that changes them and read by the pass that
+    follows at once, on the tracer's streams."""
+    sc = _scene()
+    r = er.Renderer(sc)
+    for radius, spatial, rng in [(2, 1.5, 20.0), (7, 4.0, 60.0), (0, 1.0, 1.0), (32, 9.0, 30.0), (2, 1.5, 20.0)]:
+        print(f"[rebind] filter {radius} {spatial} {rng}", flush=True)
+        images = []
+        for d in (r.tracer, sc.tracer):
+            d.settings.bilateral_radius, d.settings.bilateral_sigma_spatial, d.settings.bilateral_sigma_range = radius, spatial, rng
+        r.rebind()
+        f = er.Renderer(sc)
+        for x in (r, f):
+            images.append(_passes(x)[2])
+        f.close()
+        assert np.array_equal(*images)
+    r.close()

@@ -119,6 +119,17 @@ __device__ __forceinline__ bool clipped(const DevParams& p, f3 P)
 /* no occupancy test per sample, table of products with the step size */
 #define ER_MARCH_IS_PLAIN(M) ((M) == ER_MARCH_PLAIN || (M) == ER_MARCH_CLIP)
 
+/* The samples of a primary march iteration. The general form keeps an occupancy flag and a value
+ * for each sample besides its cell, so 10 of them take 222 VGPRs (2 waves per SIMD); 6, with 6 in
+ * the groups of 4 lanes, take 161 (3 waves). 8 passes of the CT volume with a band of negative
+ * opacity at 1024 x 768, 10 against 6: untuned 3.56 -> 3.07 ms, with 256 heavy tiles 4.54 -> 3.77,
+ * with none 4.08 -> 4.51; a batch of clipped and Woodcock jobs 20.1 -> 18.7 ms. 8, or 8 in the
+ * groups, lie in between. */
+#ifndef ER_BATCH_PRIMARY_ANY
+#define ER_BATCH_PRIMARY_ANY 6
+#endif
+template<int M> struct PrimaryBatch { static constexpr int value = M == ER_MARCH_ANY ? ER_BATCH_PRIMARY_ANY : ER_BATCH_PRIMARY; };
+
 /* Per-block copies of the macrocell occupancy bits and (when it fits) the opacity LUT. */
 struct Tables {
     /* bit m set <=> macrocell m holds a sample with sigma > 0: in LDS, or (bits_glb set) in
@@ -1004,7 +1015,7 @@ __device__ __forceinline__ bool march_v(const DevParams& p, const Tables& T, con
 
 /* The rest of one primary march (SampleVolume's loop, raymarching.h:55-68) run by the whole
  * wave on one ray: m is the same in every lane. A march whose wave has only a few lanes still
- * marching would otherwise spend one memory round trip per ER_BATCH_PRIMARY samples; here each
+ * marching would otherwise spend one memory round trip per PrimaryBatch samples; here each
  * round trip reads 64 consecutive samples, lane k taking sample k. Lane k finds t_k with the
  * same k float additions of StepSize as the sequential loop, and the optical depth is then
  * accumulated in sample order (one addition per sample, broadcast from its lane), with the
@@ -1013,7 +1024,7 @@ __device__ __forceinline__ bool march_v(const DevParams& p, const Tables& T, con
  * skipped by march_step's exact skip. Returns 1 on an event (Pout = the sample, m.MinT one step
  * beyond it), -1 when the ray leaves the volume first; the same in every lane. Counts go to
  * lane 0's cnt; steps counts the iterations the per-lane loop would have taken (a skip, or
- * ER_BATCH_PRIMARY samples). */
+ * PrimaryBatch samples). */
 template<int FULL, int COUNT>
 __device__ int coop_march(const DevParams& p, const Tables& T, MarchState& m, float StepSize, int lane, Cnt& cnt, f3& Pout,
                           int& steps)
@@ -1059,7 +1070,7 @@ __device__ int coop_march(const DevParams& p, const Tables& T, MarchState& m, fl
         }
         const unsigned long long lm = __ballot(live);
         const int ns = term == 1 ? kend + 1 : kend;
-        steps += (ns + ER_BATCH_PRIMARY - 1) / ER_BATCH_PRIMARY;   /* the sequential loop's iterations */
+        steps += (ns + PrimaryBatch<FULL>::value - 1) / PrimaryBatch<FULL>::value;   /* the sequential loop's iterations */
         if (COUNT && lane == 0) {
             const unsigned long long within = ns >= 64 ? ~0ull : ((1ull << ns) - 1ull);
             cnt.primary += (uint32_t)ns;
@@ -1081,15 +1092,20 @@ __device__ int coop_march(const DevParams& p, const Tables& T, MarchState& m, fl
 }
 
 /* samples each lane of a G-lane group loads per round trip in group_march (3 or 4 for G = 16:
- * within 2% of 2); observed marches (the adjoint's) hold more registers per sample */
+ * within 2% of 2); observed marches (the adjoint's) and the general form hold more registers per
+ * sample */
 #ifndef ER_GROUP4_BATCH
 #define ER_GROUP4_BATCH 8
 #endif
 #ifndef ER_GROUP4_BATCH_VISIT
 #define ER_GROUP4_BATCH_VISIT 6
 #endif
-template<int G, bool VISIT> struct GroupBatch {
-    static constexpr int value = G >= 16 ? 2 : (VISIT ? ER_GROUP4_BATCH_VISIT : ER_GROUP4_BATCH);
+#ifndef ER_GROUP4_BATCH_ANY
+#define ER_GROUP4_BATCH_ANY 6
+#endif
+template<int M, int G, bool VISIT> struct GroupBatch {
+    static constexpr int value = G >= 16 ? 2 : (VISIT ? ER_GROUP4_BATCH_VISIT
+                                                      : (M == ER_MARCH_ANY ? ER_GROUP4_BATCH_ANY : ER_GROUP4_BATCH));
 };
 
 /* lane Q's v within each aligned group of G lanes (Q a constant): a DPP quad permutation for
@@ -1143,7 +1159,7 @@ __device__ __forceinline__ void group_count(const float (&c)[KB], float Sum, flo
  * (G = 4 or 16; 64 / G rays per wave): m is the same in every lane of the group. A round either
  * skips the empty macrocell at MinT (march_step's exact skip) or reads B = GroupBatch x G
  * consecutive samples, lane k of the group taking samples k, k + G, ..., k + (B/G - 1) G, so a
- * ray advances B samples per memory round trip instead of ER_BATCH_PRIMARY / ER_BATCH_SHADOW.
+ * ray advances B samples per memory round trip instead of PrimaryBatch / ER_BATCH_SHADOW.
  * As in coop_march every position is the sequential loop's (the same float additions of
  * StepSize), the optical depth is accumulated in sample order (one addition per sample, its
  * addend fetched from the lane that loaded it) with the loop's end test before each sample and
@@ -1152,7 +1168,7 @@ __device__ __forceinline__ void group_count(const float (&c)[KB], float Sum, flo
  * cross-lane reads stay inside active lanes. Returns 0 to go on, 1 on an event (Pout = the
  * sample, m.MinT one step beyond it), -1 when the ray leaves the volume first; counts go to
  * the group's first lane. iters: the iterations the one-lane-per-ray loop would have taken for
- * this round (1 for a skip, else the samples consumed over ER_BATCH_PRIMARY, rounded up).
+ * this round (1 for a skip, else the samples consumed over PrimaryBatch, rounded up).
  * group_step_v also reports the round's fetched samples to an observer: each lane passes its
  * own samples that the round consumed (vis.sample, in sample order within the lane, so each
  * lane's observer sees a subsequence of the march), and on an event every lane of the group
@@ -1161,7 +1177,7 @@ template<int FULL, int COUNT, int G, bool PRIMARY, class Visit>
 __device__ __forceinline__ int group_step_v(const DevParams& p, const Tables& T, MarchState& m, float StepSize, int lane,
                                             Cnt& cnt, f3& Pout, int& iters, Visit& vis)
 {
-    constexpr int KB = GroupBatch<G, !IsNoVisit<Visit>::value>::value;
+    constexpr int KB = GroupBatch<FULL, G, !IsNoVisit<Visit>::value>::value;
     constexpr int NS = KB * G;
     const int k = lane & (G - 1);
     const int gb = lane & ~(G - 1);
@@ -1231,7 +1247,7 @@ __device__ __forceinline__ int group_step_v(const DevParams& p, const Tables& T,
         } else {
             te = group_bcast<G, G - 1>(tk[KB - 1]);
         }
-        iters = (last + ER_BATCH_PRIMARY) / ER_BATCH_PRIMARY;
+        iters = (last + PrimaryBatch<FULL>::value) / PrimaryBatch<FULL>::value;
         m.Sum = Sum;
         m.MinT = te + StepSize;
         if (PRIMARY ? (te >= m.MaxT) : (te > m.MaxT)) return -1;
@@ -1274,7 +1290,7 @@ __device__ __forceinline__ int group_step_v(const DevParams& p, const Tables& T,
 #pragma unroll
         for (int j = 0; j < KB; ++j)
             vis.maybe(j * G + k <= last && (PRIMARY ? (tk[j] < m.MaxT) : (tk[j] <= m.MaxT)) && sg[j] > 0.0f, ivs[j], sg[j]);
-        iters = (last + ER_BATCH_PRIMARY) / ER_BATCH_PRIMARY;
+        iters = (last + PrimaryBatch<FULL>::value) / PrimaryBatch<FULL>::value;
         m.Sum = Sum;
         m.MinT = te + StepSize;
         if (PRIMARY ? (te >= m.MaxT) : (te > m.MaxT)) return -1;
@@ -1316,7 +1332,7 @@ __device__ __forceinline__ int group_step_v(const DevParams& p, const Tables& T,
     int send = NS, term = 0;
     group_accumulate<G, KB>(c, Sum, m.S, nin, send, term);
     const int ns = term == 1 ? send + 1 : send;
-    iters = (ns + ER_BATCH_PRIMARY - 1) / ER_BATCH_PRIMARY;
+    iters = (ns + PrimaryBatch<FULL>::value - 1) / PrimaryBatch<FULL>::value;
     if constexpr (!IsNoVisit<Visit>::value) {
 #pragma unroll
         for (int j = 0; j < KB; ++j)

@@ -192,7 +192,7 @@ __device__ __forceinline__ void primary_tile(const DevParams& p, const Tables& T
         if (nm == 0 || nm <= (ER_PRIMARY_DRAIN_G > 0 ? 64 / GD : ER_COOP_LANES) || ray >= 0) break;
         if (marching) {
             ++it;
-            const int st = march_step<FULL, COUNT, ER_BATCH_PRIMARY, NoVisit>(p, T, m, true, StepSize, cnt, nv, Pv);
+            const int st = march_step<FULL, COUNT, PrimaryBatch<FULL>::value, NoVisit>(p, T, m, true, StepSize, cnt, nv, Pv);
             if (st != 0) { marching = false; vol = st > 0; Tv = m.MinT; }
         }
     }

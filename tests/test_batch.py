@@ -193,3 +193,55 @@ def test_cached_batch_graph_reproduces_the_batch(fresh):
         assert np.array_equal(want[0], got[k][0]) and np.array_equal(want[2], got[k][2]), f"job {k}"
     for r in rs:
         r.close()
+
+
+def _with(sc, kind):
+    if "clip" in kind:
+        tm, inv = scenes.look_at((0.2, 0.1, 0.3), (1.0, 0.5, 0.2))
+        sc.add_clip(scenes.clipping_shape(capi.SHAPE_BOX, tm, inv, size=(0.5, 0.6, 0.4)))
+    if "woodcock" in kind:
+        sc.tracer.settings.sampler = capi.SAMPLER_WOODCOCK
+    if "negative" in kind:
+        sc.tracer.opacity.init()
+        sc.tracer.opacity.add(0.0, 0.0).add(300.0, 0.0).add(900.0, -0.05).add(1500.0, 0.3).add(4095.0, 1.0)
+    if "wide" in kind:        # values up to 65535: the opacity tables stay in global memory
+        sc.voxels[:] = np.minimum(sc.voxels.astype(np.uint32) * 16, 65535).astype(np.uint16)
+        sc.tracer.opacity.init()
+        sc.tracer.opacity.add(0.0, 0.0).add(4800.0, 0.0).add(24000.0, 0.3).add(65535.0, 1.0)
+
+
+#: the jobs' kinds, in turn; the batch takes their common march form
+MIXES = [("clip",), ("plain", "clip"), ("clip", "plain"), ("clip", "woodcock"), ("woodcock", "clip"), ("plain", "negative"),
+         ("negative", "plain"), ("clip", "negative"), ("clip wide",), ("plain", "clip wide"), ("plain wide", "clip")]
+
+
+@pytest.mark.parametrize("mix", MIXES, ids=lambda m: "+".join(m).replace(" ", "_"))
+@pytest.mark.parametrize("rays", [64, 4])
+def test_batches_of_mixed_march_forms_match_sequential(fresh, mix, rays):
+    """One form of the marches for a whole batch: clipped jobs, clipped beside plain ones (either
+    first) and jobs that only the general form can march render in a batch what each renders alone
+    in its own form, bit for bit, with one lane to a ray and with sixteen."""
+    jobs = scenes.config_batch(n_jobs=4, scale=0.1, seed=12)
+    for k, sc in enumerate(jobs):
+        _with(sc, mix[k % len(mix)])
+    passes = [min(sc.passes, 3 + k) for k, sc in enumerate(jobs)]
+    print(f"[batch] forms {mix} rays {rays} films={[sc.film for sc in jobs]} passes={passes}", flush=True)
+    out = []
+    for batched in (False, True):
+        rs = [er.Renderer(sc) for sc in jobs]
+        for k, r in enumerate(rs):
+            r.set_seeds(*er.seeds_for(r.W, r.H, 80 + k))
+            if rays != 64:
+                r.set_tune(8, 8, 7, 4, 0, rays, rays, 4)
+        if batched:
+            er.render_batch(rs, passes)
+        else:
+            for r, n in zip(rs, passes):
+                r.render_passes(n)
+        out.append([state(r) for r in rs])
+        for r in rs:
+            r.close()
+    for k, (a, b) in enumerate(zip(*out)):
+        for name, x, y in zip(("frame", "running", "seeds1", "seeds2", "display"), a[:5], b[:5]):
+            assert np.array_equal(x, y), f"job {k}: {name} differs"
+        assert a[5] == b[5] == passes[k]

@@ -222,3 +222,41 @@ def test_display_filter_follows_each_bind(fresh):
         f.close()
         assert np.array_equal(*images)
     r.close()
+
+
+@pytest.mark.parametrize("tuned", [False, True])
+def test_clipping_object_comes_and_goes(fresh, tuned):
+    """A kept tracer changes march form, and untuned its bricks, when its clipping object is added
+    to it, taken from it or unbound; each time it renders as a tracer bound fresh."""
+    def scene(clip):
+        sc = scenes.config_ct(scale=0.2, bilateral=True)
+        sc.tracer.camera.film_size[0], sc.tracer.camera.film_size[1] = 90, 70
+        if clip:
+            sc.add_clip(scenes.clipping_box((0.3, 0.0, 0.0), (0.4, 1.1, 1.1)))
+        return sc
+
+    def passes(r):
+        if tuned:
+            r.set_tune(4, 8, 4, 4, 64, 64, 64, 16)
+        out = _passes(r)
+        r.seed(7)
+        r.render_estimate()
+        return out + (r.frame(),)
+    want = {}
+    for clip in (False, True):
+        f = er.Renderer(scene(clip))
+        want[clip] = passes(f)
+        f.close()
+    assert not np.array_equal(want[False][2], want[True][2])
+    r = er.Renderer(scene(True))
+    ident = r.tracer.clipping_ids[0]
+    for clip, count, bound in [(True, 1, True), (False, 0, True), (True, 1, True), (False, 1, False)]:
+        print(f"[rebind] clipping object: listed {count} bound {bound} tuned {tuned}", flush=True)
+        r.tracer.clipping_count, r.tracer.clipping_ids[0] = count, ident
+        if not bound:
+            assert r.lib.er_bind_clipping_object(C.byref(r.clips[0]), 0) == capi.ER_OK
+        r.rebind()
+        got = passes(r)
+        assert all(np.array_equal(a, b) for a, b in zip((got[0], got[2], got[3]), (want[clip][0], want[clip][2], want[clip][3])))
+        assert all(np.array_equal(a, b) for a, b in zip(got[1], want[clip][1]))
+    r.close()

@@ -471,6 +471,7 @@ struct Tracer {
     int mc_shift = 0, tile_shift = 3, blocks_per_cu = 0, shadow_waves_per_cu = 4, heavy_tiles = 0, rays_per_wave = 64,
         shadow_rays_per_wave = 64, heavy_rays_per_wave = 4;
     bool tuned = false;               /* set by er_set_tune / er_autotune; until then launch_for chooses */
+    bool given = false;               /* the configuration is er_set_tune's, for every pass */
     /* primary tiles: each pass records its tiles' march steps and orders the next pass's tiles
      * most expensive first; the order is valid for the tile shape and count it was built for */
     DevBuf<uint32_t> tile_cost, tile_order;
@@ -1325,8 +1326,10 @@ bool use_bilateral(const Tracer& t)
     return t.desc.settings.estimator == ER_ESTIMATOR_FULL && t.desc.settings.bilateral;
 }
 
-/* How a tracer's passes are launched. Tuned: as er_set_tune or er_autotune set it. Otherwise by the
- * film's size and by whether the pass runs alone (er_render_estimate) or overlaps others:
+/* How a tracer's passes are launched. As er_set_tune gave it, or, passes that overlap, as er_autotune
+ * found it by timing such passes (what it found for the CT workload took a pass alone from 0.51 to
+ * 0.55 ms, for the 256 x 256 blobs from 0.20 to 0.23); otherwise by the film's size and by whether
+ * the pass runs alone (er_render_estimate) or overlaps others:
  *  - 64 rays per wave, the rays of the 768 most expensive tiles in groups of 4 lanes (their long
  *    marches end the kernel): against no heavy tiles, one frame of the CT volume at 640 x 480
  *    0.68 -> 0.61 ms, the compat loop 3.96 -> 3.61, 8 passes with objects 3.50 -> 3.08, 16 CT
@@ -1344,7 +1347,7 @@ struct Launch {
 };
 Launch launch_for(const Tracer& t, bool alone)
 {
-    if (t.tuned)
+    if (t.given || (t.tuned && !alone))
         return {t.blocks_per_cu, t.shadow_waves_per_cu, t.heavy_tiles, t.rays_per_wave, t.shadow_rays_per_wave,
                 t.heavy_rays_per_wave};
     if (alone && (long long)t.W * t.H <= (long long)g_cus * 4 * 2 * 64) return {4, 16, 0, 16, 16, 4};
@@ -1488,6 +1491,45 @@ void fill_tune(const Tracer& t, er_tune& r)
     r.shadow_rays_per_wave = t.shadow_rays_per_wave;
     r.heavy_rays_per_wave = t.heavy_rays_per_wave;
 }
+
+/* What a built tracer's overlapped passes run with, where the searches start: until it is tuned not
+ * what fill_tune reports but launch_for's choice, which a search has to beat. (Started from the
+ * reported 8-cell bricks without heavy tiles it could end slower than no tuning: 64^3 blobs at 640 x
+ * 480 0.206 -> 0.213 ms a pass, now 0.205 -> 0.201; 512 x 512 x 460 at 1080p 1.178 -> 1.187, now
+ * 1.172 -> 1.161.) */
+void running_tune(const Tracer& t, er_tune& r)
+{
+    fill_tune(t, r);
+    if (t.tuned) return;
+    const Launch L = launch_for(t, false);
+    r.brick = 1 << t.host_params.mc_shift;
+    r.blocks_per_cu = L.blocks_per_cu;
+    r.shadow_waves_per_cu = L.shadow_waves_per_cu;
+    r.heavy_tiles = L.heavy_tiles;
+    r.rays_per_wave = L.rays_per_wave;
+    r.shadow_rays_per_wave = L.shadow_rays_per_wave;
+    r.heavy_rays_per_wave = L.heavy_rays_per_wave;
+}
+
+/* a tracer's configuration as it is, to be put back when a search fails */
+struct TuneState {
+    int mc_shift, tile_shift, blocks_per_cu, shadow_waves_per_cu, heavy_tiles, rays_per_wave, shadow_rays_per_wave,
+        heavy_rays_per_wave;
+    bool tuned, given;
+    explicit TuneState(const Tracer& t)
+        : mc_shift(t.mc_shift), tile_shift(t.tile_shift), blocks_per_cu(t.blocks_per_cu),
+          shadow_waves_per_cu(t.shadow_waves_per_cu), heavy_tiles(t.heavy_tiles), rays_per_wave(t.rays_per_wave),
+          shadow_rays_per_wave(t.shadow_rays_per_wave), heavy_rays_per_wave(t.heavy_rays_per_wave), tuned(t.tuned),
+          given(t.given) {}
+    void restore(Tracer& t) const
+    {
+        t.mc_shift = mc_shift; t.tile_shift = tile_shift; t.blocks_per_cu = blocks_per_cu;
+        t.shadow_waves_per_cu = shadow_waves_per_cu; t.heavy_tiles = heavy_tiles; t.rays_per_wave = rays_per_wave;
+        t.shadow_rays_per_wave = shadow_rays_per_wave; t.heavy_rays_per_wave = heavy_rays_per_wave;
+        t.tuned = tuned; t.given = given;
+        t.built_version = 0;
+    }
+};
 
 int apply_tune(Tracer& t, const er_tune& r)
 {
@@ -1938,10 +1980,11 @@ ER_API int er_render_passes(int tracer_id, int passes, er_timing* timing)
     return ER_OK;
 }
 
-/* Coordinate search over brick size, tile shape and persistent workgroups per CU. Each
- * candidate renders the same passes from the same seeds (median of three trials of about
- * 30 ms, or `passes` passes when given); a candidate must be 3% faster to be taken. The
- * tracer's render state is restored afterwards. Results are cached by scene. */
+/* Coordinate search over brick size, tile shape and persistent workgroups per CU, from the
+ * configuration the tracer's passes run with. Each candidate renders the same passes from the
+ * same seeds (median of three trials of about 30 ms, or `passes` passes when given); a candidate
+ * must be 3% faster to be taken. The tracer's render state is restored afterwards. Results are
+ * cached by scene. */
 ER_API int er_autotune(int tracer_id, int passes, int flags, er_tune* out)
 {
     std::lock_guard<std::recursive_mutex> lk(g_mutex);
@@ -1955,6 +1998,7 @@ ER_API int er_autotune(int tracer_id, int passes, int flags, er_tune* out)
     if (cached != g_tune_cache.end() && !(flags & ER_TUNE_FORCE)) {
         er_tune r = cached->second;
         if ((st = apply_tune(t, r))) return st;
+        t.given = false;
         if ((st = build_params(t))) return st;
         r.trials = 0;
         if (out) *out = r;
@@ -1963,11 +2007,11 @@ ER_API int er_autotune(int tracer_id, int passes, int flags, er_tune* out)
     if (t.W == 0 || t.H == 0) return set_error(ER_ERROR, "tracer %d has an empty film", tracer_id);
     Snapshot snap;
     if ((st = snap.save(t))) return st;
-    const int mc0 = t.mc_shift, ts0 = t.tile_shift, bpc0 = t.blocks_per_cu, sw0 = t.shadow_waves_per_cu,
-              ht0 = t.heavy_tiles, rw0 = t.rays_per_wave, srw0 = t.shadow_rays_per_wave, hrw0 = t.heavy_rays_per_wave;
-    const bool tuned0 = t.tuned;
+    const TuneState before(t);
     er_tune cur{};
-    fill_tune(t, cur);
+    running_tune(t, cur);
+    const er_tune start = cur;
+    bool moved_ever = false;
     int trials = 0;
     int reps = 3;
     /* a candidate's time is the median of its trials: some configurations (many shadow waves
@@ -1993,7 +2037,13 @@ ER_API int er_autotune(int tracer_id, int passes, int flags, er_tune* out)
             passes = std::max(2, std::min(64, (int)std::ceil(ER_TUNE_TRIAL_MS / std::max(probe / 2.0f, 1e-3f))));
     }
     if (!st) st = measure(cur, cur_ms);
-    const float default_ms = cur_ms;
+    float default_ms = cur_ms;
+    /* the incumbent measured again; the start's time goes along while it is the incumbent */
+    auto measure_again = [&]() -> int {
+        const int s = measure(cur, cur_ms);
+        if (!s && !moved_ever) default_ms = cur_ms;
+        return s;
+    };
     std::vector<const Volume*> vols{g_volumes.find(t.desc.volume_id)};
     /* rays per wave right after the brick: the later axes are tuned around them. A second sweep,
      * from a fresh measurement of the incumbent, catches axes that interact (the primary
@@ -2001,13 +2051,13 @@ ER_API int er_autotune(int tracer_id, int passes, int flags, er_tune* out)
      * nothing. */
     for (int sweep = 0; sweep < 2 && !st; ++sweep) {
         bool moved = false;
-        if (sweep > 0 && (st = measure(cur, cur_ms))) break;
+        if (sweep > 0 && (st = measure_again())) break;
         for (int axis : {0, 5, 6, 1, 2, 3, 4, 7}) {
             if (st) break;
             for (const er_tune& c : tune_candidates(axis, cur, vols)) {
                 float ms = 0.0f;
                 if ((st = measure(c, ms))) break;
-                if (ms < ER_TUNE_MARGIN * cur_ms) { cur = c; cur_ms = ms; moved = true; }
+                if (ms < ER_TUNE_MARGIN * cur_ms) { cur = c; cur_ms = ms; moved = moved_ever = true; }
             }
         }
         if (!moved) break;
@@ -2017,23 +2067,20 @@ ER_API int er_autotune(int tracer_id, int passes, int flags, er_tune* out)
      * and a candidate need only be 1.5% faster */
     if (!st) {
         reps = 6;
-        st = measure(cur, cur_ms);
+        st = measure_again();
         for (int axis : {1, 2, 3}) {
             if (st) break;
             for (const er_tune& c : tune_candidates(axis, cur, vols)) {
                 float ms = 0.0f;
                 if ((st = measure(c, ms))) break;
-                if (ms < ER_TUNE_FINE_MARGIN * cur_ms) { cur = c; cur_ms = ms; }
+                if (ms < ER_TUNE_FINE_MARGIN * cur_ms) { cur = c; cur_ms = ms; moved_ever = true; }
             }
         }
     }
-    if (!st) st = apply_tune(t, cur);
-    if (st) {
-        t.mc_shift = mc0; t.tile_shift = ts0; t.blocks_per_cu = bpc0; t.shadow_waves_per_cu = sw0; t.heavy_tiles = ht0;
-        t.rays_per_wave = rw0; t.shadow_rays_per_wave = srw0; t.heavy_rays_per_wave = hrw0;
-        t.tuned = tuned0;
-        t.built_version = 0;
-    }
+    /* a gain that a closer look did not bear out */
+    if (cur_ms > default_ms) { cur = start; cur_ms = default_ms; }
+    if (!st && !(st = apply_tune(t, cur))) t.given = false;
+    if (st) before.restore(t);
     const int rst = snap.restore(t);
     if (st) return st;
     if (rst) return rst;
@@ -2067,12 +2114,14 @@ ER_API int er_autotune_batch(const er_batch_item* items, int n, int rounds, er_t
     }
     std::vector<std::unique_ptr<Snapshot>> snaps;
     std::vector<er_tune> orig(n);
-    std::vector<char> tuned0(n);
+    std::vector<TuneState> before;
+    bool one_brick = true;
     for (int k = 0; k < n; ++k) {
-        tuned0[k] = ts[k]->tuned;
+        before.emplace_back(*ts[k]);
         snaps.emplace_back(new Snapshot());
         if ((st = snaps[k]->save(*ts[k]))) return st;
-        fill_tune(*ts[k], orig[k]);
+        running_tune(*ts[k], orig[k]);
+        one_brick = one_brick && orig[k].brick == orig[0].brick;
     }
     std::vector<er_batch_item> trial(items, items + n);
     for (auto& it : trial) it.passes = rounds;
@@ -2081,7 +2130,8 @@ ER_API int er_autotune_batch(const er_batch_item* items, int n, int rounds, er_t
         int s;
         for (int k = 0; k < n; ++k) {
             er_tune x = c;
-            if (vols[k] && !brick_fits(vols[k]->desc, vols[k]->vmax, (int)std::log2((double)c.brick))) x.brick = orig[k].brick;
+            if (c.brick == 0 || (vols[k] && !brick_fits(vols[k]->desc, vols[k]->vmax, (int)std::log2((double)c.brick))))
+                x.brick = orig[k].brick;
             if ((s = apply_tune(*ts[k], x))) return s;
         }
         return ER_OK;
@@ -2101,7 +2151,7 @@ ER_API int er_autotune_batch(const er_batch_item* items, int n, int rounds, er_t
         return ER_OK;
     };
     er_tune cur = orig[0];
-    cur.brick = orig[0].brick;
+    if (!one_brick) cur.brick = 0;   /* the jobs start with their own bricks */
     float cur_ms = 0.0f;
     st = measure(cur, cur_ms);
     const float default_ms = cur_ms;
@@ -2114,11 +2164,11 @@ ER_API int er_autotune_batch(const er_batch_item* items, int n, int rounds, er_t
         }
     }
     if (!st) st = apply_all(cur);
-    if (st)
-        for (int k = 0; k < n; ++k) {
-            (void)apply_tune(*ts[k], orig[k]);
-            ts[k]->tuned = tuned0[k];
-        }
+    for (int k = 0; k < n; ++k) {
+        if (st) before[k].restore(*ts[k]);
+        else ts[k]->given = false;
+    }
+    if (cur.brick == 0) cur.brick = orig[0].brick;
     for (int k = 0; k < n; ++k) {
         const int rst = snaps[k]->restore(*ts[k]);
         if (!st) st = rst;
@@ -2139,7 +2189,9 @@ ER_API int er_set_tune(int tracer_id, const er_tune* tune)
     if (!t) return st;
     if (!tune) return set_error(ER_ERROR, "tune is NULL");
     if ((st = sync_tracer(*t))) return st;
-    return apply_tune(*t, *tune);
+    if ((st = apply_tune(*t, *tune))) return st;
+    t->given = true;
+    return ER_OK;
 }
 
 ER_API int er_get_tune(int tracer_id, er_tune* tune)

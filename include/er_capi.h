@@ -375,15 +375,19 @@ ER_API int er_set_list_capacity(int capacity);
 
 /* A tracer's launch configuration. None of it changes the image: paths are per pixel and the
  * empty-space skipping is exact, so every configuration renders the same bits. */
-/* Until a tracer is tuned (er_set_tune, er_autotune) er_get_tune reports the configuration the
- * tuner's search starts from, and the library chooses for itself per pass: 4-cell bricks where
- * they fit, 4 workgroups per CU, 768 heavy tiles at 16 rays per wave; a pass rendered alone
- * (er_render_estimate) on a film of at most two tiles per SIMD takes 16 rays per wave, primary and
- * shadow, and 16 shadow waves per CU. */
+/* Until a tracer is tuned the library chooses for itself per pass: 4-cell bricks where they fit
+ * (the volume's default bricks with clipping objects or Woodcock tracking), 4 workgroups per CU,
+ * 768 heavy tiles at 16 rays per wave; a pass rendered alone (er_render_estimate, or one pass of
+ * er_render_passes) on a film of at most two tiles per SIMD takes 16 rays per wave, primary and
+ * shadow, and 16 shadow waves per CU. er_get_tune does not report that choice but the volume's
+ * default bricks and the defaults below; handed to er_set_tune they are taken as given, like any
+ * configuration, for every pass. A search (er_autotune, er_autotune_batch) starts from what the
+ * tracer runs with, times passes that overlap and sets the configuration of those: a pass rendered
+ * alone keeps the library's choice (with the bricks and tiles that were found). */
 typedef struct er_tune {
     int   brick;                  /* macrocell (brick) edge in cells: 2, 4, 8, 16, 32 */
     int   tile_w, tile_h;         /* primary tile, 64 pixels: 4x16, 8x8, 16x4 or 32x2 */
-    int   blocks_per_cu;          /* persistent 256-lane primary workgroups per CU */
+    int   blocks_per_cu;          /* persistent 256-lane primary workgroups per CU (default 7) */
     int   shadow_waves_per_cu;    /* persistent 64-lane shadow-march waves per CU (default 4) */
     int   heavy_tiles;            /* most expensive tiles of a pass whose rays the next pass marches
                                      with several lanes per ray (heavy_rays_per_wave; default 0,

@@ -1567,7 +1567,8 @@ int apply_tune(Tracer& t, const er_tune& r)
 }
 
 /* The per-tracer state a timing trial overwrites, saved and put back so that tuning leaves
- * a render where it was. */
+ * a render where it was. The copies go through the tracer's stream: a copy within the device need
+ * not have ended when hipMemcpy returns, and the null stream is not ordered with the tracer's. */
 struct Snapshot {
     DevBuf<uint32_t> s1, s2;
     DevBuf<float4> run;
@@ -1583,15 +1584,15 @@ struct Snapshot {
         if ((st = s1.alloc(n)) || (st = s2.alloc(n)) || (st = run.alloc(n)) || (st = disp.alloc(n)) ||
             (st = filt.alloc(n)) || (st = cnt.alloc(12)))
             return st;
-        HIP_TRY(hipMemcpy(s1.ptr, t.seeds1.ptr, n * 4, hipMemcpyDeviceToDevice));
-        HIP_TRY(hipMemcpy(s2.ptr, t.seeds2.ptr, n * 4, hipMemcpyDeviceToDevice));
-        HIP_TRY(hipMemcpy(run.ptr, t.running.ptr, n * sizeof(float4), hipMemcpyDeviceToDevice));
-        HIP_TRY(hipMemcpy(disp.ptr, t.display.ptr, n * sizeof(uchar4), hipMemcpyDeviceToDevice));
+        HIP_TRY(hipMemcpyAsync(s1.ptr, t.seeds1.ptr, n * 4, hipMemcpyDeviceToDevice, t.stream));
+        HIP_TRY(hipMemcpyAsync(s2.ptr, t.seeds2.ptr, n * 4, hipMemcpyDeviceToDevice, t.stream));
+        HIP_TRY(hipMemcpyAsync(run.ptr, t.running.ptr, n * sizeof(float4), hipMemcpyDeviceToDevice, t.stream));
+        HIP_TRY(hipMemcpyAsync(disp.ptr, t.display.ptr, n * sizeof(uchar4), hipMemcpyDeviceToDevice, t.stream));
         /* the bilateral filter's output is what er_get_estimate returns when it is on */
-        HIP_TRY(hipMemcpy(filt.ptr, t.disp_filt.ptr, n * sizeof(uchar4), hipMemcpyDeviceToDevice));
-        HIP_TRY(hipMemcpy(cnt.ptr, t.counters.ptr, 12 * sizeof(unsigned long long), hipMemcpyDeviceToDevice));
+        HIP_TRY(hipMemcpyAsync(filt.ptr, t.disp_filt.ptr, n * sizeof(uchar4), hipMemcpyDeviceToDevice, t.stream));
+        HIP_TRY(hipMemcpyAsync(cnt.ptr, t.counters.ptr, 12 * sizeof(unsigned long long), hipMemcpyDeviceToDevice, t.stream));
         no_iter = t.desc.no_iterations;
-        return ER_OK;
+        return sync_tracer(t);
     }
     /* the seeds only: every trial traces the same paths */
     int rewind(Tracer& t)
@@ -1606,14 +1607,14 @@ struct Snapshot {
         int st;
         const size_t n = (size_t)t.W * t.H;
         if ((st = sync_tracer(t))) return st;
-        HIP_TRY(hipMemcpy(t.seeds1.ptr, s1.ptr, n * 4, hipMemcpyDeviceToDevice));
-        HIP_TRY(hipMemcpy(t.seeds2.ptr, s2.ptr, n * 4, hipMemcpyDeviceToDevice));
-        HIP_TRY(hipMemcpy(t.running.ptr, run.ptr, n * sizeof(float4), hipMemcpyDeviceToDevice));
-        HIP_TRY(hipMemcpy(t.display.ptr, disp.ptr, n * sizeof(uchar4), hipMemcpyDeviceToDevice));
-        HIP_TRY(hipMemcpy(t.disp_filt.ptr, filt.ptr, n * sizeof(uchar4), hipMemcpyDeviceToDevice));
-        HIP_TRY(hipMemcpy(t.counters.ptr, cnt.ptr, 12 * sizeof(unsigned long long), hipMemcpyDeviceToDevice));
+        HIP_TRY(hipMemcpyAsync(t.seeds1.ptr, s1.ptr, n * 4, hipMemcpyDeviceToDevice, t.stream));
+        HIP_TRY(hipMemcpyAsync(t.seeds2.ptr, s2.ptr, n * 4, hipMemcpyDeviceToDevice, t.stream));
+        HIP_TRY(hipMemcpyAsync(t.running.ptr, run.ptr, n * sizeof(float4), hipMemcpyDeviceToDevice, t.stream));
+        HIP_TRY(hipMemcpyAsync(t.display.ptr, disp.ptr, n * sizeof(uchar4), hipMemcpyDeviceToDevice, t.stream));
+        HIP_TRY(hipMemcpyAsync(t.disp_filt.ptr, filt.ptr, n * sizeof(uchar4), hipMemcpyDeviceToDevice, t.stream));
+        HIP_TRY(hipMemcpyAsync(t.counters.ptr, cnt.ptr, 12 * sizeof(unsigned long long), hipMemcpyDeviceToDevice, t.stream));
         t.desc.no_iterations = no_iter;
-        return ER_OK;
+        return sync_tracer(t);
     }
 };
 
@@ -2642,7 +2643,7 @@ ER_API int er_adjoint_value(int tracer_id, const uint32_t* seeds1, const uint32_
     HIP_TRY(hipMemcpy(d2.ptr, seeds2, n * 4, hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(lut_e.ptr, eval_lut, ER_TF_LUT_NODES * 4 * sizeof(float), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(sig_e.ptr, sig.data(), sig.size() * sizeof(float), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemset(running.ptr, 0, n * sizeof(float4)));
+    HIP_TRY(erd_launch_zero_words((uint32_t*)running.ptr, n * 4, t->stream));
     /* value mode reads every sample: all occupancy bits set, plus the decision table */
     const size_t lds = (size_t)P.mc_words * 4 + ((size_t)P.lut_max + 1) * sizeof(float);
     for (int k = 0; k < passes; ++k) {

@@ -322,7 +322,8 @@ __device__ __forceinline__ CellFetch cell_fetch(const DevParams& p, const Lattic
     return f;
 }
 
-/* whether the sample's eight corners are voxels of the volume, none of them clamped (not for NaN) */
+/* whether the sample's cell needs no clamp to the lattice (corners beyond the last voxel are clamped in
+ * the cell's record already); false for NaN */
 __device__ __forceinline__ bool lattice_inside(const DevParams& p, const Lattice& l)
 {
     return fminf(l.Lx, fminf(l.Ly, l.Lz)) >= 0.0f && l.Lx < p.resf[0] && l.Ly < p.resf[1] && l.Lz < p.resf[2];

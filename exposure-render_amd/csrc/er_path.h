@@ -68,16 +68,19 @@ __device__ __forceinline__ bool clipped(const DevParams& p, f3 P)
 #define ER_CNT_LINES (3 + ER_TILE_QUEUES)
 #define ER_CNT_WORDS ER_CNT(ER_CNT_LINES)
 
-/* dense samples per march iteration (loads in flight together) in the primary and shadow kernels */
 #define ER_BATCH_CONST_JOBS 128   /* jobs per batch graph (parameter blocks in constant memory) */
 
-/* A march iteration costs about 2000 cycles besides its samples (the look at the occupancy bits,
+/* Dense samples per march iteration (loads in flight together) in the primary and shadow kernels.
+ * A march iteration costs about 2000 cycles besides its samples (the look at the occupancy bits,
  * the loads' latency, the skips of the wave's other lanes) and 300 per sample, so the primary
  * march, whose longest rays end last, takes 10 samples at once: against 6, one pass of the 256^3
  * CT volume at 640 x 480 0.75 -> 0.68 ms, the compat loop 4.6 -> 4.0, 16 passes of the CT workload
- * 9.4 -> 8.7. 16 samples (2 waves per SIMD) gain 4 - 6% more where few tiles are in flight and
- * lose 4 - 9% where passes overlap; the heavy tiles' lane groups make up for the former. Shadow
- * marches refill their lanes: 12 or 16 samples instead of 8 lose up to 8% on the large workloads. */
+ * 9.4 -> 8.7 (timed together with cell_fetch_inside). The one-lane plain and clip kernels take 171
+ * and 181 VGPRs at 10 samples, 2 waves per SIMD (3 need at most 168: 138 and 170 at 6 samples, 146
+ * and 170 at 8), and 247 and 256 at 16, 2 waves as well: 16 gain 4 - 6% more where few tiles are in
+ * flight and lose 4 - 9% where passes overlap; the heavy tiles' lane groups make up for the former.
+ * The general form has a number of its own (ER_BATCH_PRIMARY_ANY). Shadow marches refill their
+ * lanes: 12 or 16 samples instead of 8 lose up to 8% on the large workloads. */
 #ifndef ER_BATCH_PRIMARY
 #define ER_BATCH_PRIMARY 10
 #endif
@@ -101,9 +104,10 @@ __device__ __forceinline__ bool clipped(const DevParams& p, f3 P)
  * negative opacity (the host checks the table): then a sample in a macrocell without its
  * occupancy bit reads 0 from the table anyway, so a batch need not look the bits up, and the
  * optical depth never falls, so its last value tells whether any of the batch's samples crossed
- * the threshold. A marched sample takes about 80 instructions instead of 110 and the one-lane
- * primary kernel 118 VGPRs instead of 162 (4 waves per SIMD instead of 3): 16 passes of the CT
- * workload 11.37 -> 9.08 ms, of the 64^3 blobs at 256 x 256 3.95 -> 3.25 ms. */
+ * the threshold. A marched sample takes about 80 instructions instead of 110 and fewer registers
+ * (the one-lane primary kernel 118 VGPRs instead of 162 when both took 6 samples and this form had
+ * one cell fetch; see ER_BATCH_PRIMARY for now): 16 passes of the CT workload 11.37 -> 9.08 ms, of
+ * the 64^3 blobs at 256 x 256 3.95 -> 3.25 ms. */
 #define ER_MARCH_ANY 1
 #define ER_MARCH_PLAIN 2
 /* ER_MARCH_CLIP: the plain form with clipping objects. A batch whose first and last sample lie in

@@ -328,8 +328,9 @@ struct Volume {
  * 2^ER_GROUP_SHIFT macrocells a side), the groups' clip-free bits and, when it takes at most
  * 32 KB, the opacity table (one float per intensity up to the volume's maximum) are staged in
  * LDS by the march kernels; together they must fit 52.5 KB (105 LDS allocation blocks of 512
- * bytes, with one more for a kernel's own LDS), so that three march workgroups (the primary
- * kernel's register-bound occupancy) share a CU's 160 KB. */
+ * bytes, with one more for a kernel's own LDS), so that three march workgroups share a CU's 160 KB.
+ * Registers let in two of the plain and clip one-lane primary kernels, three of the general and
+ * Woodcock ones and four of the one-lane shadow kernels beside them (three of the general form's). */
 const size_t ER_MAX_TABLES_BYTES = 53760;
 bool brick_fits(const er_volume_desc& d, uint16_t vmax, int shift)
 {
@@ -934,7 +935,7 @@ void clip_classes(const DevParams& P, int nmc, double edge_ext, std::vector<uint
 
 /* The brick (macrocell) edge of a tracer's marches, as a shift: the tuned one where it fits the
  * volume, else 4 cells where that fits (against 8, with 768 heavy tiles: one frame of the CT
- * volume 0.61 -> 0.59 ms, 16 passes 7.3 -> 7.0 ms, 8 with objects 3.08 -> 2.91), else the volume's
+ * volume 0.61 -> 0.59 ms, 16 passes 7.4 -> 7.1 ms, 8 with objects 3.15 -> 2.94), else the volume's
  * default. Scenes with clipping objects keep the volume's: the host classifies every macrocell.
  * Woodcock tracking reads no macrocells. */
 int brick_shift(const Tracer& t, const Volume& v, int clip_count)
@@ -1331,17 +1332,19 @@ bool use_bilateral(const Tracer& t)
  * 0.55 ms, for the 256 x 256 blobs from 0.20 to 0.23); otherwise by the film's size and by whether
  * the pass runs alone (er_render_estimate) or overlaps others:
  *  - 64 rays per wave, the rays of the 768 most expensive tiles in groups of 4 lanes (their long
- *    marches end the kernel): against no heavy tiles, one frame of the CT volume at 640 x 480
- *    0.68 -> 0.61 ms, the compat loop 3.96 -> 3.61, 8 passes with objects 3.50 -> 3.08, 16 CT
- *    passes 8.1 -> 7.3 ms; 256 or 2048 tiles are within 2% of 768 or worse, groups of 16 lanes
- *    5 - 15% slower;
+ *    marches end the kernel), 4^3 bricks: against no heavy tiles, one frame of the CT volume at
+ *    640 x 480 0.65 -> 0.59 ms, 8 frames of the compat loop 3.82 -> 3.49, 8 passes with objects
+ *    3.36 -> 2.94, 16 CT passes at 1024 x 768 7.7 -> 7.1 ms; 256 or 2048 tiles are within 2% of 768
+ *    or worse (CT 7.8, 7.0), groups of 16 lanes 5 - 17% slower;
  *  - a pass alone on a film of at most two tiles per SIMD cannot fill the device with a lane per
- *    ray: 16 rays per wave, primary and shadow, and 16 shadow waves per CU (256 x 256: 0.31 ->
- *    0.25 ms a frame). Overlapped passes do (16 passes: 2.5 ms with heavy tiles, 2.9 so); and on
- *    larger films the groups' redundant skips cost more than the lanes gain (8 passes at 643 x 479
- *    3.9 ms).
- * 4 primary workgroups per CU, what the registers let in: the 7 of before only staged their
- * tables to find no tile left. */
+ *    ray: 16 rays per wave, primary and shadow, and 16 shadow waves per CU (256 x 256: 0.30 ->
+ *    0.23 ms a frame); on larger films the groups' redundant skips cost more than the lanes gain
+ *    (8 passes at 643 x 479 2.9 -> 5.1 ms, a CT frame at 640 x 480 0.59 -> 0.63). Passes that
+ *    overlap on such a small film would gain by it too (16 of 256 x 256: 2.7 -> 2.2, 2.2 -> 2.0
+ *    and 3.6 -> 2.8 ms on three volumes); the line is drawn at single passes so far.
+ * 4 primary workgroups per CU: registers let in 2 of the plain form's, and a workgroup beyond those
+ * that are resident stages its tables only to find few tiles left, or none. 16 CT passes at
+ * 1024 x 768 with 2 / 3 / 4 / 7 of them: 6.85 / 6.97 / 7.05 / 7.34 ms; elsewhere within 1%. */
 struct Launch {
     int blocks_per_cu, shadow_waves_per_cu, heavy_tiles, rays_per_wave, shadow_rays_per_wave, heavy_rays_per_wave;
 };
@@ -2546,7 +2549,7 @@ ER_API int er_adjoint_lut(int tracer_id, const uint32_t* seeds1, const uint32_t*
 
 /* er_adjoint_lut with every work buffer in the device scratch array: no hipMalloc or hipFree.
  * The same kernels run for one pass at a time on the tracer's first stream (er_adjoint_lut
- * overlaps consecutive passes on two buffer sets). */
+ * overlaps consecutive passes on ER_ADJ_SETS buffer sets). */
 ER_API int er_adjoint_lut_noalloc(int tracer_id, const uint32_t* seeds1, const uint32_t* seeds2, size_t count, int passes,
                                   const float* dL_drunning_xyz, double* dL_dlut)
 {

@@ -3,7 +3,7 @@
  *
  * A pass is a short pipeline of kernels over the whole film (KrnlSingleScattering,
  * Source/singlescattering.cuh:27-38, split where the paths diverge):
- *   k_primary  persistent waves take 8 x 8 pixel tiles from an atomic counter; each lane
+ *   k_primary  persistent waves take 8 x 8 pixel tiles from eight atomic counters; each lane
  *              generates its camera ray and marches it (SampleVolume, raymarching.h:30-71);
  *              pixels without a volume event are final, the others are appended to a
  *              scatter queue (wave-aggregated atomics);
@@ -18,7 +18,8 @@
  *
  * Template parameters: in the shading kernels FULL selects the full estimator (shading-mode
  * selection, both halves of MIS); in the march kernels it is the march functions' mode
- * (ER_MARCH_ANY, ER_MARCH_PLAIN). COUNT adds the sample counters.
+ * (ER_MARCH_ANY, ER_MARCH_PLAIN, ER_MARCH_CLIP, ER_MARCH_WOODCOCK). COUNT adds the sample
+ * counters.
  */
 #include "er_path.h"
 

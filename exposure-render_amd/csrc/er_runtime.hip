@@ -620,13 +620,16 @@ int tracer_seed(Tracer& t, uint64_t seed)
     return ER_OK;
 }
 
-/* FrameBuffer::Resize (Source/framebuffer.h:45-68): buffers, zeroed estimates, new seeds */
+/* FrameBuffer::Resize (Source/framebuffer.h:45-68): buffers, zeroed estimates, new seeds. A size that
+ * is refused changes nothing; a failure after that (out of memory) leaves the tracer with an empty
+ * film, never with buffers of two sizes. */
 int tracer_resize(Tracer& t, int W, int H, int id)
 {
     if (W == t.W && H == t.H && t.set[0].frame.ptr) return ER_OK;
     if (W < 0 || H < 0) return set_error(ER_ERROR, "invalid film size %d x %d", W, H);
     int st;
     if ((st = sync_tracer(t))) return st;
+    t.W = t.H = 0;
     const size_t n = (size_t)W * H;
     if ((st = t.running.alloc(n)) || (st = t.display.alloc(n)) || (st = t.disp_tmp.alloc(n)) ||
         (st = t.disp_filt.alloc(n)) || (st = t.seeds1.alloc(n)) || (st = t.seeds2.alloc(n)))
@@ -648,14 +651,13 @@ int tracer_resize(Tracer& t, int W, int H, int id)
         }
     }
     t.cur = 0;
-    t.W = W; t.H = H;
     if (n) {
         HIP_TRY(hipMemset(t.running.ptr, 0, n * sizeof(float4)));
         HIP_TRY(hipMemset(t.display.ptr, 0, n * sizeof(uchar4)));
         HIP_TRY(hipMemset(t.disp_filt.ptr, 0, n * sizeof(uchar4)));
-        return tracer_seed(t, 0x45787052ull + (uint64_t)id);
     }
-    return ER_OK;
+    t.W = W; t.H = H;
+    return n ? tracer_seed(t, 0x45787052ull + (uint64_t)id) : ER_OK;
 }
 
 void mat34(float dst[3][4], const float src[4][4])
@@ -1852,9 +1854,9 @@ ER_API int er_bind_tracer(er_tracer_desc* d, int bind)
                 st = set_error(ER_ERROR, "hipMemset failed");
             if (st) { delete t; t = nullptr; return st; }
         }
-        t->desc = desc;
-        int st = tracer_resize(*t, desc.camera.film_size[0], desc.camera.film_size[1], desc.id);
-        if (st && fresh) { delete t; t = nullptr; }
+        const int st = tracer_resize(*t, desc.camera.film_size[0], desc.camera.film_size[1], desc.id);
+        if (!st) t->desc = desc;
+        else if (fresh) { delete t; t = nullptr; }
         return st;
     });
 }

@@ -260,3 +260,28 @@ def test_clipping_object_comes_and_goes(fresh, tuned):
         assert all(np.array_equal(a, b) for a, b in zip((got[0], got[2], got[3]), (want[clip][0], want[clip][2], want[clip][3])))
         assert all(np.array_equal(a, b) for a, b in zip(got[1], want[clip][1]))
     r.close()
+
+
+@pytest.mark.parametrize("film", [(-3, 70), (90, -1)])
+def test_a_refused_film_leaves_the_bound_tracer(fresh, film):
+    """A rebind whose film is refused changes nothing, its other settings included."""
+    print(f"[rebind] refused film {film}", flush=True)
+    r = er.Renderer(_scene())
+    base = _passes(r)
+    t = r.tracer
+    kept = type(t).from_buffer_copy(t)
+    t.camera.film_size[0], t.camera.film_size[1] = film
+    t.settings.density_scale = 1.0
+    assert r.lib.er_bind_tracer(C.byref(t), 1) == capi.ER_ERROR
+    _bind(r, "clip")                 # a bind of something else: parameters are built again
+    r.seed(11)
+    r.render_passes(2)               # passes 3 and 4 of the tracer as it was
+    got = r.frame(), r.get_seeds()
+    assert r.no_iterations() == 4
+    assert np.array_equal(got[0], base[0])
+    assert np.array_equal(got[1][0], base[1][0]) and np.array_equal(got[1][1], base[1][1])
+    C.memmove(C.byref(t), C.byref(kept), C.sizeof(t))
+    r.rebind()
+    again = _passes(r)
+    r.close()
+    assert np.array_equal(again[0], base[0])

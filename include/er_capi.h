@@ -394,7 +394,8 @@ typedef struct er_tune {
                                      with 64 rays per wave only) */
     int   rays_per_wave;          /* primary rays one 64-lane wave marches at once: 64 (one lane per
                                      ray, default), 16 or 4 (groups of 4 or 16 lanes per ray, each
-                                     round trip reading 24 or 32 consecutive samples of the ray), 1
+                                     round trip reading 32 consecutive samples of the ray, 24 in the
+                                     general march form with 4 lanes), 1
                                      (the whole wave per ray); Woodcock tracking always takes 64.
                                      The reference runs one thread per pixel
                                      (singlescattering.cuh:34-38). */

@@ -25,12 +25,16 @@ def _overlapped(r):
 
 
 def _alone(r):
-    times = []
-    for _ in range(60):
-        a = time.perf_counter()
-        r.render_estimate()
-        times.append(time.perf_counter() - a)
-    return statistics.median(times) * 1e3
+    """a pass alone, ms: the best of five medians, so that a busy host does not count"""
+    medians = []
+    for _ in range(5):
+        times = []
+        for _ in range(20):
+            a = time.perf_counter()
+            r.render_estimate()
+            times.append(time.perf_counter() - a)
+        medians.append(statistics.median(times))
+    return min(medians) * 1e3
 
 
 @pytest.mark.parametrize("film", [(360, 340), (640, 480)])
